@@ -6,48 +6,18 @@
 //
 // The kernels (MI355X-first designs, not translations of the reference's
 // cuTile/WMMA kernels) all compute D^T = B^T . A^T, so each lane holds runs
-// of four consecutive n of one row of C and the epilogue writes 8-byte bf16
-// quads; workgroup ids are remapped so that tiles sharing A rows / B
-// columns run on the same XCD (own L2), in groups of GROUP_M tile rows.
+// of four consecutive n of one row of C; workgroup ids are remapped so that
+// tiles sharing A rows / B columns run on the same XCD (own L2).  A and B go
+// HBM -> LDS by direct loads into rings, and every kernel takes any K (a
+// multiple of 8): the K % 64 tail is computed before the K loop, from a ring
+// slot that the prologue leaves free.
 //
-// gemm_bf16_dma16_kernel (the large problems: at least one 256x256 tile
-// per CU, K % 32 == 0; also 128x128 tiles when those are at least one per
-// CU): 16x16x32 bf16 MFMAs, 8 waves of 128x64 (64x32 at 128x128 tiles),
-// A/B tiles copied HBM -> LDS by direct loads into a 5-stage (6 at
-// 128x128) ring, one barrier per K tile, the next K tile's fragments read
-// during the current tile's MFMAs.  Details at the kernel.
-// gemm_bf16_dma16s_kernel takes the 256x256 tiles when K % 64 == 0: the
-// same MFMAs and schedule, with A in 64-deep blocks of whole 128-byte lines
-// through a ring of its own beside the B ring.
-//
-// gemm_bf16_sdma_kernel (about one 64x64 tile per CU and a long K, e.g.
-// 1024^3): two wave groups split K, each with its own direct-load ring.
-//
-// gemm_bf16_stream_kernel (K % 64 == 0; M <= 64 and N >= 256, or at most 64
-// tiles of 64x64 and K >= 512): products too small to fill the CUs with
-// tiles stream B through workgroups of 32 columns x 32 or 64 rows whose
-// waves split K.
-//
+// gemm_bf16_dma16s_kernel: 256x256 tiles, the large products.
+// gemm_bf16_dma64_kernel: tiles of 64x64 to 128x192, single and batched.
+// gemm_bf16_stream_kernel: few rows or few tiles; workgroups of 32 columns x
+// 32 or 64 rows stream B, their waves splitting K.
 // gemm_bf16_smallm_kernel / gemm_bf16_smallm_sk_kernel (batched items with
 // M <= 32): single-wave or K-split 4-wave workgroups over the whole K.
-//
-// gemm_bf16_kernel (everything else: small or ragged-K problems; 32x32x16
-// bf16 MFMAs):
-//  * One workgroup computes a BM x BN tile of C with WM x WN waves; each
-//    wave owns a (BM/WM) x (BN/WN) sub-tile of 32x32 fragments.
-//  * K advances in 64-deep tiles staged through LDS via registers, double
-//    buffered: the next tile's global loads are in flight while MFMAs
-//    consume the current one; one barrier per K tile.  The loads are
-//    buffer loads: chunks past M, N or K get an out-of-range offset and
-//    read as zero, so edge tiles and the K tail run the same branch-free
-//    code as interior ones.
-//  * A is stored k-contiguous ([BM][64]); B is stored exactly as it sits in
-//    memory ([64][BN], n contiguous) and its k-contiguous MFMA operand is
-//    read with gfx950's transposing LDS read (ds_read_b64_tr_b16), so no
-//    thread ever transposes B in registers.
-//  * LDS rows are padded (A: +16 B, B: +64 B) so that the 16-lane phases of
-//    the A reads and the 32-lane phases of the transposing B reads hit
-//    distinct banks, and every fragment address is base + immediate.
 #include <type_traits>
 
 #include "mx_common.h"
@@ -55,263 +25,14 @@
 namespace mx {
 namespace gemm {
 
-// The direct-load 16x16x32 kernel: K depth of a ring stage (bf16 elements),
-// ring stages and waves at 256x256 tiles, and stages and waves across N at
-// 128x128 tiles (16 KB stages; 6 measured best of 4..9 at 2048^3).
-constexpr int DMA_BK = 32;
-constexpr int DMA_NS = 5, DMA_WM = 2, DMA_WN = 4;
-constexpr int D128_NS = 6, D128_WN = 4;
-
-constexpr int BK = 64;  // K tile depth (bf16 elements)
 constexpr int GROUP_M = 8;
 
-template <int BM, int BN, int WM, int WN>
-struct Cfg {
-  static constexpr int NT = 64 * WM * WN;          // threads
-  static constexpr int TM = BM / WM, TN = BN / WN; // wave tile
-  static constexpr int FM = TM / 32, FN = TN / 32; // 32x32 fragments per wave
-  static constexpr int A_ROW = BK * 2 + 16;        // bytes per A row in LDS
-  static constexpr int B_ROW = BN * 2 + 64;        // bytes per B row in LDS
-  static constexpr int A_CHUNKS = BM * BK / 8 / NT;  // 16-B chunks of A per thread
-  static constexpr int B_CHUNKS = BK * BN / 8 / NT;  // 16-B chunks of B per thread
-  static constexpr int LDS_A = BM * A_ROW;
-  static constexpr int LDS_B = BK * B_ROW;
-  static constexpr int LDS_STAGE = LDS_A + LDS_B;
-  static_assert(A_CHUNKS >= 1 && B_CHUNKS >= 1, "tile split");
-  static_assert(BM * BK / 8 % NT == 0 && BK * BN / 8 % NT == 0, "tile split");
-  static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile");
-};
-
-// gridDim.y indexes a batch of independent products whose operands sit
-// sA / sB / sC elements apart (0 and gridDim.y = 1 for a single GEMM).
-// KS > 1 splits K inside the workgroup: KS groups of WM x WN waves, each
-// with its own double buffer, take consecutive runs of K tiles of the same
-// C tile, and their fp32 accumulators are summed through LDS at the end.
-// For grids of about one tile per CU, where the serial K loop's load latency
-// (not the MFMAs) sets the time, it runs KS loads in flight per CU.
-// PF = 2 stages the global loads two K tiles ahead in two register sets
-// (the LDS double buffer is unchanged), for the same latency-bound case.
-// Buffer resource over [base, base + 2^31 - 16) for loads whose offsets
-// stay below 2^31; an offset of kOobOffset is out of range and reads zero.
-constexpr uint32_t kOobOffset = 0x7ffffff0u;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)kOobOffset, 0x00020000);
-}
-__device__ __forceinline__ u32x4 buffer_ld128(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
-  return __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0);
-}
-// The register-staged kernel's in-range offsets (BM rows of A, BK k-rows of
-// B from a tile's base) stay below that range: leading dimensions up to
-// 4M (A, BM = 256) and 16M (B) elements.
+// The interface's bound on the leading dimensions of shapes with K % 32 != 0,
+// of small grids and of batched items with more than 32 rows: BM rows of A
+// and 64 k-rows of B span less than 2^31 bytes.
 template <int BM>
-inline bool staged_strides_ok(int lda, int ldb) {
-  return (long long)lda * 2 * BM < (long long)kOobOffset && (long long)ldb * 2 * BK < (long long)kOobOffset;
-}
-
-template <int BM, int BN, int WM, int WN, int KS = 1, int PF = 1>
-__global__ __launch_bounds__(64 * WM * WN * KS, 1) void gemm_bf16_kernel(
-    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C, int M,
-    int N, int K, int lda, int ldb, int ldc, long long sA, long long sB, long long sC) {
-  using CF = Cfg<BM, BN, WM, WN>;
-  constexpr int NT = CF::NT, FM = CF::FM, FN = CF::FN;
-  extern __shared__ __align__(16) unsigned char smem_all[];
-  A += (size_t)blockIdx.y * sA;
-  B += (size_t)blockIdx.y * sB;
-  C += (size_t)blockIdx.y * sC;
-
-  const int grp = KS > 1 ? (int)threadIdx.x / NT : 0;  // K group
-  unsigned char* const smem = smem_all + grp * 2 * CF::LDS_STAGE;
-  const int tid = (int)threadIdx.x % NT;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave / WN, wn = wave % WN;
-  const int g = lane >> 5;
-
-  // ---- tile coordinates: XCD-aware remap, then grouped row-major order ----
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  const int nblk = tiles_m * tiles_n;
-  const int id = xcd_remap(blockIdx.x, nblk);
-  const int per_group = GROUP_M * tiles_n;
-  const int group = id / per_group;
-  const int first_m = group * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int tm = first_m + (id % per_group) % gsz;
-  const int tn = (id % per_group) / gsz;
-  const int m0 = tm * BM, n0 = tn * BN;
-
-  // ---- global -> register staging.  A: chunk q -> row q/8, chunk q%8.
-  //      B: chunk q -> k row q/(BN/8), column chunk q%(BN/8). ----
-  static_assert(PF == 1 || PF == 2, "one or two register sets");
-  u32x4 ra[PF][CF::A_CHUNKS], rb[PF][CF::B_CHUNKS];
-  constexpr int BCH = BN / 8;
-
-  // Loads go through buffer resources based at the K tile: a chunk past M,
-  // N or K gets an offset past the resource's range and reads as zero, so
-  // every tile, edge or interior, K tail or not, runs the same branch-free
-  // code (the host keeps lda * 2 * BM and ldb * 2 * BK below 2^31).
-  auto load_tile = [&](int k0, auto set_tag) {
-    constexpr int SET = decltype(set_tag)::value;
-    const __amdgpu_buffer_rsrc_t rs_a = tile_rsrc(A + (size_t)m0 * lda + k0);
-    const __amdgpu_buffer_rsrc_t rs_b = tile_rsrc(B + (size_t)k0 * ldb + n0);
-#pragma unroll
-    for (int i = 0; i < CF::A_CHUNKS; ++i) {
-      const int q = tid + i * NT;
-      const int r = q >> 3, c = (q & 7) * 8;
-      const bool ok = m0 + r < M && k0 + c < K;
-      ra[SET][i] = buffer_ld128(rs_a, ok ? (uint32_t)r * (uint32_t)lda * 2u + 2u * c : kOobOffset);
-    }
-#pragma unroll
-    for (int i = 0; i < CF::B_CHUNKS; ++i) {
-      const int q = tid + i * NT;
-      const int r = q / BCH, c = (q % BCH) * 8;
-      const bool ok = k0 + r < K && n0 + c < N;
-      rb[SET][i] = buffer_ld128(rs_b, ok ? (uint32_t)r * (uint32_t)ldb * 2u + 2u * c : kOobOffset);
-    }
-  };
-
-  auto store_tile = [&](int stage, auto set_tag) {
-    constexpr int SET = decltype(set_tag)::value;
-    unsigned char* sa = smem + stage * CF::LDS_STAGE;
-    unsigned char* sb = sa + CF::LDS_A;
-#pragma unroll
-    for (int i = 0; i < CF::A_CHUNKS; ++i) {
-      const int q = tid + i * NT;
-      *reinterpret_cast<u32x4*>(sa + (q >> 3) * CF::A_ROW + (q & 7) * 16) = ra[SET][i];
-    }
-#pragma unroll
-    for (int i = 0; i < CF::B_CHUNKS; ++i) {
-      const int q = tid + i * NT;
-      *reinterpret_cast<u32x4*>(sb + (q / BCH) * CF::B_ROW + (q % BCH) * 16) = rb[SET][i];
-    }
-  };
-
-  f32x16 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
-
-  // Fragment addressing (32x32x16, k = 16 per step, lane half g holds k 8g..8g+7):
-  //  A operand: row wm*TM + 32i + lane%32, 16-B chunk 2ks + g.
-  //  B^T operand via transposing reads: lane (g, sg, 4j+a) reads B row
-  //  (k) 16ks + 8g + 4r + j at column wn*TN + 32jn + 16sg + 4a, r = 0, 1.
-  const int a_off = (wm * CF::TM + (lane & 31)) * CF::A_ROW + g * 16;
-  const int b_sg = (lane >> 4) & 1, b_j = (lane >> 2) & 3, b_a = lane & 3;
-  const int b_off = (8 * g + b_j) * CF::B_ROW + (wn * CF::TN + 16 * b_sg + 4 * b_a) * 2;
-
-  // this group's K tiles: [kt0, kt0 + cnt); every group runs nkg loop trips
-  // so the barriers match
-  const int nk_all = (K + BK - 1) / BK;
-  const int nkg = (nk_all + KS - 1) / KS;
-  const int kt0 = grp * nkg;
-  const int nk = max(0, min(nkg, nk_all - kt0));
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, PF - 1>;
-  // MFMAs of the K tile in LDS stage `stage`
-  auto compute = [&](int stage) {
-    const unsigned char* sa = smem + stage * CF::LDS_STAGE;
-    const unsigned char* sb = sa + CF::LDS_A;
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      u32x4 af[FM], bfr[FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i) af[i] = *reinterpret_cast<const u32x4*>(sa + a_off + i * 32 * CF::A_ROW + ks * 32);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const unsigned char* p = sb + b_off + (16 * ks) * CF::B_ROW + j * 64;
-        const u32x2 lo = lds_read_tr16(p);
-        const u32x2 hi = lds_read_tr16(p + 4 * CF::B_ROW);
-        bfr[j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-      }
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = mfma32<BF16>(bfr[j], af[i], acc[i][j]);
-    }
-  };
-
-  if (nk > 0) {
-    load_tile(kt0 * BK, S0{});
-    store_tile(0, S0{});
-  }
-  if constexpr (PF == 2) {
-    if (nk > 1) load_tile((kt0 + 1) * BK, S1{});
-  }
-  __syncthreads();
-
-  if constexpr (PF == 2) {
-    // Iteration it: register set it&1 (its tile already in LDS) takes tile
-    // it+2; stage it&1 holds tile it; set (it+1)&1, loaded one iteration
-    // earlier, goes to stage (it+1)&1, freed by the previous barrier.
-    auto step = [&](int it, auto par) {
-      constexpr int P = decltype(par)::value;
-      if (it < nk) {
-        if (it + 2 < nk) load_tile((kt0 + it + 2) * BK, std::integral_constant<int, P>{});
-        compute(P);
-        if (it + 1 < nk) store_tile(P ^ 1, std::integral_constant<int, P ^ 1>{});
-      }
-      __syncthreads();
-    };
-    for (int it = 0; it < nkg; it += 2) {
-      step(it, S0{});
-      if (it + 1 < nkg) step(it + 1, S1{});
-    }
-  } else {
-    for (int it = 0; it < nkg; ++it) {
-      const int cur = it & 1;
-      if (it < nk) {
-        if (it + 1 < nk) load_tile((kt0 + it + 1) * BK, S0{});
-        compute(cur);
-        if (it + 1 < nk) store_tile(cur ^ 1, S0{});
-      }
-      __syncthreads();
-    }
-  }
-
-  if constexpr (KS > 1) {
-    // Sum the groups' accumulators into group 0's (the loop's last barrier
-    // freed every stage).  Element e of thread t of group g >= 1 sits at
-    // float ((g-1)·E + e)·NT + t: consecutive threads, consecutive banks.
-    constexpr int E = FM * FN * 16;
-    static_assert((KS - 1) * E * NT * 4 <= KS * 2 * CF::LDS_STAGE, "the partial sums fit in the stages");
-    float* red = reinterpret_cast<float*>(smem_all);
-    if (grp > 0) {
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) red[((grp - 1) * E + (i * FN + j) * 16 + e) * NT + tid] = acc[i][j][e];
-    }
-    __syncthreads();
-    if (grp > 0) return;  // no barrier follows
-#pragma unroll
-    for (int q = 1; q < KS; ++q)
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] += red[((q - 1) * E + (i * FN + j) * 16 + e) * NT + tid];
-  }
-
-  // ---- epilogue: lane holds C[m][n .. n+3], m = row of lane, n = 8r + 4g ----
-#pragma unroll
-  for (int i = 0; i < FM; ++i) {
-    const int gm = m0 + wm * CF::TM + i * 32 + (lane & 31);
-    if (gm >= M) continue;
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gn = n0 + wn * CF::TN + j * 32 + 8 * r + 4 * g;
-        if (gn < N) {
-          const f32x16& a = acc[i][j];
-          st64(C + (size_t)gm * ldc + gn,
-               u32x2{pack_bf16x2(a[4 * r], a[4 * r + 1]), pack_bf16x2(a[4 * r + 2], a[4 * r + 3])});
-        }
-      }
-  }
+inline bool strides_2g(int lda, int ldb) {
+  return (long long)lda * 2 * BM < 0x7ffffff0LL && (long long)ldb * 2 * 64 < 0x7ffffff0LL;
 }
 
 // A-row chunk swizzle of the small-M kernels' LDS rows: a 16-lane
@@ -323,209 +44,55 @@ __device__ __forceinline__ int swz_a(int m) {
   return BK == 64 ? ((m >> 1) & 7) : ((m >> 2) & 3);
 }
 
-// ---------------------------------------------------------------------------
-// gemm_bf16_sdma_kernel: grids of about one 64x64 tile per CU with a long K
-// (1024^3).  There the time is the latency of streaming each tile's 64 rows
-// of A and 64 columns of B (256 KB per CU at 1024^3), not the MFMAs, so the
-// loads go HBM -> LDS directly through a deep ring:
-//  * 8 waves = 2 K groups x (2 x 2 waves of 32x32); group q takes the K
-//    tiles q*nk .. q*nk + nk - 1, and the two groups' accumulators are
-//    summed through LDS at the end;
-//  * each group has a 5-slot ring of 64-deep K tiles (A: 64 rows x 128 B,
-//    B: 64 k-rows x 128 B; both groups fill the 160 KB of LDS) with four
-//    tiles (64 KB) in flight;
-//  * 16-byte chunks are XOR-swizzled per row, chunk ^ ((m >> 1) & 7) for A
-//    and chunk ^ (((k >> 1) & 1) << 2) for B: LDS serves a 128-bit read in
-//    16-lane groups keyed by lane bit 5 and the parity of lane bits 2..4,
-//    a transposing 64-bit read in 32-lane halves, and both fragment reads
-//    below then touch distinct bank slots within every group.
-// Shapes: M, N multiples of 64, K a multiple of 128.
-// ---------------------------------------------------------------------------
-struct SCfg {
-  static constexpr int BM = 64, BN = 64, BK = 64, NSL = 5, KSG = 2;
-  static constexpr int NW = 8, NWG = NW / KSG, NT = 64 * NW;  // waves, waves per group, threads
-  static constexpr int RA = BK * 2, RB = BN * 2;              // LDS row bytes (128)
-  static constexpr int A_B = BM * RA, B_B = BK * RB;          // 8 KB each
-  static constexpr int STAGE = A_B + B_B;
-  static constexpr int GRP = NSL * STAGE;                     // ring of one group
-  static constexpr int LDS = KSG * GRP;
-  static constexpr int A_LPW = A_B / 1024 / NWG, B_LPW = B_B / 1024 / NWG;  // 1 KB loads per wave per tile
-  static constexpr int LPW = A_LPW + B_LPW;
-  static constexpr int RPL = 1024 / RA;                       // rows per 1 KB load
-  static_assert(LDS <= 160 * 1024 && (NSL - 2) * LPW < 64 && RA == RB, "ring");
-};
-__device__ __forceinline__ int swz_sa(int m) { return (m >> 1) & 7; }
-__device__ __forceinline__ int swz_sb(int k) { return ((k >> 1) & 1) << 2; }
-
-__global__ __launch_bounds__(SCfg::NT, 1) void gemm_bf16_sdma_kernel(const uint16_t* __restrict__ A,
-                                                                    const uint16_t* __restrict__ B,
-                                                                    uint16_t* __restrict__ C, int M, int N, int K,
-                                                                    int lda, int ldb, int ldc) {
-  using CF = SCfg;
-  extern __shared__ __align__(1024) unsigned char smem[];
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int grp = wave / CF::NWG, wg = wave % CF::NWG;  // K group, wave within the group
-  const int wm = wg / 2, wn = wg % 2;
-  const int g = lane >> 5;
-
-  // ---- tile -> (tm, tn), grouped for L2 reuse, XCD-aware ----
-  const int tiles_m = M / CF::BM, tiles_n = N / CF::BN;
-  const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
-  const int per_group = GROUP_M * tiles_n;
-  const int first_m = (id / per_group) * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int m0 = (first_m + (id % per_group) % gsz) * CF::BM;
-  const int n0 = ((id % per_group) / gsz) * CF::BN;
-  const int nk = K / CF::BK / CF::KSG;  // K tiles per group
-  const int kt0 = grp * nk;
-
-  // ---- direct loads: load n of this wave fills rows (k-rows) RPL*(wg*LPW+n)
-  // + lane/8 of the tile, lane taking the chunk stored at position lane%8 ----
-  const uint32_t lds0 = lds_addr(smem) + grp * CF::GRP;
-  uint32_t a_off[CF::A_LPW], b_off[CF::B_LPW];
-#pragma unroll
-  for (int n = 0; n < CF::A_LPW; ++n) {
-    const int row = CF::RPL * (wg * CF::A_LPW + n) + lane / 8;
-    a_off[n] = (uint32_t)row * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_sa(row));
-  }
-#pragma unroll
-  for (int n = 0; n < CF::B_LPW; ++n) {
-    const int row = CF::RPL * (wg * CF::B_LPW + n) + lane / 8;
-    b_off[n] = (uint32_t)row * (uint32_t)ldb * 2u + 16u * ((lane % 8) ^ swz_sb(row));
-  }
-  auto issue = [&](int kt, int slot) {
-    const uint32_t st = lds0 + slot * CF::STAGE;
-    const uint16_t* abase = A + (size_t)m0 * lda + (size_t)(kt0 + kt) * CF::BK;
-    const uint16_t* bbase = B + (size_t)(kt0 + kt) * CF::BK * ldb + n0;
-#pragma unroll
-    for (int n = 0; n < CF::A_LPW; ++n) dma16(abase, a_off[n], st + (wg * CF::A_LPW + n) * 1024);
-#pragma unroll
-    for (int n = 0; n < CF::B_LPW; ++n) dma16(bbase, b_off[n], st + CF::A_B + (wg * CF::B_LPW + n) * 1024);
-  };
-
-  // ---- fragment addresses in slot 0.  A^T (B operand): m = 32 wm +
-  // lane%32, k-chunk 2 ks + g.  B^T (A operand) by transposing reads: lane
-  // (g, sg, 4j+a) reads k-row 16 ks + 8 g + j (+4 for the upper half),
-  // columns 32 wn + 16 sg + 4a .. +3. ----
-  const int am = 32 * wm + (lane & 31);
-  uint32_t a_frag[4];
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) a_frag[ks] = lds0 + am * CF::RA + 16 * ((2 * ks + g) ^ swz_sa(am));
-  const int b_sg = (lane >> 4) & 1, b_j = (lane >> 2) & 3, b_a = lane & 3;
-  const uint32_t b_frag = lds0 + CF::A_B + (8 * g + b_j) * CF::RB +
-                          16 * (((32 * wn + 16 * b_sg + 4 * b_a) >> 3) ^ swz_sb(b_j)) + 8 * (b_a & 1);
-
-  f32x16 acc = f32x16{};
-  auto compute = [&](int slot) {
-    const uint32_t so = slot * CF::STAGE;
-    u32x4 af[4], bf[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      af[ks] = lds_ld128(a_frag[ks] + so);
-      const u32x2 lo = lds_read_tr16_at(b_frag + so + 16 * ks * CF::RB);
-      const u32x2 hi = lds_read_tr16_at(b_frag + so + (16 * ks + 4) * CF::RB);
-      bf[ks] = u32x4{lo[0], lo[1], hi[0], hi[1]};
-    }
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) acc = mfma32<BF16>(bf[ks], af[ks], acc);
-  };
-
-  land_args(C);  // C is used only after the K loop
-  // Tiles 0 .. NSL-2 in flight; every iteration issues one more (past the
-  // end the last tile again, into slots nobody reads), so the wait is the
-  // same in every iteration: tile kt has landed once at most NSL-2 tiles
-  // issued after it are outstanding.
-#pragma unroll
-  for (int p = 0; p < CF::NSL - 1; ++p) issue(min(p, nk - 1), p);
-  for (int kt = 0; kt < nk; ++kt) {
-    wait_vmcnt<(CF::NSL - 2) * CF::LPW>();
-    lds_barrier();  // tile kt visible to every wave; slot (kt-1) % NSL free
-    issue(min(kt + CF::NSL - 1, nk - 1), (kt + CF::NSL - 1) % CF::NSL);
-    compute(kt % CF::NSL);
-  }
-  wait_vmcnt<0>();  // no load lands after this point
-  __syncthreads();  // ... and every fragment read is done: the LDS is free
-
-  // ---- sum the two groups' accumulators (group 1 -> LDS -> group 0) ----
-  float* red = reinterpret_cast<float*>(smem);
-  const int tid = threadIdx.x % (64 * CF::NWG);
-  if (grp == 1) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) red[e * 64 * CF::NWG + tid] = acc[e];
-  }
-  __syncthreads();
-  if (grp == 1) return;  // no barrier follows
-#pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] += red[e * 64 * CF::NWG + tid];
-
-  // ---- epilogue: lane holds m = m0 + am, n = n0 + 32 wn + 8 i + 4 g + {0..3} ----
-  uint16_t* crow = C + (size_t)(m0 + am) * ldc + n0 + 32 * wn + 4 * g;
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    st64(crow + 8 * i, u32x2{pack_bf16x2(acc[4 * i], acc[4 * i + 1]), pack_bf16x2(acc[4 * i + 2], acc[4 * i + 3])});
-}
-
-static int launch_sdma(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
-                       hipStream_t stream) {
-  const long long tiles = (long long)(M / SCfg::BM) * (N / SCfg::BN);
-  if (tiles > 0x7fffffffLL) return MX_ERR_SHAPE;
-  constexpr auto kern = gemm_bf16_sdma_kernel;
-  MX_RETURN_IF_HIP(lds_limit_once<kern>(SCfg::LDS));
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(SCfg::NT), SCfg::LDS, stream, (const uint16_t*)A,
-                     (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
-}
+// A fragment whose k values lie past K counts as zero on both sides, so
+// whatever was loaded in their place (an infinity too) adds nothing.
+__device__ __forceinline__ u32x4 keep_if(bool keep, const u32x4& x) { return keep ? x : u32x4{0, 0, 0, 0}; }
 
 // ---------------------------------------------------------------------------
-// gemm_bf16_dma16_kernel: the direct-load design above on 16x16x32 MFMAs.
-// Under a sustained full-chip MFMA load the 16x16x32 shape delivers about
-// 11% more bf16 throughput than 32x32x16 on MI355X (same FLOPs, less
-// operand/accumulator traffic per FLOP, so less power at the same clock
-// cap), which is what sets the large-GEMM rate.
+// gemm_bf16_dma64_kernel: tiles of up to 128 x 192 by direct loads, on
+// 16x16x32 MFMAs.  Under a sustained full-chip MFMA load the 16x16x32 shape
+// delivers about 11% more bf16 throughput than 32x32x16 on MI355X (same
+// FLOPs, less operand/accumulator traffic per FLOP, so less power at the same
+// clock cap).
 //
-//  * BM x BN tile (256x256, or 128x128 for mid-size problems), BK = 32 (one
-//    16x16x32 k-step per K tile), WM x WN waves, each owning (BM/WM) x
-//    (BN/WN) of C as 16x16 fragments.
+//  * WM x WN waves, each owning (BM/WM) x (BN/WN) of C as 16x16 fragments.
+//  * K advances in 64-deep stages, two k-steps each: a stage holds whole
+//    128-byte lines of A, and there is one barrier per two k-steps.
 //  * Operand layouts (16x16x32): the "A" operand holds 8 consecutive k of
 //    row l%16 at k-group l/16; "B" the same for column l%16; D holds rows
 //    4(l/16)..+3 of column l%16.  Issued as D^T = B^T . A^T: B^T fragments
 //    come from the K-major B tile by transposing reads (lane (kg, j, a)
 //    reads k-row 8kg + 4r + j, columns 4a..+3, r = 0, 1), A^T fragments are
 //    one 16-byte read of an A row; each lane's D is four consecutive n of
-//    one row of C (an 8-byte store).
-//  * A rows are 64 B and a fragment read covers 16 rows x 4 chunks: chunk
-//    kg ^ ((m >> 1) & 3) is the XOR that measured conflict-free on gfx950
-//    (SQ_LDS_BANK_CONFLICT 0; the (m >> 2) and (m & 3) forms conflict).  B
-//    rows are 512 B or 256 B (same banks every row): a 32-lane phase of transposing
-//    reads covers 8 k-rows (two k-groups x 4) of 32 bytes each, and chunk
-//    c ^ 2((k & 3) | ((k >> 3) & 1) << 2) gives the 8 rows distinct 32-byte
-//    slots.  The DMA applies the same XOR on the global side.
-//  * Ring of NS stages, one barrier per K tile (as above).  Tile kt+1's
-//    fragments are read during step kt: B^T ones into the other half of a
-//    parity double buffer at the step's start, each A^T one in place right
-//    after the four MFMAs that consumed the previous tile's.
+//    one row of C.
+//  * A rows are 128 B: chunk c ^ ((m >> 1) & 7) keeps the 16-lane phases of
+//    the A^T reads on distinct bank slots.  B rows of 512 or 256 B start at
+//    bank 0: a 32-lane phase of transposing reads covers 8 k-rows (two
+//    k-groups x 4) of 32 bytes each, and chunk c ^ 2((k & 3) | ((k >> 3) & 1)
+//    << 2) gives the 8 rows distinct 32-byte slots.  The direct loads apply
+//    the same XOR on the global side.
+//  * Ring of NS stages.  The next half's fragments are read during the
+//    current half: B^T ones into the other half of a double buffer at its
+//    start, each A^T one in place right after the MFMAs that consumed the
+//    previous one's.
 // ---------------------------------------------------------------------------
-template <int NS, int WM, int WN, int BM_ = 256, int BN_ = 256>
-struct D16Cfg {
-  static constexpr int BM = BM_, BN = BN_, BK = 32;
+__device__ __forceinline__ int swz_a16w(int m) { return (m >> 1) & 7; }
+__device__ __forceinline__ int swz_b16(int k) { return 2 * ((k & 3) | (((k >> 3) & 1) << 2)); }
+template <int BM_, int BN_, int WM, int WN, int NS_>
+struct D64Cfg {
+  static constexpr int BM = BM_, BN = BN_, BK = 64, NS = NS_;
   static constexpr int NW = WM * WN, NT = 64 * NW;
   static constexpr int TM = BM / WM, TN = BN / WN;  // wave block
   static constexpr int FM = TM / 16, FN = TN / 16;  // 16x16 fragments
   static constexpr int RA = BK * 2, RB = BN * 2;    // LDS row bytes
   static constexpr int A_B = BM * RA, B_B = BK * RB;
   static constexpr int STAGE = A_B + B_B;
-  static constexpr int A_LPW = A_B / 1024 / NW;  // 1 KB loads per wave per stage
-  static constexpr int B_LPW = B_B / 1024 / NW;
-  static constexpr int LPW = A_LPW + B_LPW;
-  static constexpr int A_CH = RA / 16, A_RPL = 1024 / RA;  // chunks per A row, A rows per load
-  static constexpr int B_CH = RB / 16, B_RPL = 1024 / RB;
-  static_assert(NS >= 4 && NS <= 9 && NS * STAGE <= 160 * 1024, "LDS ring");
-  static_assert((NS - 3) * LPW < 64, "vmcnt range");
-  static_assert(A_LPW >= 1 && B_LPW >= 1 && FM >= 1 && FN >= 1, "tile split");
+  static constexpr int A_L = A_B / 1024, A_RPL = 1024 / RA;  // direct loads of A per stage, A rows per load
+  static constexpr int LPW = STAGE / 1024 / NW;              // 1 KB loads per wave per stage
+  static_assert(NS >= 4 && NS * STAGE <= 160 * 1024, "LDS ring");
+  static_assert((NS - 1) * LPW < 64, "vmcnt range");
+  static_assert(STAGE % (1024 * NW) == 0 && TM % 16 == 0 && TN % 16 == 0, "tile split");
 };
-__device__ __forceinline__ int swz_a16(int m) { return (m >> 1) & 3; }
 // Schedule of one K tile: per row block FN MFMAs, then LDS reads: the 2FN
 // B^T reads spread over the first half of the row blocks, each A^T read
 // right behind its row block.
@@ -539,39 +106,94 @@ __device__ __forceinline__ void interleave_rows16() {
     interleave_rows16<FM, FN, I + 1>();
   }
 }
-__device__ __forceinline__ int swz_b16(int k) { return 2 * ((k & 3) | (((k >> 3) & 1) << 2)); }
+// B rows of 64 or 192 columns start at two bank phases (k even, odd), 128 B
+// apart, so the four rows of each parity take the four 32-byte slots of an
+// aligned 128 bytes.
+template <int BN>
+__device__ __forceinline__ int swz_b16n(int k) {
+  static_assert(BN == 64 || BN == 128 || BN == 192 || BN == 256, "row size");
+  return BN == 64 || BN == 192 ? 2 * (((k >> 1) & 1) | (((k >> 3) & 1) << 1)) : swz_b16(k);
+}
 
-// Steps I .. P-1 of a period of the K loop: stage I % NS, parity I % 2.
-template <int NS, int P, int I = 0, typename Step>
+// Steps I .. NS-1 of a period of the K loop: stage I.
+template <int NS, int I = 0, typename Step>
 __device__ __forceinline__ void step_period(Step& step, int kt) {
-  if constexpr (I < P) {
-    step(kt + I, std::integral_constant<int, I % NS>{}, std::integral_constant<int, I % 2>{});
-    step_period<NS, P, I + 1>(step, kt);
+  if constexpr (I < NS) {
+    step(kt + I, std::integral_constant<int, I>{});
+    step_period<NS, I + 1>(step, kt);
   }
 }
-// The first n (< P) steps of a period, for the tail of the K loop.
-template <int NS, int P, int I = 0, typename Step>
+// The first n (< NS) steps of a period, for the tail of the K loop.
+template <int NS, int I = 0, typename Step>
 __device__ __forceinline__ void step_tail(Step& step, int kt, int n) {
-  if constexpr (I < P - 1) {
+  if constexpr (I < NS - 1) {
     if (I < n) {
-      step(kt + I, std::integral_constant<int, I % NS>{}, std::integral_constant<int, I % 2>{});
-      step_tail<NS, P, I + 1>(step, kt, n);
+      step(kt + I, std::integral_constant<int, I>{});
+      step_tail<NS, I + 1>(step, kt, n);
     }
   }
 }
 
-template <int NS, int WM, int WN, int BM_ = 256, int BN_ = 256>
-__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_dma16_kernel(const uint16_t* __restrict__ A,
-                                                                        const uint16_t* __restrict__ B,
-                                                                        uint16_t* __restrict__ C, int M, int N,
-                                                                        int K, int lda, int ldb, int ldc) {
-  using CF = D16Cfg<NS, WM, WN, BM_, BN_>;
-  constexpr int FM = CF::FM, FN = CF::FN, BK = CF::BK;
+// Store a C tile through LDS: the tile goes there as bf16 rows (padded by 16
+// bytes) and is stored as whole rows, each lane 16 contiguous bytes, instead
+// of 8-byte pieces that the memory system writes back as partial lines.  The
+// lane holds rows am + 16 mf, columns cn + 16 nf .. +3; the LDS is free once
+// every wave is past its last fragment reads.
+template <int BM, int BN, int NT, int FM, int FN>
+__device__ __forceinline__ void store_tile_lds(unsigned char* smem, const f32x4 (&acc)[FM][FN], int am, int cn,
+                                               uint16_t* C, int m0, int n0, int M, int N, int ldc) {
+  constexpr int CROW = BN * 2 + 16;
+  __syncthreads();
+#pragma unroll
+  for (int mf = 0; mf < FM; ++mf) {
+    const int r = am + 16 * mf;
+#pragma unroll
+    for (int nf = 0; nf < FN; ++nf) {
+      const f32x4& a = acc[mf][nf];
+      *reinterpret_cast<u32x2*>(smem + r * CROW + 2 * (cn + 16 * nf)) =
+          u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
+    }
+  }
+  __syncthreads();
+  constexpr int CPR = BN / 8;  // 16-byte chunks per tile row
+  constexpr int CH = BM * CPR;
+  static_assert(CH % NT == 0, "whole passes");
+  if constexpr (NT % CPR == 0) {
+    constexpr int RPI = NT / CPR;  // rows per workgroup-wide store
+    const int t = threadIdx.x;
+    const int cc = t % CPR, r0 = t / CPR;
+    const int gn = n0 + 8 * cc;
+#pragma unroll 4
+    for (int r = r0; r < BM; r += RPI) {
+      const int gm = m0 + r;
+      if (gm < M && gn < N)
+        st128(C + (size_t)gm * ldc + gn, *reinterpret_cast<const u32x4*>(smem + r * CROW + 16 * cc));
+    }
+  } else {
+#pragma unroll 4
+    for (int q = threadIdx.x; q < CH; q += NT) {
+      const int r = q / CPR, cc = q % CPR;
+      const int gm = m0 + r, gn = n0 + 8 * cc;
+      if (gm < M && gn < N)
+        st128(C + (size_t)gm * ldc + gn, *reinterpret_cast<const u32x4*>(smem + r * CROW + 16 * cc));
+    }
+  }
+}
+
+template <int BM_, int BN_, int WM_, int WN_, int NS_, bool TAIL>
+__global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C, int M, int N, int K,
+    int lda, int ldb, int ldc, long long sA, long long sB, long long sC) {
+  using CF = D64Cfg<BM_, BN_, WM_, WN_, NS_>;
+  constexpr int NS = CF::NS, FM = CF::FM, FN = CF::FN, BK = CF::BK;
   extern __shared__ __align__(1024) unsigned char smem[];
+  A += (size_t)blockIdx.y * sA;
+  B += (size_t)blockIdx.y * sB;
+  C += (size_t)blockIdx.y * sC;
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave / WN, wn = wave % WN;
+  const int wm = wave / WN_, wn = wave % WN_;
   const int kg = lane >> 4;  // k-group of the lane's operand and row quad of its result
 
   // ---- tile -> (tm, tn), grouped for L2 reuse, XCD-aware ----
@@ -586,57 +208,60 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_dma16_kernel(const 
   const int m0 = tm * CF::BM, n0 = tn * CF::BN;
   const int nk = K / BK;
 
-  // ---- direct-load lane offsets (bytes from the tile's first element).
-  // Rows past M / columns past N re-read the last valid ones; their
-  // results are never stored. ----
+  // ---- direct loads: load ld = wave * LPW + n of a stage fills its bytes
+  // 1024 ld .. +1023 (A rows, then B k-rows).  Rows past M / columns past N
+  // re-read the last valid ones; their results are never stored. ----
   const uint32_t lds0 = lds_addr(smem);
-  const bool full_m = m0 + CF::BM <= M, full_n = n0 + CF::BN <= N;
-  uint32_t a_off[CF::A_LPW], b_off[CF::B_LPW];
+  uint32_t off[CF::LPW];
 #pragma unroll
-  for (int n = 0; n < CF::A_LPW; ++n) {
-    const int row = CF::A_RPL * (wave * CF::A_LPW + n) + lane / CF::A_CH;
-    const int gm = full_m ? m0 + row : min(m0 + row, M - 1);
-    a_off[n] = (uint32_t)(gm - m0) * (uint32_t)lda * 2u + 16u * ((lane % CF::A_CH) ^ swz_a16(row));
-  }
-#pragma unroll
-  for (int n = 0; n < CF::B_LPW; ++n) {
-    const int row = CF::B_RPL * (wave * CF::B_LPW + n) + lane / CF::B_CH;
-    int col = 8 * ((lane % CF::B_CH) ^ swz_b16(row));  // elements
-    if (!full_n) col = min(n0 + col, N - 8) - n0;
-    b_off[n] = (uint32_t)row * (uint32_t)ldb * 2u + 2u * col;
+  for (int n = 0; n < CF::LPW; ++n) {
+    const int ld = wave * CF::LPW + n;
+    if (ld < CF::A_L) {
+      const int row = CF::A_RPL * ld + lane / 8;
+      off[n] = (uint32_t)(min(m0 + row, M - 1) - m0) * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_a16w(row));
+    } else {
+      const int byte = 1024 * (ld - CF::A_L) + 16 * lane;
+      const int row = byte / CF::RB;
+      const int col = 8 * (((byte % CF::RB) / 16) ^ swz_b16n<CF::BN>(row));  // elements
+      off[n] = (uint32_t)row * (uint32_t)ldb * 2u + 2u * (min(n0 + col, N - 8) - n0);
+    }
   }
   auto issue = [&](int kt, int stage) {
     const uint32_t st = lds0 + stage * CF::STAGE;
     const uint16_t* abase = A + (size_t)m0 * lda + (size_t)kt * BK;
     const uint16_t* bbase = B + (size_t)kt * BK * ldb + n0;
 #pragma unroll
-    for (int n = 0; n < CF::A_LPW; ++n) dma16(abase, a_off[n], st + (wave * CF::A_LPW + n) * 1024);
-#pragma unroll
-    for (int n = 0; n < CF::B_LPW; ++n) dma16(bbase, b_off[n], st + CF::A_B + (wave * CF::B_LPW + n) * 1024);
+    for (int n = 0; n < CF::LPW; ++n) {
+      const int ld = wave * CF::LPW + n;
+      dma16(ld < CF::A_L ? abase : bbase, off[n], st + ld * 1024);
+    }
   };
 
   // ---- fragment lane addresses, one base per ring stage (stages lie past
   // ds_read's 16-bit immediate), fragments at immediates from it ----
-  // A^T (B operand): row am + 16 mf, chunk kg ^ swz(am) (swz is the same
-  // for every mf).
+  // A^T (B operand): row am + 16 mf, chunk (4 h + kg) ^ swz(am) (swz is the
+  // same for every mf).
   const int am = wm * CF::TM + (lane & 15);
-  uint32_t a_col[NS];
+  uint32_t a_col[NS][2];
 #pragma unroll
-  for (int st = 0; st < NS; ++st) {
-    a_col[st] = lds0 + st * CF::STAGE + am * CF::RA + 16 * (kg ^ swz_a16(am));
-    asm volatile("" : "+v"(a_col[st]));  // keep it a base register
-  }
-  // B^T (A operand): lane (kg, j, a) reads k-rows 8kg + 4r + j, columns
+  for (int st = 0; st < NS; ++st)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      a_col[st][h] = lds0 + st * CF::STAGE + am * CF::RA + 16 * ((4 * h + kg) ^ swz_a16w(am));
+      asm volatile("" : "+v"(a_col[st][h]));  // keep it a base register
+    }
+  // B^T (A operand): lane (kg, j, a) reads k-rows 32h + 8kg + 4r + j, columns
   // wn*TN + 16 nf + 4a .. +3 (8 bytes of a 16-byte chunk).
   const int b_j = (lane >> 2) & 3, b_a = lane & 3;
-  const int bk = 8 * kg + b_j;  // k-row of the r = 0 read; r = 1 is 4 rows further, same swizzle
+  const int bk = 8 * kg + b_j;  // k-row of the r = 0 read; rows 4 and 32 further share its swizzle
   uint32_t b_col[NS][FN];
 #pragma unroll
   for (int st = 0; st < NS; ++st)
 #pragma unroll
     for (int nf = 0; nf < FN; ++nf) {
       const int chunk = (wn * CF::TN + 16 * nf + 4 * b_a) >> 3;
-      b_col[st][nf] = lds0 + st * CF::STAGE + CF::A_B + bk * CF::RB + 16 * (chunk ^ swz_b16(bk)) + 8 * (b_a & 1);
+      b_col[st][nf] =
+          lds0 + st * CF::STAGE + CF::A_B + bk * CF::RB + 16 * (chunk ^ swz_b16n<CF::BN>(bk)) + 8 * (b_a & 1);
       asm volatile("" : "+v"(b_col[st][nf]));
     }
 
@@ -646,93 +271,132 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_dma16_kernel(const 
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{};
 
-  u32x4 af[FM];     // A^T fragments of the current tile, refilled in place
-  u32x4 bf[2][FN];  // B^T fragments, double buffered by tile parity
-  auto read_b = [&](int stg, int buf) {
+  u32x4 af[FM];     // A^T fragments of the current half, refilled in place
+  u32x4 bf[2][FN];  // B^T fragments of the stage's two halves
+  auto read_b = [&](int stg, int h) {
 #pragma unroll
     for (int nf = 0; nf < FN; ++nf) {
-      const u32x2 lo = lds_read_tr16_at(b_col[stg][nf]);
-      const u32x2 hi = lds_read_tr16_at(b_col[stg][nf] + 4 * CF::RB);
-      bf[buf][nf] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+      const u32x2 lo = lds_read_tr16_at(b_col[stg][nf] + 32 * h * CF::RB);
+      const u32x2 hi = lds_read_tr16_at(b_col[stg][nf] + (32 * h + 4) * CF::RB);
+      bf[h][nf] = u32x4{lo[0], lo[1], hi[0], hi[1]};
     }
   };
-  auto read_a = [&](int stg, int mf) { af[mf] = lds_ld128(a_col[stg] + 16 * mf * CF::RA); };
-
-  // One K tile: its fragments are in af and bf[PAR].  Every step issues
-  // exactly one tile of loads (near the end the last tile again, into
-  // stages nobody reads), so the ring accounting is the same in every step.
-  auto step = [&](int kt, auto stg_tag, auto par_tag) {
-    constexpr int STG = decltype(stg_tag)::value;
-    constexpr int PAR = decltype(par_tag)::value;
-    constexpr int NXT = (STG + 1) % NS;
-    // Every wave has read tile kt (during step kt-1) and its own loads of
-    // tile kt+1 have landed (at most the NS-3 tiles issued after it are in
-    // flight): after the barrier tile kt+1 is readable and stage
-    // (kt-1)%NS, last read during step kt-2, takes tile kt+NS-1.
-    wait_vmcnt<(NS - 3) * CF::LPW>();
-    lds_barrier();
-    issue(min(kt + NS - 1, nk - 1), (STG + NS - 1) % NS);
+  auto read_a = [&](int stg, int h, int mf) { af[mf] = lds_ld128(a_col[stg][h] + 16 * mf * CF::RA); };
+  // the MFMAs of one half, whose fragments are in af and bf[h], while the
+  // fragments of half nh of stage nstg are read
+  auto half = [&](int h, int nstg, int nh) {
     __builtin_amdgcn_sched_barrier(0);
-    read_b(NXT, PAR ^ 1);
+    read_b(nstg, nh);
 #pragma unroll
     for (int mf = 0; mf < FM; ++mf) {
 #pragma unroll
-      for (int nf = 0; nf < FN; ++nf) acc[mf][nf] = mfma16<BF16>(bf[PAR][nf], af[mf], acc[mf][nf]);
-      read_a(NXT, mf);
+      for (int nf = 0; nf < FN; ++nf) acc[mf][nf] = mfma16<BF16>(bf[h][nf], af[mf], acc[mf][nf]);
+      read_a(nstg, nh, mf);
     }
     interleave_rows16<FM, FN>();
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  // One K tile: the fragments of its first half are in af and bf[0].  Every
+  // step issues exactly one tile of loads (near the end the last tile again,
+  // into stages nobody reads), so the ring accounting is the same in every
+  // step.
+  auto step = [&](int kt, auto stg_tag) {
+    constexpr int STG = decltype(stg_tag)::value;
+    constexpr int NXT = (STG + 1) % NS;
+    half(0, STG, 1);
+    // This wave's loads of tile kt+1 have landed (at most the NS-3 tiles
+    // issued after it are in flight): after the barrier tile kt+1 is
+    // readable, and stage (kt-1)%NS, whose last reads every wave waited for
+    // before its first half's MFMAs, takes tile kt+NS-1.
+    wait_vmcnt<(NS - 3) * CF::LPW>();
+    lds_barrier();
+    issue(min(kt + NS - 1, nk - 1), (STG + NS - 1) % NS);
+    half(1, NXT, 0);
+  };
+
   land_args(C);  // C is used only after the K loop
+  // The K % 64 tail is computed first, from stage NS-1, which the ring fills
+  // only after step 0's barrier: its loads share the prologue's latency
+  // instead of adding a round trip at the end.  Chunks and k-rows past K
+  // re-read the last valid ones.
+  if constexpr (TAIL) {
+    const int kr = K - nk * BK;
+    const uint32_t st = lds0 + (NS - 1) * CF::STAGE;
+    const uint16_t* abase = A + (size_t)m0 * lda + (size_t)nk * BK;
+    const uint16_t* bbase = B + (size_t)nk * BK * ldb + n0;
+#pragma unroll
+    for (int n = 0; n < CF::LPW; ++n) {
+      const int ld = wave * CF::LPW + n;
+      if (ld < CF::A_L) {
+        const uint32_t swz = 16u * ((lane % 8) ^ swz_a16w(CF::A_RPL * ld + lane / 8));
+        dma16(abase, off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), st + ld * 1024);
+      } else {
+        const int row = (1024 * (ld - CF::A_L) + 16 * lane) / CF::RB;
+        dma16(bbase, off[n] - (uint32_t)(row - min(row, kr - 1)) * (uint32_t)ldb * 2u, st + ld * 1024);
+      }
+    }
+  }
   // Prologue: tiles 0 .. NS-2 in flight (tiles past the end re-load the
   // last one), wait for tile 0, read its fragments.
+  if (!TAIL || nk > 0) {
 #pragma unroll
-  for (int p = 0; p < NS - 1; ++p) issue(min(p, nk - 1), p);
-  wait_vmcnt<(NS - 2) * CF::LPW>();
-  lds_barrier();
-  read_b(0, 0);
+    for (int p = 0; p < NS - 1; ++p) issue(min(p, nk - 1), p);
+  }
+  if constexpr (TAIL) {
+    if (nk > 0)
+      wait_vmcnt<(NS - 1) * CF::LPW>();
+    else
+      wait_vmcnt<0>();
+    lds_barrier();
 #pragma unroll
-  for (int mf = 0; mf < FM; ++mf) read_a(0, mf);
-  // stage kt % NS and parity kt % 2 repeat every P tiles
-  constexpr int P = NS % 2 == 0 ? NS : 2 * NS;
-  int kt = 0;
-  for (; kt + P <= nk; kt += P) step_period<NS, P>(step, kt);
-  step_tail<NS, P>(step, kt, nk - kt);
+    for (int h = 0; h < 2; ++h) {
+      const bool keep = 32 * h + 8 * kg < K - nk * BK;
+      read_b(NS - 1, h);
+#pragma unroll
+      for (int nf = 0; nf < FN; ++nf) bf[h][nf] = keep_if(keep, bf[h][nf]);
+#pragma unroll
+      for (int mf = 0; mf < FM; ++mf) {
+        read_a(NS - 1, h, mf);
+        af[mf] = keep_if(keep, af[mf]);
+#pragma unroll
+        for (int nf = 0; nf < FN; ++nf) acc[mf][nf] = mfma16<BF16>(bf[h][nf], af[mf], acc[mf][nf]);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage's reads are done before the next barrier frees it
+  }
+  if (!TAIL || nk > 0) {
+    wait_vmcnt<(NS - 2) * CF::LPW>();
+    lds_barrier();
+    read_b(0, 0);
+#pragma unroll
+    for (int mf = 0; mf < FM; ++mf) read_a(0, 0, mf);
+    int kt = 0;
+    for (; kt + NS <= nk; kt += NS) step_period<NS>(step, kt);
+    step_tail<NS>(step, kt, nk - kt);
+  }
   wait_vmcnt<0>();  // no DMA may land in LDS after the workgroup ends
 
   // ---- epilogue: lane holds m = am + 16 mf, n = wn*TN + 16 nf + 4 kg + {0..3}
-  // of the tile.  The tile goes through LDS (bf16 rows padded by 16 bytes)
-  // and is stored as whole rows, each lane 16 contiguous bytes, instead of
-  // 8-byte pieces that the memory system writes back as partial lines.  The
-  // ring is free once every wave is past its last fragment reads. ----
-  constexpr int CROW = CF::BN * 2 + 16;
-  static_assert(CF::BM * CROW <= NS * CF::STAGE, "C tile fits the ring");
-  __syncthreads();
-#pragma unroll
-  for (int mf = 0; mf < FM; ++mf) {
-    const int r = am + 16 * mf;
-#pragma unroll
-    for (int nf = 0; nf < FN; ++nf) {
-      const int c = wn * CF::TN + 16 * nf + 4 * kg;
-      const f32x4& a = acc[mf][nf];
-      *reinterpret_cast<u32x2*>(smem + r * CROW + 2 * c) = u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
-    }
-  }
-  __syncthreads();
-  {
-    constexpr int CPR = CF::BN / 8;     // 16-byte chunks per tile row
-    constexpr int RPI = CF::NT / CPR;   // rows per workgroup-wide store
-    const int t = threadIdx.x;
-    const int cc = t % CPR, r0 = t / CPR;
-    const int gn = n0 + 8 * cc;
-#pragma unroll 4
-    for (int r = r0; r < CF::BM; r += RPI) {
-      const int gm = m0 + r;
-      if (gm < M && gn < N)
-        st128(C + (size_t)gm * ldc + gn, *reinterpret_cast<const u32x4*>(smem + r * CROW + 16 * cc));
-    }
-  }
+  // of the tile ----
+  store_tile_lds<CF::BM, CF::BN, CF::NT, FM, FN>(smem, acc, am, wn * CF::TN + 4 * kg, C, m0, n0, M, N, ldc);
+}
+
+template <int BM, int BN, int WM, int WN, int NS>
+static int launch_dma64(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
+                        hipStream_t stream, int batch = 1, long long sA = 0, long long sB = 0, long long sC = 0) {
+  using CF = D64Cfg<BM, BN, WM, WN, NS>;
+  const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (tiles > 0x7fffffffLL || batch > 65535) return MX_ERR_SHAPE;
+  auto go = [&](auto tail) {
+    constexpr auto kern = gemm_bf16_dma64_kernel<BM, BN, WM, WN, NS, decltype(tail)::value>;
+    MX_RETURN_IF_HIP(lds_limit_once<kern>(NS * CF::STAGE));
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch), dim3(CF::NT), NS * CF::STAGE, stream,
+                       (const uint16_t*)A, (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
+    MX_RETURN_IF_HIP(hipGetLastError());
+    return MX_OK;
+  };
+  return K % CF::BK ? go(std::true_type{}) : go(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -754,7 +418,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_bf16_dma16_kernel(const 
 // ---------------------------------------------------------------------------
 struct S16Cfg {
   static constexpr int BM = 256, BN = 256, BK = 32, BKA = 64;
-  static constexpr int WM = DMA_WM, WN = DMA_WN, NW = WM * WN, NT = 64 * NW;
+  static constexpr int WM = 2, WN = 4, NW = WM * WN, NT = 64 * NW;
   static constexpr int TM = BM / WM, TN = BN / WN;   // wave block
   static constexpr int FM = TM / 16, FN = TN / 16;   // 16x16 fragments
   static constexpr int RA = BKA * 2, RB = BN * 2;    // LDS row bytes (A 128, B 512)
@@ -770,7 +434,6 @@ struct S16Cfg {
   static constexpr int P = 12;                        // steps until slots and parity repeat
   static_assert(LDS <= 160 * 1024 && A_LPW % 2 == 0 && A_LPW >= 2 && B_LPW >= 1, "rings");
 };
-__device__ __forceinline__ int swz_a16w(int m) { return (m >> 1) & 7; }
 
 template <int P, int I = 0, typename Step>
 __device__ __forceinline__ void steps_s(Step& step, int kt) {
@@ -789,6 +452,7 @@ __device__ __forceinline__ void steps_tail_s(Step& step, int kt, int n) {
   }
 }
 
+template <bool TAIL>
 __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const uint16_t* __restrict__ A,
                                                                         const uint16_t* __restrict__ B,
                                                                         uint16_t* __restrict__ C, int M, int N,
@@ -812,7 +476,7 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   const int tm = first_m + (id % per_group) % gsz;
   const int tn = (id % per_group) / gsz;
   const int m0 = tm * CF::BM, n0 = tn * CF::BN;
-  const int nk = K / BK, nka = K / CF::BKA;
+  const int nka = K / CF::BKA, nk = 2 * nka;
 
   // ---- direct-load lane offsets (bytes from the tile's first element).
   // Rows past M / columns past N re-read the last valid ones; their
@@ -921,6 +585,29 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   };
 
   land_args(C);  // C is used only after the K loop
+  // The K % 64 tail is computed first, from A slot 2 and B slots 3 and 2,
+  // which are free until then: its loads share the prologue's latency
+  // instead of adding a round trip at the end.  Chunks and k-rows past K
+  // re-read the last valid ones.
+  const int kr = K - nka * CF::BKA;
+  if constexpr (TAIL) {
+    const uint16_t* abase = A + (size_t)m0 * lda + (size_t)nka * CF::BKA;
+    const uint16_t* bbase = B + (size_t)nka * CF::BKA * ldb + n0;
+#pragma unroll
+    for (int n = 0; n < CF::A_LPW; ++n) {
+      const uint32_t swz = 16u * ((lane % 8) ^ swz_a16w(CF::A_RPL * (wave * CF::A_LPW + n) + lane / 8));
+      dma16(abase, a_off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), lds0 + 2 * CF::A_B + (wave * CF::A_LPW + n) * 1024);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int n = 0; n < CF::B_LPW; ++n) {
+        const int row = CF::B_RPL * (wave * CF::B_LPW + n) + lane / CF::B_CH;
+        const int r0 = h && kr > 32 ? 32 : 0;  // first k-row of the half, if it has any
+        dma16(bbase + (size_t)r0 * ldb, b_off[n] - (uint32_t)(row - min(row, kr - 1 - r0)) * (uint32_t)ldb * 2u,
+              lds0 + CF::B_OFF + (3 - h) * CF::B_B + (wave * CF::B_LPW + n) * 1024);
+      }
+  }
   // Prologue, in the order the waits need: A block 0, B stages 0 and 1,
   // A block 1, B stage 2; then tile 0's fragments.
   issue_a(0, 0, 0);
@@ -929,6 +616,26 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   issue_b(1, 1);
   issue_a(1, 0, 1);
   issue_a(1, 1, 1);
+  if constexpr (TAIL) {
+    wait_vmcnt<2 * CF::A_LPW + 2 * CF::B_LPW>();  // all but A blocks 0, 1 and B stages 0, 1
+    lds_barrier();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const bool keep = 32 * h + 8 * kg < kr;
+      read_b(3 - h, h);
+#pragma unroll
+      for (int nf = 0; nf < FN; ++nf) bf[h][nf] = keep_if(keep, bf[h][nf]);
+#pragma unroll
+      for (int mf = 0; mf < FM; ++mf) {
+        read_a(2, h, mf);
+        af[mf] = keep_if(keep, af[mf]);
+#pragma unroll
+        for (int nf = 0; nf < FN; ++nf) acc[mf][nf] = mfma16<BF16>(bf[h][nf], af[mf], acc[mf][nf]);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slots' reads are done before B stage 2 and step 0 refill them
+    lds_barrier();
+  }
   issue_b(2, 2);
   wait_vmcnt<2 * CF::B_LPW + CF::A_LPW>();  // B stage 1, A block 1 and B stage 2 may be in flight
   lds_barrier();
@@ -940,35 +647,9 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   steps_tail_s<CF::P>(step, kt, nk - kt);
   wait_vmcnt<0>();  // no DMA may land in LDS after the workgroup ends
 
-  // ---- epilogue (as gemm_bf16_dma16_kernel): the tile goes through LDS as
-  // bf16 rows padded by 16 bytes and is stored as whole rows. ----
-  constexpr int CROW = CF::BN * 2 + 16;
-  static_assert(CF::BM * CROW <= CF::LDS, "C tile fits the rings");
-  __syncthreads();
-#pragma unroll
-  for (int mf = 0; mf < FM; ++mf) {
-    const int r = am + 16 * mf;
-#pragma unroll
-    for (int nf = 0; nf < FN; ++nf) {
-      const int c = wn * CF::TN + 16 * nf + 4 * kg;
-      const f32x4& a = acc[mf][nf];
-      *reinterpret_cast<u32x2*>(smem + r * CROW + 2 * c) = u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])};
-    }
-  }
-  __syncthreads();
-  {
-    constexpr int CPR = CF::BN / 8;     // 16-byte chunks per tile row
-    constexpr int RPI = CF::NT / CPR;   // rows per workgroup-wide store
-    const int t = threadIdx.x;
-    const int cc = t % CPR, r0 = t / CPR;
-    const int gn = n0 + 8 * cc;
-#pragma unroll 4
-    for (int r = r0; r < CF::BM; r += RPI) {
-      const int gm = m0 + r;
-      if (gm < M && gn < N)
-        st128(C + (size_t)gm * ldc + gn, *reinterpret_cast<const u32x4*>(smem + r * CROW + 16 * cc));
-    }
-  }
+  // ---- epilogue: lane holds m = am + 16 mf, n = wn*TN + 16 nf + 4 kg + {0..3} ----
+  static_assert(CF::BM * (CF::BN * 2 + 16) <= CF::LDS, "C tile fits the rings");
+  store_tile_lds<CF::BM, CF::BN, CF::NT, FM, FN>(smem, acc, am, wn * CF::TN + 4 * kg, C, m0, n0, M, N, ldc);
 }
 
 static int launch_dma16s(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
@@ -976,44 +657,15 @@ static int launch_dma16s(const void* A, const void* B, void* C, int M, int N, in
   using CF = S16Cfg;
   const long long tiles = (long long)((M + CF::BM - 1) / CF::BM) * ((N + CF::BN - 1) / CF::BN);
   if (tiles > 0x7fffffffLL) return MX_ERR_SHAPE;
-  constexpr auto kern = gemm_bf16_dma16s_kernel;
-  MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(CF::NT), CF::LDS, stream, (const uint16_t*)A,
-                     (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
-}
-
-template <int NS, int WM, int WN, int BM_ = 256, int BN_ = 256>
-static int launch_dma16(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
-                        hipStream_t stream) {
-  using CF = D16Cfg<NS, WM, WN, BM_, BN_>;
-  const long long tiles = (long long)((M + CF::BM - 1) / CF::BM) * ((N + CF::BN - 1) / CF::BN);
-  if (tiles > 0x7fffffffLL) return MX_ERR_SHAPE;
-  const int smem = NS * CF::STAGE;
-  constexpr auto kern = gemm_bf16_dma16_kernel<NS, WM, WN, BM_, BN_>;
-  MX_RETURN_IF_HIP(lds_limit_once<kern>(smem));
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(CF::NT), smem, stream, (const uint16_t*)A,
-                     (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
-}
-
-template <int BM, int BN, int WM, int WN, int KS = 1, int PF = 1>
-static int launch(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
-                  hipStream_t stream, int batch = 1, long long sA = 0, long long sB = 0, long long sC = 0) {
-  using CF = Cfg<BM, BN, WM, WN>;
-  const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-  if (tiles > 0x7fffffffLL || batch > 65535) return MX_ERR_SHAPE;
-  if (!staged_strides_ok<BM>(lda, ldb)) return MX_ERR_SHAPE;
-  const size_t smem = (size_t)KS * 2 * CF::LDS_STAGE;
-  static_assert(KS * 2 * CF::LDS_STAGE <= 160 * 1024, "double buffers fit in the LDS");
-  constexpr auto kern = gemm_bf16_kernel<BM, BN, WM, WN, KS, PF>;
-  MX_RETURN_IF_HIP(lds_limit_once<kern>((int)smem));
-  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch), dim3(CF::NT * KS), smem, stream, (const uint16_t*)A,
-                     (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
+  auto go = [&](auto tail) {
+    constexpr auto kern = gemm_bf16_dma16s_kernel<decltype(tail)::value>;
+    MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
+    hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(CF::NT), CF::LDS, stream, (const uint16_t*)A,
+                       (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
+    MX_RETURN_IF_HIP(hipGetLastError());
+    return MX_OK;
+  };
+  return K % CF::BKA ? go(std::true_type{}) : go(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -1360,7 +1012,7 @@ __device__ __forceinline__ void unroll_n(F&& f) {
   }
 }
 
-template <int MF, int NW, int NSL>
+template <int MF, int NW, int NSL, bool TAIL>
 __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint16_t* __restrict__ A,
                                                                     const uint16_t* __restrict__ B,
                                                                     uint16_t* __restrict__ C, int M, int N, int K,
@@ -1385,17 +1037,14 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
   // A load n: rows 8n + l/8, LDS chunk l%8 taking global chunk (l%8) ^
   // swz(row) (rows past M re-read row M-1); B load n: k-rows 16n + l/4,
   // chunk l%4 (columns past N re-read the last 8 valid ones; never stored).
-  uint32_t a_off[CF::A_L], b_off[CF::B_L];
+  uint32_t a_off[CF::A_L];
 #pragma unroll
   for (int n = 0; n < CF::A_L; ++n) {
     const int row = 8 * n + (lane >> 3);
     a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_s(row));
   }
-#pragma unroll
-  for (int n = 0; n < CF::B_L; ++n) {
-    const int col = min(n0 + 8 * (lane & 3), N - 8) - n0;
-    b_off[n] = (uint32_t)(16 * n + (lane >> 2)) * (uint32_t)ldb * 2u + 2u * col;
-  }
+  const uint32_t b_col_off = 2u * (min(n0 + 8 * (lane & 3), N - 8) - n0);
+  const uint32_t b_off = (uint32_t)(lane >> 2) * (uint32_t)ldb * 2u + b_col_off;  // from k-row 16 n
   auto issue = [&](int i, auto slot_tag) {
     constexpr int I = decltype(slot_tag)::value;
     const int kb = cnt > 0 ? wave + NW * min(i, cnt - 1) : 0;
@@ -1403,7 +1052,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
 #pragma unroll
     for (int n = 0; n < CF::A_L; ++n) dma16(A + (size_t)kb * 64, a_off[n], st + n * 1024);
 #pragma unroll
-    for (int n = 0; n < CF::B_L; ++n) dma16(B + (size_t)kb * 64 * ldb + n0, b_off[n], st + CF::A_B + n * 1024);
+    for (int n = 0; n < CF::B_L; ++n) dma16(B + ((size_t)kb * 64 + 16 * n) * ldb + n0, b_off, st + CF::A_B + n * 1024);
   };
 
   // fragment lane addresses within a slot.  A^T (B operand): row am, chunk
@@ -1420,21 +1069,47 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
 #pragma unroll
   for (int f = 0; f < MF; ++f) acc[f] = f32x16{};
 
-  auto compute = [&](auto slot_tag) {
+  // the first kr k values of a slot count (64: all of them)
+  auto compute = [&](auto slot_tag, int kr) {
     constexpr int I = decltype(slot_tag)::value;
     const uint32_t st = ring + I * CF::SLOT;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       const u32x2 lo = lds_read_tr16_at(st + b_col + 16 * ks * 64);
       const u32x2 hi = lds_read_tr16_at(st + b_col + 16 * ks * 64 + 4 * 64);
-      const u32x4 bt{lo[0], lo[1], hi[0], hi[1]};
+      const bool keep = 16 * ks + 8 * g < kr;
+      const u32x4 bt = keep_if(keep, u32x4{lo[0], lo[1], hi[0], hi[1]});
 #pragma unroll
-      for (int f = 0; f < MF; ++f) acc[f] = mfma32<BF16>(bt, lds_ld128(st + 32 * f * 128 + a_col[ks]), acc[f]);
+      for (int f = 0; f < MF; ++f)
+        acc[f] = mfma32<BF16>(bt, keep_if(keep, lds_ld128(st + 32 * f * 128 + a_col[ks])), acc[f]);
     }
   };
 
   land_args(C);
+  // The K % 64 tail is one more block of the next wave in turn, computed
+  // first, from the slot that the prologue leaves free.  Chunks and k-rows
+  // past K re-read the last valid ones.
+  const int kr = K - kblocks * 64;
+  const bool mine = TAIL && wave == kblocks % NW;
+  if (mine) {
+    const uint32_t st = ring + (NSL - 1) * CF::SLOT;
+#pragma unroll
+    for (int n = 0; n < CF::A_L; ++n) {
+      const uint32_t swz = 16u * ((lane & 7) ^ swz_s(8 * n + (lane >> 3)));
+      dma16(A + (size_t)kblocks * 64, a_off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), st + n * 1024);
+    }
+#pragma unroll
+    for (int n = 0; n < CF::B_L; ++n) {
+      const int r0 = min(16 * n, kr - 1);
+      dma16(B + ((size_t)kblocks * 64 + r0) * ldb + n0,
+            (uint32_t)(min(16 * n + (lane >> 2), kr - 1) - r0) * (uint32_t)ldb * 2u + b_col_off, st + CF::A_B + n * 1024);
+    }
+  }
   unroll_n<NSL - 1>([&](auto i_tag) { issue(decltype(i_tag)::value, i_tag); });
+  if (mine) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"i"((NSL - 1) * CF::VM) : "memory");
+    compute(std::integral_constant<int, NSL - 1>{}, kr);
+  }
   // block i: issue block i + NSL - 1 into the slot block i - 1 used (its
   // reads completed), then wait for block i
   auto step = [&](int i, auto slot_tag) {
@@ -1442,7 +1117,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     issue(i + NSL - 1, std::integral_constant<int, (I + NSL - 1) % NSL>{});
     asm volatile("s_waitcnt vmcnt(%0)" ::"i"((NSL - 1) * CF::VM) : "memory");
-    compute(slot_tag);
+    compute(slot_tag, 64);
   };
   int i = 0;
   for (; i + NSL <= cnt; i += NSL) unroll_n<NSL>([&](auto s_tag) { step(i + decltype(s_tag)::value, s_tag); });
@@ -1477,14 +1152,94 @@ template <int MF, int NSL>
 static int launch_stream(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
                          hipStream_t stream) {
   using CF = StreamCfg<MF, 4, NSL>;
-  constexpr auto kern = gemm_bf16_stream_kernel<MF, 4, NSL>;
-  MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
   const long long grid = (long long)((N + 31) / 32) * ((M + 32 * MF - 1) / (32 * MF));
   if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), CF::LDS, stream, (const uint16_t*)A,
-                     (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
+  auto go = [&](auto tail) {
+    constexpr auto kern = gemm_bf16_stream_kernel<MF, 4, NSL, decltype(tail)::value>;
+    MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), CF::LDS, stream, (const uint16_t*)A,
+                       (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
+    MX_RETURN_IF_HIP(hipGetLastError());
+    return MX_OK;
+  };
+  return K % 64 ? go(std::true_type{}) : go(std::false_type{});
+}
+
+// The kernels of mx_gemm_bf16, and what one launch of each takes in
+// microseconds: fixed + rounds (round + step K/64) + fill (tiles / slots) K/64
+// with rounds = ceil(tiles / slots).  A round of workgroups costs its slowest
+// one (round, step), and more workgroups at once share the L2 and the clock
+// (fill).  Fitted (relative least squares, no negative term) to 228 random
+// shapes, M 1..8192, N and K 512..8192, ragged and whole, each timed on every
+// kernel by graph replay; the kernel picked is on average 0.8% slower than
+// the fastest of the seven, at worst 26% (a single shape, 94x6904x6368).
+enum class Path { None, Stream32, Stream64, T64, T64x128, T128, T128x192, T256 };
+struct Kernel {
+  Path path;
+  int bm, bn, slots;  // tile, workgroups resident at once
+  float fixed, round, step, fill;
+};
+constexpr Kernel kKernels[] = {
+    {Path::Stream32, 32, 32, 256, 1.393f, 1.922f, 0.097f, 0.064f},
+    {Path::Stream64, 64, 32, 256, 1.048f, 2.553f, 0.121f, 0.095f},
+    {Path::T64, 64, 64, 512, 2.301f, 1.117f, 0.184f, 0.298f},
+    {Path::T64x128, 64, 128, 256, 2.332f, 1.946f, 0.254f, 0.111f},
+    {Path::T128, 128, 128, 256, 1.749f, 2.956f, 0.353f, 0.187f},
+    {Path::T128x192, 128, 192, 256, 1.803f, 3.855f, 0.499f, 0.225f},
+    {Path::T256, 256, 256, 256, 2.082f, 6.139f, 0.977f, 0.532f},
+};
+
+// batch items of a strided-batched product (the tiled kernels only), or 0 for
+// a single one.
+static Path gemm_path(int M, int N, int K, int lda, int ldb, int batch) {
+  Path best = Path::None;
+  double least = 0;
+  for (const Kernel& k : kKernels) {
+    const bool stream = k.bn == 32;
+    const bool plain = stream || k.path == Path::T256;  // no batch, and at least one whole 64-deep K block
+    if (plain && (K < 64 || batch > 0)) continue;
+    // The lane offsets of the direct loads are 32-bit: bm rows of A, and the
+    // k-rows of B that share a base (16, 32 or 64), span less than 4 GiB.
+    const long long brows = stream ? 16 : k.path == Path::T256 ? 32 : K < 64 ? K : 64;
+    if ((long long)lda * 2 * k.bm > 0xffffffffLL || (long long)ldb * 2 * (brows - 1) + 2 * k.bn > 0xffffffffLL) continue;
+    const double tiles = (double)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn) * (batch > 0 ? batch : 1);
+    const double rounds = __builtin_ceil(tiles / k.slots), kb = K / 64.0;
+    const double t = k.fixed + rounds * (k.round + k.step * kb) + k.fill * kb * tiles / k.slots;
+    if (best == Path::None || t < least) {
+      best = k.path;
+      least = t;
+    }
+  }
+  return best;
+}
+
+static int launch_tiled(Path path, const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb,
+                        int ldc, hipStream_t s, int batch, long long sA, long long sB, long long sC) {
+  switch (path) {
+    case Path::T64: return launch_dma64<64, 64, 2, 2, 4>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+    case Path::T64x128: return launch_dma64<64, 128, 2, 4, 6>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+    case Path::T128: return launch_dma64<128, 128, 2, 4, 5>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+    case Path::T128x192: return launch_dma64<128, 192, 2, 4, 4>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+    default: return MX_ERR_SHAPE;
+  }
+}
+
+// The leading dimensions the interface takes: with K % 32 != 0 or a small
+// grid, lda * 2 * BM (BM rows per tile: 256, 128 or 64) and ldb * 2 * 64 below
+// 2^31; otherwise spans below 4 GiB.
+static bool strides_ok(int M, int N, int K, int lda, int ldb) {
+  const long long la = lda, lb = ldb, four_g = 0xffffffffLL;
+  auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t); };
+  const bool span64 = la * 2 * 64 <= four_g && lb * 2 * 64 <= four_g;
+  if (((M <= 64 && N >= 256) || (tiles(64) <= 64 && K >= 512)) && K % 64 == 0 && span64) return true;
+  const bool big = tiles(256) >= 256 || 13 * ((tiles(256) + 255) / 256) < 5 * ((tiles(128) + 255) / 256);
+  const bool b_fits = lb * 2 * 31 + 512 <= four_g;
+  if (big && K % 32 == 0 && la * 2 * 256 <= four_g) return b_fits;
+  if (tiles(256) >= 512) return strides_2g<256>(lda, ldb);
+  if (tiles(128) >= 256 && K % 32 == 0 && la * 2 * 128 <= four_g) return b_fits;
+  if (tiles(128) >= 256) return strides_2g<128>(lda, ldb);
+  if (tiles(64) <= 256 && K >= 512 && M % 64 == 0 && N % 64 == 0 && K % 128 == 0 && span64) return true;
+  return strides_2g<64>(lda, ldb);
 }
 
 }  // namespace gemm
@@ -1498,69 +1253,24 @@ extern "C" int mx_gemm_bf16(const void* A, const void* B, void* C, int M, int N,
   if ((K % 8) || (N % 8) || (lda % 8) || (ldb % 8) || (ldc % 8)) return MX_ERR_ALIGN;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) return MX_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
-  // Stream the weights with whole 64-deep K blocks (32-bit lane offsets: 64
-  // rows of A and 64 k-rows of B span < 4 GiB) for decode-sized M against
-  // at least 256 columns, and for any product with at most 64 tiles of
-  // 64x64 and K >= 512, which the tiled kernels cannot spread over the CUs
-  // (graph-replayed: 256x512x4096 17.6 -> 9.4 us, 96x512x8192 44.9 -> 14.4
-  // us; 1024^3, 256 such tiles, stays tiled: 8.3 against 10.6 us).
-  const long long tiles64s = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  if (((M <= 64 && N >= 256) || (tiles64s <= 64 && K >= 512)) && K % 64 == 0 &&
-      (long long)lda * 2 * 64 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL)
-    return M <= 32 ? mx::gemm::launch_stream<1, 4>(A, B, C, M, N, K, lda, ldb, ldc, s)
-                   : mx::gemm::launch_stream<2, 3>(A, B, C, M, N, K, lda, ldb, ldc, s);
-  const long long tiles256 = (long long)((M + 255) / 256) * ((N + 255) / 256);
-  const long long tiles128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  // Rounds of 256 workgroups: a round of 256x256 tiles of the direct-load
-  // kernel takes ~2.6 times a round of its 128x128 tiles at the same K
-  // (measured 2.2-3.0 at 2048-4096), so 256x256 also wins below one tile
-  // per CU when 128x128 tiles would need more than 2.6 times the rounds
-  // (3072^3: 69 vs 78 us; 2560^3 stays on 128x128: 48 vs 59 us).
-  const long long r256 = (tiles256 + 255) / 256, r128 = (tiles128 + 255) / 256;
-  const bool big = tiles256 >= 256 || 13 * r256 < 5 * r128;
-  // Whole K tiles: the direct-load kernel (its lane offsets are 32-bit: 256
-  // rows of A must span < 4 GiB).
-  if (big && K % 64 == 0 && (long long)lda * 2 * 256 <= 0xffffffffLL && (long long)ldb * 2 * 32 <= 0xffffffffLL)
-    return mx::gemm::launch_dma16s(A, B, C, M, N, K, lda, ldb, ldc, s);
-  if (big && K % mx::gemm::DMA_BK == 0 && (long long)lda * 2 * 256 <= 0xffffffffLL)
-    return mx::gemm::launch_dma16<mx::gemm::DMA_NS, mx::gemm::DMA_WM, mx::gemm::DMA_WN>(A, B, C, M, N, K, lda, ldb,
-                                                                                          ldc, s);
-  // Otherwise: register-staged kernels, big tiles when they still cover the
-  // 256 CUs twice, else smaller tiles for parallelism.
-  if (tiles256 >= 512) return mx::gemm::launch<256, 256, 2, 4>(A, B, C, M, N, K, lda, ldb, ldc, s);
-  // At least one 128x128 tile per CU and whole K tiles: the direct-load
-  // kernel on 128x128 tiles, whose 16 KB stages allow a deeper ring.
-  if (tiles128 >= 256 && K % mx::gemm::DMA_BK == 0 && (long long)lda * 2 * 128 <= 0xffffffffLL)
-    return mx::gemm::launch_dma16<mx::gemm::D128_NS, 2, mx::gemm::D128_WN, 128, 128>(A, B, C, M, N, K, lda, ldb,
-                                                                                      ldc, s);
-  if (tiles128 >= 256) return mx::gemm::launch<128, 128, 2, 2>(A, B, C, M, N, K, lda, ldb, ldc, s);
-  // About one 64x64 tile per CU or fewer and a long K (e.g. 1024^3): split
-  // K between two wave groups of each workgroup.
-  const long long tiles64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
-  // ... with whole 64x64 tiles and 128-deep K chunks: the direct-load ring
-  // (32-bit lane offsets: 64 rows of A and 64 k-rows of B span < 4 GiB).
-  if (tiles64 <= 256 && K >= 512 && M % 64 == 0 && N % 64 == 0 && K % 128 == 0 &&
-      (long long)lda * 2 * 64 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL)
-    return mx::gemm::launch_sdma(A, B, C, M, N, K, lda, ldb, ldc, s);
-  if (tiles64 <= 256 && K >= 512) return mx::gemm::launch<64, 64, 2, 2, 2, 2>(A, B, C, M, N, K, lda, ldb, ldc, s);
-  return mx::gemm::launch<64, 64, 2, 2, 1, 2>(A, B, C, M, N, K, lda, ldb, ldc, s);
+  using namespace mx::gemm;
+  if (!strides_ok(M, N, K, lda, ldb)) return MX_ERR_SHAPE;
+  const Path path = gemm_path(M, N, K, lda, ldb, 0);
+  switch (path) {
+    case Path::Stream32: return launch_stream<1, 4>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::Stream64: return launch_stream<2, 3>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::T256: return launch_dma16s(A, B, C, M, N, K, lda, ldb, ldc, s);
+    default: return launch_tiled(path, A, B, C, M, N, K, lda, ldb, ldc, s, 1, 0, 0, 0);
+  }
 }
 
 namespace mx {
 namespace gemm {
 
-// Which kernel mx_gemm_bf16_batched runs for these sizes.
-enum class BatchedPath { SmallM, T128, T64 };
-
-static BatchedPath batched_path(int batch, int M, int N, int K, int lda, int ldb) {
-  // Decode-sized items (M <= 32, whole 64-deep K chunks): the
-  // weight-streaming small-M kernel.  Its lane offsets are 32-bit.
-  if (M <= 32 && K % 64 == 0 && (long long)lda * 2 * 32 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL)
-    return BatchedPath::SmallM;
-  // Otherwise the register-staged kernel with tiles sized to the item.
-  const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128) * batch;
-  if (M >= 128 && t128 >= 256) return BatchedPath::T128;
-  return BatchedPath::T64;
+// Decode-sized items (M <= 32, whole 64-deep K chunks) run the
+// weight-streaming small-M kernels.  Their lane offsets are 32-bit.
+static bool batched_small(int M, int K, int lda, int ldb) {
+  return M <= 32 && K % 64 == 0 && (long long)lda * 2 * 32 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL;
 }
 
 // Every check mx_gemm_bf16_batched makes before it launches, the grid
@@ -1575,18 +1285,11 @@ int batched_check(const void* A, const void* B, void* C, int batch, int M, int N
   if ((K % 8) || (N % 8) || (lda % 8) || (ldb % 8) || (ldc % 8)) return MX_ERR_ALIGN;
   if ((strideA % 8) || (strideB % 8) || (strideC % 8)) return MX_ERR_ALIGN;
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) return MX_ERR_ALIGN;
-  long long grid = 0;
-  switch (batched_path(batch, M, N, K, lda, ldb)) {
-    case BatchedPath::SmallM: grid = (long long)batch * ((N + 31) / 32); break;  // widest grid of the three widths
-    case BatchedPath::T128:
-      grid = (long long)((M + 127) / 128) * ((N + 127) / 128);
-      if (!staged_strides_ok<128>(lda, ldb)) return MX_ERR_SHAPE;
-      break;
-    case BatchedPath::T64:
-      grid = (long long)((M + 63) / 64) * ((N + 63) / 64);
-      if (!staged_strides_ok<64>(lda, ldb)) return MX_ERR_SHAPE;
-      break;
-  }
+  const auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t); };
+  const bool small = batched_small(M, K, lda, ldb);
+  if (!small && !(M >= 128 && tiles(128) * batch >= 256 ? strides_2g<128>(lda, ldb) : strides_2g<64>(lda, ldb)))
+    return MX_ERR_SHAPE;
+  const long long grid = small ? (long long)batch * ((N + 31) / 32) : tiles(64);  // widest grid of the kernels
   return grid > 0x7fffffffLL ? MX_ERR_SHAPE : MX_OK;
 }
 
@@ -1599,12 +1302,8 @@ extern "C" int mx_gemm_bf16_batched(const void* A, const void* B, void* C, int b
   using namespace mx::gemm;
   if (const int e = batched_check(A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC)) return e;
   hipStream_t s = (hipStream_t)stream;
-  switch (batched_path(batch, M, N, K, lda, ldb)) {
-    case BatchedPath::SmallM:
-      return launch_smallm(A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, s);
-    case BatchedPath::T128:
-      return launch<128, 128, 2, 2>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, strideA, strideB, strideC);
-    default:
-      return launch<64, 64, 2, 2, 1, 2>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, strideA, strideB, strideC);
-  }
+  if (batched_small(M, K, lda, ldb))
+    return launch_smallm(A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, s);
+  return launch_tiled(gemm_path(M, N, K, lda, ldb, batch), A, B, C, M, N, K, lda, ldb, ldc, s, batch, strideA, strideB,
+                      strideC);
 }

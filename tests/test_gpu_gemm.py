@@ -276,3 +276,74 @@ def test_batched_vs_oracle(ops, bmnk):
         ref = ogemm.gemm_ref(a[i], b[i])
         assert normwise_rel_err(c[i], ref) <= TOL
         assert torch.all((c[i].float() - ref).abs() <= 0.2 + 0.05 * ref.abs())
+
+
+def _check_elementwise(c, a, b):
+    """|C - A.B| within one bf16 rounding (2^-8 relative) plus fp32 sums of K
+    terms (K 2^-24 of the sum of magnitudes), against a 64-bit product."""
+    a64, b64 = a.double(), b.double()
+    ref = a64 @ b64
+    bound = ref.abs() * 2.0 ** -8 + (a64.abs() @ b64.abs()) * (a.shape[1] * 2.0 ** -24) + 1e-30
+    worst = ((c.double() - ref).abs() / bound).max().item()
+    assert worst <= 1.0, f"{worst:.2f} times the bound"
+
+
+# every kernel of the dispatch: 32- and 64-row streams, 64x64, 64x128,
+# 128x128, 128x192 and 256x256 tiles, with K tails on both sides of 32, K
+# below one 64-deep block, a single block, and edges off the tiles
+RAGGED_K = [(1, 8, 8), (16, 520, 72), (33, 264, 520), (1, 1024, 2056), (50, 5288, 2168), (100, 3200, 1800),
+            (129, 200, 24), (300, 1104, 656), (129, 136, 40), (500, 1496, 1048), (1315, 840, 1128),
+            (777, 3592, 200), (2000, 2040, 264), (554, 7384, 136), (607, 7040, 104), (3500, 1032, 16),
+            (1937, 7024, 104), (4000, 4040, 72), (4096, 4096, 152)]
+
+
+@pytest.mark.parametrize("mnk", RAGGED_K)
+def test_any_k_on_every_kernel(ops, mnk):
+    """A and B sit inside wider buffers filled with NaN, so anything read past
+    K, N or M that reached a sum would show; C's surroundings stay untouched."""
+    m, n, k = mnk
+    announce(f"gemm_bf16 {m}x{n}x{k} any K")
+    lib = import_submodule("_lib")
+    a, b = (t.cuda() for t in inputs.gemm_inputs(shapes.GemmShape("t", m, n, k)))
+    wide = lambda r, c: torch.full((r + 2, c + 16), float("nan"), dtype=torch.bfloat16, device="cuda")
+    aw, bw, cw = wide(m, k), wide(k, n), torch.full((m + 2, n + 16), 7.0, dtype=torch.bfloat16, device="cuda")
+    aw[:m, :k], bw[:k, :n] = a, b
+    lib.call("mx_gemm_bf16", aw.data_ptr(), bw.data_ptr(), cw.data_ptr(), m, n, k, k + 16, n + 16, n + 16, 0)
+    torch.cuda.synchronize()
+    _check_elementwise(cw[:m, :n], a, b)
+    assert torch.all(cw[m:] == 7.0) and torch.all(cw[:, n:] == 7.0)
+    c = ops.gemm_bf16(a, b)
+    torch.cuda.synchronize()
+    assert torch.equal(c, cw[:m, :n])
+
+
+@pytest.mark.parametrize("mnk", [(40, 600, 328), (300, 1104, 264), (700, 1400, 520), (2000, 2040, 264), (4000, 4040, 104)])
+def test_infinity_in_the_last_k_row(ops, mnk):
+    """The K tail re-reads the last k-row for the missing ones: an infinity
+    there counts once, against zeros it gives NaN only where A holds a zero."""
+    m, n, k = mnk
+    announce(f"gemm_bf16 {m}x{n}x{k} infinity in the last k-row")
+    a, b = (t.cuda() for t in inputs.gemm_inputs(shapes.GemmShape("t", m, n, k)))
+    b[-1, 3] = float("inf")
+    a[::7, -1] = 0.0
+    c = ops.gemm_bf16(a, b)
+    torch.cuda.synchronize()
+    want = torch.where(a[:, -1] == 0, float("nan"), torch.sign(a[:, -1].float()) * float("inf"))
+    assert torch.equal(c[:, 3].float().nan_to_num(nan=123.0), want.nan_to_num(nan=123.0))
+    assert torch.isfinite(c[:, :3].float()).all() and torch.isfinite(c[:, 4:].float()).all()
+
+
+@pytest.mark.parametrize("bmnk", [(5, 40, 1000, 72), (16, 48, 128, 512), (3, 300, 264, 136), (40, 200, 640, 136),
+                                  (30, 600, 400, 104), (2, 33, 8, 8), (70, 130, 200, 24)])
+def test_batched_larger_items(ops, bmnk):
+    """Batched items with more than 32 rows, or a K that is no whole number of
+    64-deep chunks, run the tiled kernels over the batch."""
+    nb, m, n, k = bmnk
+    announce(f"gemm_bf16_batched {nb}x{m}x{n}x{k}")
+    g = torch.Generator().manual_seed(nb + m + n + k)
+    a = (torch.rand((nb, m, k), generator=g) * 2 - 1).to(torch.bfloat16).cuda()
+    b = (torch.rand((nb, k, n), generator=g) * 2 - 1).to(torch.bfloat16).cuda()
+    c = ops.gemm_bf16_batched(a, b)
+    torch.cuda.synchronize()
+    for i in range(nb):
+        _check_elementwise(c[i], a[i], b[i])
