@@ -53,8 +53,11 @@ def common_flags() -> list[str]:
 # the score MFMAs write VGPRs and only the P.V accumulators, issued as
 # inline asm, live in AGPRs.  The kernels with at most 256 registers
 # already get the VGPR form.
+# mla_decode_few.hip: its kernel may use more than 256 registers (one wave per
+# SIMD), and the AGPR form would copy the accumulators on every block.
 SOURCE_FLAGS = {
     "gqa_fwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "mla_decode_few.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

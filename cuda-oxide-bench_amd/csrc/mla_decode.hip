@@ -38,14 +38,11 @@
 //    the log-sum-exp rule.  With one split, O is written directly.
 #include <type_traits>
 
-#include "mx_common.h"
+#include "mla_common.h"
 
 namespace mx {
 namespace mla {
 
-constexpr int DQK = 576;
-constexpr int DV = 512;
-constexpr int ROW_B = DQK * 2;          // 1152 bytes per cache row in HBM
 constexpr int HPW = 32;                 // heads per score wave
 constexpr int NWAVES = 4;
 constexpr int NT = 64 * NWAVES;
@@ -67,8 +64,6 @@ constexpr int F_OFF = C_OFF + 2 * NWAVES * 32 * 4;     // rescale flags: [2 buf]
 constexpr int L_OFF = F_OFF + 2 * NWAVES * 4;          // final row sums: [4 group][32] fp32
 constexpr int LDS_BYTES = L_OFF + NWAVES * 32 * 4;
 constexpr int Q_WAVE_B = HPW * (1024 + 128);            // Q staging per wave (prologue only)
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLazy = 16.0f;          // log2 headroom before a rescale
 static_assert(BT * DQK / 8 == 64 * NWAVES * LPW, "a stage splits into whole wave loads");
 static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
 static_assert(NWAVES * Q_WAVE_B <= LDS_BYTES, "Q staging fits the LDS allocation");
@@ -95,18 +90,20 @@ static_assert(DV / 16 == 32 && (DQK - DV) / 16 == 4, "Q fragment split: 32 laten
 __device__ __forceinline__ int swz_lat(int t) { return ((t & 3) << 2) | ((t >> 2) & 3); }
 __device__ __forceinline__ int swz_rope(int t) { return (t >> 1) & 7; }
 
-struct Split {
-  int nsplit;
-  int tps;  // tokens per split (multiple of the stage)
-};
+inline bool few_heads(int H) { return H <= kFewHeads; }
+inline int tile_heads(int H) { return few_heads(H) ? kFewTile : HPW; }  // heads per partial tile
 
-__host__ __device__ inline Split pick_split(int B, int H, int T) {
+inline Split pick_split(int B, int H, int T) {
+  if (few_heads(H)) return few_split(B, T);
   const int hg = (H + HPG - 1) / HPG;
   const int nblk = (T + BT - 1) / BT;
-  // Aim for >= 256 workgroups (one per CU) with at least 2 stages per split.
-  int ns = 1;
-  while ((long long)B * hg * ns < 256 && ns * 2 <= nblk / 2) ns *= 2;
-  const int blocks_per = (nblk + ns - 1) / ns;
+  // As many splits as one round of workgroups takes (one per CU), of at least
+  // two stages each.  A round more costs more than idle CUs: B48 H128 T3000
+  // takes 61 us with 5 splits (240 workgroups) and 79 us with 8 (384).
+  long long ns = 256 / ((long long)B * hg);
+  if (ns > nblk / 2) ns = nblk / 2;
+  if (ns < 1) ns = 1;
+  const int blocks_per = (int)((nblk + ns - 1) / ns);
   Split s;
   s.nsplit = (nblk + blocks_per - 1) / blocks_per;
   s.tps = blocks_per * BT;
@@ -479,26 +476,30 @@ __global__ __launch_bounds__(NT, 1) void mla_decode_kernel(const uint16_t* __res
 // split slices (measured: 512 took B4 H128 T4096 from 27.9 to 25.9 us; at
 // one slice 256 measured 0.5-2 us faster than 512 at B16-B64).
 constexpr int CMB_WG_ONE = 256, CMB_WG_MANY = 512;
-constexpr int CMB_ET = VT * 4 * 32;  // element-threads per (b, 32-head group) tile = 2048
 
-template <int SG>
+template <int SG, int TH>
 struct CmbCfg {
+  static constexpr int CMB_ET = DV * TH / 8;  // element-threads per (b, TH-head) tile
   // Threads per workgroup: with split slices, larger workgroups cover more
   // output elements each, so fewer of them stage the same (m, l) pairs.
   static constexpr int WG = SG == 1 ? CMB_WG_ONE : CMB_WG_MANY;
   static constexpr int ET = WG / SG;         // element-threads per workgroup
   static constexpr int PER = CMB_ET / ET;    // workgroups per tile
   static constexpr int MAXS = SG == 1 ? 32 : 256;  // most splits; their (m, l) are staged in LDS (8 or 64 KB)
-  static constexpr int MXS = WG / 16;        // slices of the splits in the per-head max
+  static constexpr int MXS = 2 * WG / TH;    // slices of the splits in the per-head max
+  static constexpr int ML_V = MAXS * TH / 2, RED_V = SG > 1 ? WG * 10 / 4 : 0;
+  static constexpr int LDS_V = ML_V > RED_V ? ML_V : RED_V;  // the (m, l) pairs, then the slices' sums
   static_assert(WG % 256 == 0 && WG <= 1024 && CMB_ET % ET == 0, "merge workgroup size");
 };
 
-template <int SG>
-__global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint32_t* __restrict__ ws_o,
+template <int SG, int TH>
+__global__ __launch_bounds__((CmbCfg<SG, TH>::WG)) void mla_combine_kernel(const uint32_t* __restrict__ ws_o,
                                                             const float* __restrict__ ws_ml,
                                                             uint16_t* __restrict__ O, int H, int nsplit) {
-  using CF = CmbCfg<SG>;
-  const int HW = (H + HPW - 1) / HPW;
+  using CF = CmbCfg<SG, TH>;
+  constexpr int HP = TH / 2;                    // head pairs of a tile
+  constexpr size_t TILE = (size_t)DV * TH / 2;  // dwords of a partial tile
+  const int HW = (H + TH - 1) / TH;
   const int gi = blockIdx.x / CF::PER;          // b * HW + hw
   const int part = blockIdx.x % CF::PER;
   const int b = gi / HW, hw = gi % HW;
@@ -506,20 +507,20 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
   const int idx = part * CF::ET + (int)threadIdx.x % CF::ET;  // slot * 32 + lane pair
   const int lp = idx & 31, slot = idx >> 5;
   const int lane0 = 2 * lp;                     // lanes lane0, lane0 + 1
-  const int l32 = lane0 & 31, hsel = lane0 >> 5;
+  const int lh = lane0 % TH, quad = lane0 / TH;  // head of lane0 in the tile, column quad within the slot
   const size_t g0 = (size_t)b * nsplit * HW + hw;  // tile of split 0; split stride HW
-  // The (m, l) pairs of the tile's 32 heads for every split (256 B per
+  // The (m, l) pairs of the tile's heads for every split (8 TH bytes per
   // split) are read once per workgroup into LDS, eight loads in flight per
   // thread; the host keeps nsplit <= MAXS.
-  __shared__ f32x4 ml_lds[CF::MAXS * 16];
-  __shared__ float2 mx_part[CF::MXS][16];  // [split residue mod MXS][head pair]: partial maxima
-  const int n4 = nsplit * 16;
+  __shared__ f32x4 ml_lds[CF::LDS_V];
+  __shared__ float2 mx_part[CF::MXS][HP];  // [split residue mod MXS][head pair]: partial maxima
+  const int n4 = nsplit * HP;
   for (int base = 0; base < n4; base += 8 * CF::WG) {
     f32x4 v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = base + u * CF::WG + (int)threadIdx.x;
-      if (i < n4) v[u] = *reinterpret_cast<const f32x4*>(ws_ml + (g0 + (size_t)(i >> 4) * HW) * 64 + 4 * (i & 15));
+      if (i < n4) v[u] = *reinterpret_cast<const f32x4*>(ws_ml + (g0 + (size_t)(i / HP) * HW) * (2 * TH) + 4 * (i % HP));
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -529,21 +530,21 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
   }
   __syncthreads();
   {  // per-head maxima over the splits: MXS threads per head pair
-    const int hp = threadIdx.x & 15, j = threadIdx.x >> 4;
+    const int hp = threadIdx.x % HP, j = threadIdx.x / HP;
     float2 m{-1e30f, -1e30f};
     for (int t = j; t < nsplit; t += CF::MXS) {
-      const f32x4 x = ml_lds[t * 16 + hp];
+      const f32x4 x = ml_lds[t * HP + hp];
       m.x = fmaxf(m.x, x[0]);
       m.y = fmaxf(m.y, x[2]);
     }
     mx_part[j][hp] = m;
   }
   __syncthreads();
-  auto mlv_of = [&](int t) { return ml_lds[t * 16 + (l32 >> 1)]; };  // (m, l) of heads l32, l32 + 1 in split t
+  auto mlv_of = [&](int t) { return ml_lds[t * HP + (lh >> 1)]; };  // (m, l) of heads lh, lh + 1 in split t
   float2 mmax{-1e30f, -1e30f};
 #pragma unroll
   for (int j = 0; j < CF::MXS; ++j) {
-    const float2 x = mx_part[j][l32 >> 1];
+    const float2 x = mx_part[j][lh >> 1];
     mmax.x = fmaxf(mmax.x, x.x);
     mmax.y = fmaxf(mmax.y, x.y);
   }
@@ -551,8 +552,8 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
   const int s0 = (int)(((long long)nsplit * sg) / SG), s1 = (int)(((long long)nsplit * (sg + 1)) / SG);
   f32x4 o0{0.f, 0.f, 0.f, 0.f}, o1{0.f, 0.f, 0.f, 0.f};
   float l0 = 0.f, l1 = 0.f;
-  const uint32_t* po = ws_o + g0 * PT_U32 + ((size_t)slot * 64 + lane0) * 2;
-  const size_t sstride = (size_t)HW * PT_U32;
+  const uint32_t* po = ws_o + g0 * TILE + ((size_t)slot * 64 + lane0) * 2;
+  const size_t sstride = HW * TILE;
   auto acc1 = [&](const u32x4 p, const f32x4 mlv) {
     const float w0 = mlv[1] * __builtin_amdgcn_exp2f(mlv[0] - mmax.x);
     const float w1 = mlv[3] * __builtin_amdgcn_exp2f(mlv[2] - mmax.y);
@@ -564,6 +565,8 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
                      bf16_bits_to_f32(p[3] & 0xffffu), bf16_bits_to_f32(p[3] >> 16)};
   };
   // Eight splits per batch of loads: all independent, issued together.
+  // A last, partial batch re-reads its last split in place of the missing
+  // ones, so that it too costs one round trip.
   int s = s0;
   for (; s + 8 <= s1; s += 8) {
     u32x4 p[8];
@@ -576,7 +579,14 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc1(p[u], mlv[u]);
   }
-  for (; s < s1; ++s) acc1(ld128(po + (size_t)s * sstride), mlv_of(s));
+  if (s < s1) {
+    u32x4 p[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u) p[u] = ld128(po + (size_t)min(s + u, s1 - 1) * sstride);
+#pragma unroll
+    for (int u = 0; u < 7; ++u)
+      if (s + u < s1) acc1(p[u], mlv_of(s + u));
+  }
   if constexpr (SG > 1) {
     // the slices' sums meet in LDS (reusing the (m, l) staging area)
     __syncthreads();
@@ -599,10 +609,10 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
     l0 = t[8];
     l1 = t[9];
   }
-  const int vt = slot >> 2, i = slot & 3;
-  const int head0 = hw * HPW + l32;
+  // a slot is 64 / TH column quads: 8 columns (TH = 32) or 16 (TH = 16)
+  const int head0 = hw * TH + lh;
   const float inv0 = l0 > 0.f ? 1.f / l0 : 0.f, inv1 = l1 > 0.f ? 1.f / l1 : 0.f;
-  uint16_t* orow = O + ((size_t)b * H + head0) * DV + 32 * vt + 8 * i + 4 * hsel;
+  uint16_t* orow = O + ((size_t)b * H + head0) * DV + 4 * (64 / TH) * slot + 4 * quad;
   if (head0 < H)
     st64(orow, u32x2{pack_bf16x2(o0[0] * inv0, o0[1] * inv0), pack_bf16x2(o0[2] * inv0, o0[3] * inv0)});
   if (head0 + 1 < H)
@@ -611,29 +621,42 @@ __global__ __launch_bounds__(CmbCfg<SG>::WG) void mla_combine_kernel(const uint3
 
 // Split slices per merge element: about 32 splits per thread at most.
 inline int combine_sg(int nsplit) { return nsplit >= 128 ? 8 : nsplit >= 64 ? 4 : nsplit >= 32 ? 2 : 1; }
-inline int combine_max_splits(int nsplit) { return combine_sg(nsplit) == 1 ? CmbCfg<1>::MAXS : CmbCfg<8>::MAXS; }
-inline int combine_per(int sg) {  // workgroups per (b, 32-head) tile
-  return sg == 1 ? CmbCfg<1>::PER : sg == 2 ? CmbCfg<2>::PER : sg == 4 ? CmbCfg<4>::PER : CmbCfg<8>::PER;
+constexpr int kMaxSplits = CmbCfg<8, HPW>::MAXS;
+
+// f(integral_constant SG, integral_constant TH) for this merge.
+template <typename F>
+static auto with_combine(int nsplit, int th, F&& f) {
+  auto by_sg = [&](auto t) {
+    switch (combine_sg(nsplit)) {
+      case 1: return f(std::integral_constant<int, 1>{}, t);
+      case 2: return f(std::integral_constant<int, 2>{}, t);
+      case 4: return f(std::integral_constant<int, 4>{}, t);
+      default: return f(std::integral_constant<int, 8>{}, t);
+    }
+  };
+  return th == HPW ? by_sg(std::integral_constant<int, HPW>{}) : by_sg(std::integral_constant<int, kFewTile>{});
 }
-inline long long combine_grid(int B, int HW, int nsplit) {
-  return (long long)B * HW * combine_per(combine_sg(nsplit));
+static long long combine_grid(int B, int H, int nsplit) {
+  const int th = tile_heads(H);
+  const long long tiles = (long long)B * ((H + th - 1) / th);
+  return tiles * with_combine(nsplit, th, [](auto sg, auto t) { return CmbCfg<decltype(sg)::value, decltype(t)::value>::PER; });
 }
 
 inline size_t workspace_bytes(int B, int H, int T) {
   const Split sp = pick_split(B, H, T);
   if (sp.nsplit <= 1) return 0;
-  const size_t HW = (size_t)(H + HPW - 1) / HPW;
-  return (size_t)B * sp.nsplit * HW * (PT_U32 * sizeof(uint32_t) + 2 * HPW * sizeof(float));
+  const int th = tile_heads(H);
+  const size_t tiles = (size_t)B * sp.nsplit * ((H + th - 1) / th);
+  return tiles * ((size_t)DV * th * 2 + 2 * th * sizeof(float));
 }
 
 // Grid limits of the decode and combine launches.
 static int check_grid(int B, int H, int T) {
   const Split sp = pick_split(B, H, T);
   const long long HGB = (H + HPG - 1) / HPG;
-  const long long HW = (H + HPW - 1) / HPW;
-  const long long grid = (long long)B * HGB * sp.nsplit;
-  if (grid > 0x7fffffffLL || combine_grid(B, (int)HW, sp.nsplit) > 0x7fffffffLL) return MX_ERR_SHAPE;
-  if (sp.nsplit > combine_max_splits(sp.nsplit)) return MX_ERR_SHAPE;  // pick_split keeps nsplit <= 256
+  const long long grid = B * HGB * sp.nsplit;
+  if (grid > 0x7fffffffLL || combine_grid(B, H, sp.nsplit) > 0x7fffffffLL) return MX_ERR_SHAPE;
+  if (sp.nsplit > kMaxSplits) return MX_ERR_SHAPE;  // pick_split keeps nsplit <= 256
   return MX_OK;
 }
 
@@ -642,24 +665,29 @@ static int check_grid(int B, int H, int T) {
 static int launch_decode(const void* Q, const void* Qr, int q_ld, int qr_ld, const void* KV, void* O, int B, int H,
                          int T, float scale, void* workspace, hipStream_t s) {
   const Split sp = pick_split(B, H, T);
+  const int th = tile_heads(H);
   const long long HGB = (H + HPG - 1) / HPG;
-  const long long HW = (H + HPW - 1) / HPW;
-  const long long grid = (long long)B * HGB * sp.nsplit;
   uint32_t* ws_o = (uint32_t*)workspace;
-  float* ws_ml = sp.nsplit > 1 ? reinterpret_cast<float*>(ws_o + (size_t)B * sp.nsplit * HW * PT_U32) : nullptr;
-  MX_RETURN_IF_HIP(lds_limit_once<mla_decode_kernel>(LDS_BYTES));
-  hipLaunchKernelGGL(mla_decode_kernel, dim3((unsigned)grid), dim3(NT), LDS_BYTES, s, (const uint16_t*)Q,
-                     (const uint16_t*)Qr, (const uint16_t*)KV, (uint16_t*)O, ws_o, ws_ml, B, H, T, scale * kLog2e,
-                     sp.nsplit, sp.tps, q_ld, qr_ld);
-  MX_RETURN_IF_HIP(hipGetLastError());
+  float* ws_ml = nullptr;
+  if (sp.nsplit > 1) ws_ml = reinterpret_cast<float*>(ws_o + (size_t)B * sp.nsplit * ((H + th - 1) / th) * (DV * th / 2));
+  if (few_heads(H)) {
+    const int e = launch_few(Q, Qr, q_ld, qr_ld, KV, O, ws_o, ws_ml, B, H, T, scale * kLog2e, sp, s);
+    if (e) return e;
+  } else {
+    MX_RETURN_IF_HIP(lds_limit_once<mla_decode_kernel>(LDS_BYTES));
+    hipLaunchKernelGGL(mla_decode_kernel, dim3((unsigned)(B * HGB * sp.nsplit)), dim3(NT), LDS_BYTES, s,
+                       (const uint16_t*)Q, (const uint16_t*)Qr, (const uint16_t*)KV, (uint16_t*)O, ws_o, ws_ml, B, H, T,
+                       scale * kLog2e, sp.nsplit, sp.tps, q_ld, qr_ld);
+    MX_RETURN_IF_HIP(hipGetLastError());
+  }
   if (sp.nsplit > 1) {
-    const dim3 cg((unsigned)combine_grid(B, (int)HW, sp.nsplit));
-    switch (combine_sg(sp.nsplit)) {
-      case 1: hipLaunchKernelGGL(mla_combine_kernel<1>, cg, dim3(CmbCfg<1>::WG), 0, s, ws_o, ws_ml, (uint16_t*)O, H, sp.nsplit); break;
-      case 2: hipLaunchKernelGGL(mla_combine_kernel<2>, cg, dim3(CmbCfg<2>::WG), 0, s, ws_o, ws_ml, (uint16_t*)O, H, sp.nsplit); break;
-      case 4: hipLaunchKernelGGL(mla_combine_kernel<4>, cg, dim3(CmbCfg<4>::WG), 0, s, ws_o, ws_ml, (uint16_t*)O, H, sp.nsplit); break;
-      default: hipLaunchKernelGGL(mla_combine_kernel<8>, cg, dim3(CmbCfg<8>::WG), 0, s, ws_o, ws_ml, (uint16_t*)O, H, sp.nsplit); break;
-    }
+    const dim3 cg((unsigned)combine_grid(B, H, sp.nsplit));
+    with_combine(sp.nsplit, th, [&](auto sg, auto t) {
+      constexpr int SG = decltype(sg)::value, TH = decltype(t)::value;
+      hipLaunchKernelGGL((mla_combine_kernel<SG, TH>), cg, dim3(CmbCfg<SG, TH>::WG), 0, s, ws_o, ws_ml, (uint16_t*)O, H,
+                         sp.nsplit);
+      return 0;
+    });
     MX_RETURN_IF_HIP(hipGetLastError());
   }
   return MX_OK;

@@ -139,3 +139,47 @@ def test_absorbed_step_shapes(ops, b, h, t, dv):
     bs = list(range(min(b, 4)))
     ref = omla.mla_absorbed_ref(x["q_nope"][bs], x["q_rope"][bs], kv[bs], x["w_uk"], x["w_uv"], s.scale)
     assert normwise_rel_err(o.cpu()[bs], ref) <= 2e-2
+
+
+@pytest.mark.parametrize("bht", [(1, 16, 1), (1, 1, 15), (2, 16, 16), (3, 15, 17), (1, 16, 63), (2, 9, 65), (1, 16, 128),
+                                 (5, 16, 129), (1, 16, 1040), (48, 16, 801), (7, 16, 1300), (130, 16, 300),
+                                 (300, 16, 40)])
+def test_few_heads(ops, bht):
+    """Up to 16 heads run the kernel whose four waves take 16-token blocks in
+    turn: waves without a block, one block each, ragged last blocks, one slice
+    and slices with their merge (batches of 8 splits and remainders), more
+    workgroups than CUs.  The cache is followed by NaN, and scores grow along
+    T so that the running maximum moves in every slice.  Three roundings to
+    bf16 (probabilities, partial results, output) of at most 2^-9 each bound
+    the 2-norm of the error."""
+    B, H, T = bht
+    announce(f"mla few heads B{B} H{H} T{T}")
+    g = torch.Generator().manual_seed(B * 31 + H + T)
+    q = torch.randn((B, H, 576), generator=g).bfloat16()
+    kv = (torch.randn((B, T, 576), generator=g) * torch.linspace(0.5, 3.0, T)[None, :, None]).bfloat16()
+    buf = torch.full((B * T * 576 + 4096,), float("nan"), dtype=torch.bfloat16, device="cuda")
+    kvd = buf[:B * T * 576].view(B, T, 576)
+    kvd.copy_(kv)
+    scale = 192 ** -0.5
+    o = ops.mla_decode(q.cuda(), kvd, scale)
+    torch.cuda.synchronize()
+    kd = kv.double()
+    p = torch.softmax(q.double() @ kd.transpose(1, 2).contiguous() * scale, dim=-1)
+    ref = p @ kd[:, :, :512].contiguous()
+    assert ((o.cpu().double() - ref).norm() / ref.norm()).item() <= 3 * 2.0 ** -9
+    norm = lambda x: x.norm(dim=-1)
+    assert (norm(o.cpu().double() - ref) <= 6 * 2.0 ** -9 * norm(ref)).all()
+
+
+@pytest.mark.parametrize("bht", [(48, 128, 700), (20, 100, 900), (3, 40, 2100)])
+def test_one_round_of_splits(ops, bht):
+    """Split counts that are no power of two: their merge ends in a partial
+    batch of loads."""
+    B, H, T = bht
+    announce(f"mla splits B{B} H{H} T{T}")
+    s = shapes.MLADecodeShape("t", B, H, T)
+    q, kv = inputs.mla_inputs(s)
+    assert ops.mla_decode_splits(B, H, T) * B <= 256
+    o = ops.mla_decode(q.cuda(), kv.cuda(), s.scale)
+    torch.cuda.synchronize()
+    assert normwise_rel_err(o.cpu(), omla.mla_decode_ref(q, kv, s.scale)) <= TOL
