@@ -32,10 +32,11 @@
 //    units, is folded into Q once in the prologue, so the score MFMAs return
 //    log2-domain scores and each score costs one exp2; the row sum is
 //    accumulated with v_dot2 on the rounded P the PV MFMA consumes.
-//  * Causal: each workgroup takes a heavy and a light query block (block p
-//    and its mirror nqb-1-p), so all workgroups carry the same number of
-//    key tiles and finish together; only diagonal / ragged tiles are
-//    masked; tiles entirely above a wave's diagonal are skipped.
+//  * Causal: long query blocks first; only diagonal / ragged tiles are masked;
+//    tiles entirely above a wave's diagonal are skipped.
+//  * Short problems: a workgroup of 8 waves can split the keys between 2 or 4
+//    groups of waves, each with its own ring, that meet in LDS at the end
+//    (KSP, pick_split below).
 #include <type_traits>
 
 #include "mx_common.h"
@@ -99,41 +100,56 @@ struct Ring {
   static constexpr int NS = QT == 1 ? 2 : 3;  // stages (QT=1 keeps two waves per SIMD)
 };
 
+// LDS of a workgroup: the key groups' rings, and at the end the area where
+// their states meet.
+template <int DQK, int DV, int QT, int NWAVES, int KSP>
+constexpr int lds_bytes() {
+  const int rings = KSP * Ring<QT>::NS * Lds<DQK, DV, NWAVES / KSP>::STAGE;
+  const int merge = KSP > 1 ? NWAVES * (DV / 8 * 1024 + 256) : 0;
+  return rings > merge ? rings : merge;
+}
+
 // Waves of a workgroup for the default kernel of a head-dim pair (QT = 1).
 template <int DQK, int DV>
 constexpr int default_waves() {
   return waves_for<DQK, DV>();
 }
 
-template <int DQK, int DV, typename T, bool CAUSAL, int QT, int NWAVES>
+template <int DQK, int DV, typename T, bool CAUSAL, int QT, int NWAVES, int KSP>
 __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(const uint16_t* __restrict__ Q,
                                                                      const uint16_t* __restrict__ K,
                                                                      const uint16_t* __restrict__ V,
                                                                      uint16_t* __restrict__ O, int B, int Hq,
-                                                                     int Hkv, int S, float sl2, int hpw) {
+                                                                     int Hkv, int S, float sl2, int hpw, int pairs) {
   constexpr int QW = 32 * QT;         // queries per wave
   constexpr int DC = DQK / 16;        // 16-deep k steps of QK^T
   constexpr int DT = DV / 32;         // 32-row d tiles of O^T
   constexpr int NS = Ring<QT>::NS;
-  using L = Lds<DQK, DV, NWAVES>;
+  constexpr int QS = NWAVES / KSP;    // waves of a key group
+  static_assert(KSP == 1 || (QT == 1 && NS == 2), "key groups");
+  using L = Lds<DQK, DV, QS>;
   extern __shared__ __align__(1024) unsigned char smem[];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // wave of its key group, and the key group: group k takes the key tiles k,
+  // k + KSP, .. of the same query rows through a ring of its own
+  const int wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) % QS);
+  const int kgp = KSP > 1 ? __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) / QS) : 0;
   const int g = lane >> 5;      // lane half
   const int ql = lane & 31;     // query within a 32-query tile
 
   // ---- workgroup -> (qblock, b, kv head, head group) ----
   const int G = Hq / Hkv;
-  const int qsb = NWAVES / hpw;            // query sub-blocks per workgroup
+  const int qsb = QS / hpw;                // query sub-blocks per workgroup
   const int QB = QW * qsb;                 // query rows per workgroup
   const int hgroups = G / hpw;
   const int nqb = (S + QB - 1) / QB;
   const int per_q = B * Hkv * hgroups;
-  // Causal: workgroup p takes query block nqb-1-p, then its mirror p, so
+  // Causal: workgroup p takes query block nqb-1-p (the long ones first, so the
+  // short ones fill in at the end) and, with pairs, then its mirror p, so that
   // every workgroup carries about the same number of key tiles.
   const int p = (int)(blockIdx.x / per_q);
-  const int nrep = (CAUSAL && nqb - 1 - p != p) ? 2 : 1;
+  const int nrep = (CAUSAL && pairs && nqb - 1 - p != p) ? 2 : 1;
   int rest = blockIdx.x % per_q;
   const int hg = rest % hgroups;
   rest /= hgroups;
@@ -173,6 +189,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
   // ---- kv range ----
   const int kv_end_wg = CAUSAL ? min(S, q0wg + QB) : S;
   const int nblk = (kv_end_wg + BN - 1) / BN;
+  const int nstep = (nblk + KSP - 1) / KSP;  // loop trips: one key tile of each group
   const int kv_end_w = CAUSAL ? min(S, q0w + QW) : S;
 
   // ---- HBM -> LDS with direct loads: wave load ld of a stage fills stage
@@ -180,7 +197,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
   // 16i of it, i.e. row r = byte / ROW, chunk c = (byte % ROW) / 16, stored
   // at chunk position c ^ k/vswz(r).  Rows past S re-read row S-1 (finite
   // data that the mask or a zero P cancels). ----
-  const uint32_t lds0 = lds_addr(smem);
+  const uint32_t lds0 = lds_addr(smem) + kgp * NS * L::STAGE;
   auto ld_row = [&](int ld) {
     const bool vt = ld >= L::NLK;
     return (1024 * (vt ? ld - L::NLK : ld) + 16 * lane) / (vt ? L::ROWV : L::ROWK);
@@ -199,18 +216,19 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
     const int ld = wave * L::LPW + n;
     ld_off[n] = (uint32_t)ld_row(ld) * (ld >= L::NLK ? L::ROWV : L::ROWK) + ld_chunk(ld);
   }
-  // load n of tile blk, rows past S-1 clamped to S-1 (no branch: it can sit
-  // between the MFMAs of a k step)
-  auto issue_part = [&](int blk, int n) {
+  // load n of this group's tile of step st, rows past S-1 clamped to S-1 (no
+  // branch: it can sit between the MFMAs of a k step)
+  auto issue_part = [&](int step, int n) {
+    const int blk = step * KSP + kgp;
     const int ld = wave * L::LPW + n;
     const bool vt = ld >= L::NLK;
     const int kv = min(blk * BN + ld_row(ld), S - 1);
     dma16(vt ? Vh : Kh, (uint32_t)kv * (vt ? L::ROWV : L::ROWK) + ld_chunk(ld),
-          lds0 + (blk % NS) * L::STAGE + ld * 1024);
+          lds0 + (step % NS) * L::STAGE + ld * 1024);
   };
-  auto issue = [&](int blk) {
-    const int kv0 = blk * BN;
-    const uint32_t st = lds0 + (blk % NS) * L::STAGE;
+  auto issue = [&](int step) {
+    const int kv0 = (step * KSP + kgp) * BN;
+    const uint32_t st = lds0 + (step % NS) * L::STAGE;
     if (kv0 + BN <= S) {
 #pragma unroll
       for (int n = 0; n < L::LPW; ++n) {
@@ -230,7 +248,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
   };
   if (rep > 0) __syncthreads();  // every wave is done with the previous block's ring
   land_args(O);  // O is used only after the tile loop
-  issue(0);
+  if (KSP == 1 || kgp < nblk) issue(0);
   wait_vmcnt<0>();  // the Q loads and stage 0 complete together
 #pragma unroll
   for (int p = 1; p < NS - 1; ++p)
@@ -266,9 +284,10 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
     neg_m[qt] = f32x16{};
   }
 
-  // One key tile; STG = blk % NS is a compile-time constant so every LDS
-  // fragment address is a lane offset plus an immediate.
-  auto tile = [&](int blk, auto stg_tag) {
+  // One step (a key tile of each group); STG = step % NS is a compile-time
+  // constant so every LDS fragment address is a lane offset plus an immediate.
+  auto tile = [&](int step, auto stg_tag) {
+    const int blk = step * KSP + kgp;
     constexpr int STG = decltype(stg_tag)::value;
     // stage blk landed (this wave's loads), then visible to all waves;
     // the stage read in iteration blk-1 is free for stage blk+NS-1.
@@ -284,10 +303,10 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
     // the next tile's loads go out one per k step of the S^T MFMAs below
     // rather than all at once, which queues every wave's loads behind the
     // barrier
-    const bool load_next = blk + NS - 1 < nblk;
+    const bool load_next = blk + KSP * (NS - 1) < nblk;
     const int kv0 = blk * BN;
     // a wave that skips this tile still issues its share of the next one
-    if (kv0 >= kv_end_w && load_next) issue(blk + NS - 1);
+    if (kv0 >= kv_end_w && load_next) issue(step + NS - 1);
 
     if (kv0 < kv_end_w) {
       constexpr uint32_t st = STG * L::STAGE;
@@ -334,7 +353,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
             s[qt][t] = mfma32<T>(kb[dc % (KLA + 1)][t], qf[qt][dc], dc == 0 ? start_m(qt) : s[qt][t]);
 #pragma unroll
         for (int n = 0; n < L::LPW; ++n)
-          if (dc == n * DC / L::LPW && load_next) issue_part(blk + NS - 1, n);
+          if (dc == n * DC / L::LPW && load_next) issue_part(step + NS - 1, n);
         __builtin_amdgcn_sched_barrier(0);  // keep the read lookahead
       }
 
@@ -376,10 +395,12 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[qt][t][e]);
         mx = max_xor32(mx);
-        const bool first = blk == 0;  // every wave processes tile 0
+        const bool first = step == 0;  // every wave with a tile has one at step 0
         if (first || __any(mx > kLazy)) {
-          // first tile: the max itself; later: only upward moves
-          const float shift = first ? mx : fmaxf(mx, 0.f);
+          // first tile: the max itself; later: only upward moves.  A row that
+          // sees no key of its group's first tile sees none of the later ones
+          // either: its max stays 0, its sums 0.
+          const float shift = !first ? fmaxf(mx, 0.f) : KSP > 1 && mx == -INFINITY ? 0.f : mx;
           const float corr = __builtin_amdgcn_exp2f(-shift);
           m_run[qt] += shift;
           l_run[qt] *= corr;
@@ -466,11 +487,55 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
       __builtin_amdgcn_s_setprio(0);
     }
   };
-  for (int blk = 0; blk < nblk; blk += NS) {
-    tile(blk, std::integral_constant<int, 0>{});
-    if (blk + 1 < nblk) tile(blk + 1, std::integral_constant<int, 1>{});
+  for (int step = 0; step < nstep; step += NS) {
+    tile(step, std::integral_constant<int, 0>{});
+    if (step + 1 < nstep) tile(step + 1, std::integral_constant<int, 1>{});
     if constexpr (NS == 3)
-      if (blk + 2 < nblk) tile(blk + 2, std::integral_constant<int, 2>{});
+      if (step + 2 < nstep) tile(step + 2, std::integral_constant<int, 2>{});
+  }
+
+  // ---- the key groups' states of the same queries meet in LDS by the
+  // log-sum-exp rule: O^T as [wave][4 dt + i][lane] x 16 B, then (m, l) as
+  // [wave][32]; each of the KSP waves of a query tile sums and stores 1 / KSP
+  // of the column quads. ----
+  if constexpr (KSP > 1) {
+    constexpr int NQ = 4 * DT, QPW = NQ / KSP;
+    static_assert(NQ % KSP == 0 && NWAVES * (NQ * 1024 + 256) <= lds_bytes<DQK, DV, QT, NWAVES, KSP>(), "merge area");
+    f32x4* red = reinterpret_cast<f32x4*>(smem);
+    float2* ml = reinterpret_cast<float2*>(smem + NWAVES * NQ * 1024);
+    const int wv = kgp * QS + wave;
+    const float l_tot = sum_xor32(l_run[0]);
+    __syncthreads();  // every wave is done with the rings
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x16& a = acc_o[0][dt];
+        red[(wv * NQ + 4 * dt + i) * 64 + lane] = f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
+      }
+    if (g == 0) ml[wv * 32 + ql] = float2{l_tot > 0.f ? m_run[0] : -INFINITY, l_tot};
+    __syncthreads();
+    float mx = -INFINITY, w[KSP], l = 0.f;
+#pragma unroll
+    for (int k = 0; k < KSP; ++k) mx = fmaxf(mx, ml[(k * QS + wave) * 32 + ql].x);
+#pragma unroll
+    for (int k = 0; k < KSP; ++k) {
+      const float2 x = ml[(k * QS + wave) * 32 + ql];
+      w[k] = x.y > 0.f ? __builtin_amdgcn_exp2f(x.x - mx) : 0.f;
+      l += w[k] * x.y;
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    uint16_t* orow = O + (q_head + qrow[0]) * DV;
+#pragma unroll
+    for (int u = 0; u < QPW; ++u) {
+      const int qd = kgp * QPW + u;  // column quad: d = 8 qd + 4 g + {0..3}
+      f32x4 o{};
+#pragma unroll
+      for (int k = 0; k < KSP; ++k) o += w[k] * red[((k * QS + wave) * NQ + qd) * 64 + lane];
+      if (qrow[0] < S)
+        st64(orow + 8 * qd + 4 * g, u32x2{T::pack2(o[0] * inv, o[1] * inv), T::pack2(o[2] * inv, o[3] * inv)});
+    }
+    continue;  // the next query block starts with a barrier
   }
 
   // ---- normalise and store: lane holds query qrow, d = 32dt + 8i + 4g + j ----
@@ -500,19 +565,20 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 }  // q-block loop
 }
 
-template <int DQK, int DV, typename T, bool CAUSAL, int QT, int NWAVES>
+template <int DQK, int DV, typename T, bool CAUSAL, int QT, int NWAVES, int KSP = 1>
 static int launch(const void* Q, const void* K, const void* V, void* O, int B, int Hq, int Hkv, int S, float scale,
-                  int hpw, hipStream_t stream) {
+                  int hpw, bool pairs, hipStream_t stream) {
   const int G = Hq / Hkv;
-  const int QB = 32 * QT * (NWAVES / hpw);
+  const int QB = 32 * QT * (NWAVES / KSP / hpw);
   const int nqb = (S + QB - 1) / QB;
-  const long long grid = (long long)(CAUSAL ? (nqb + 1) / 2 : nqb) * B * Hkv * (G / hpw);
+  const long long grid = (long long)(CAUSAL && pairs ? (nqb + 1) / 2 : nqb) * B * Hkv * (G / hpw);
   if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
-  constexpr auto kern = gqa_fwd_kernel<DQK, DV, T, CAUSAL, QT, NWAVES>;
-  constexpr int lds = Ring<QT>::NS * Lds<DQK, DV, NWAVES>::STAGE;
+  constexpr auto kern = gqa_fwd_kernel<DQK, DV, T, CAUSAL, QT, NWAVES, KSP>;
+  constexpr int lds = lds_bytes<DQK, DV, QT, NWAVES, KSP>();
+  static_assert(lds <= 160 * 1024, "LDS");
   MX_RETURN_IF_HIP(lds_limit_once<kern>(lds));
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NWAVES), lds, stream, (const uint16_t*)Q, (const uint16_t*)K,
-                     (const uint16_t*)V, (uint16_t*)O, B, Hq, Hkv, S, scale * kLog2e, hpw);
+                     (const uint16_t*)V, (uint16_t*)O, B, Hq, Hkv, S, scale * kLog2e, hpw, (int)pairs);
   MX_RETURN_IF_HIP(hipGetLastError());
   return MX_OK;
 }
@@ -554,9 +620,9 @@ inline int tile_for(int G, int D, int block_m, int block_n, int wave_m, Tile* t)
 template <int D, typename T, bool CAUSAL>
 static int launch_tile(const void* Q, const void* K, const void* V, void* O, int B, int Hq, int Hkv, int S,
                        float scale, const Tile& t, hipStream_t s) {
-  if (t.qt == 2) return launch<D, D, T, CAUSAL, 2, 4>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, s);
-  if (t.nwaves == 4) return launch<D, D, T, CAUSAL, 1, 4>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, s);
-  return launch<D, D, T, CAUSAL, 1, 8>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, s);
+  if (t.qt == 2) return launch<D, D, T, CAUSAL, 2, 4>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, true, s);
+  if (t.nwaves == 4) return launch<D, D, T, CAUSAL, 1, 4>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, true, s);
+  return launch<D, D, T, CAUSAL, 1, 8>(Q, K, V, O, B, Hq, Hkv, S, scale, t.hpw, true, s);
 }
 
 template <typename T>
@@ -569,13 +635,83 @@ static int dispatch_tile(const void* Q, const void* K, const void* V, void* O, i
                 : launch_tile<64, T, false>(Q, K, V, O, B, Hq, Hkv, S, scale, t, s);
 }
 
+// How the default launch splits a problem: ksp key groups per workgroup, hpw
+// heads, and whether causal workgroups take a long and a short query block.
+//  * More key groups make the workgroups smaller (256 / ksp query rows) and
+//    their serial chain of key tiles shorter, for a dearer step: worth it while
+//    the launch is as long as its longest workgroup.  At head dim 64, B2 Hq16
+//    S1001 non-causal takes 21.6 us with one group, 15.7 with two, 20.2 with
+//    four, and causal B1 Hq8 S1092 21.1, 14.5 and 11.4; at 128, causal B1 Hq16
+//    S1335 36.1 and 25.0, but S4096 with 32 heads 126 and 142.  Four groups at
+//    128 do not fit the LDS; two at the 192-wide query of MLA spill registers
+//    and measured slower.
+//  * Pairs make equal workgroups, which is best where they fill whole rounds of
+//    the CUs (S4096, 32 heads: 126 us against 127.6 singly), and leave CUs idle
+//    elsewhere (MLA prefill, 64 heads, S2199: 128 against 116; D 128, 64 heads
+//    in all, S647: 32.6 against 22.1).
+// The estimate, in units of a step with one group: a workgroup costs its steps
+// plus a start and end per query block, 256 run at once; single causal
+// workgroups, of all lengths, fill the CUs evenly after the first round.
+// Fitted to 70 random shapes timed with every ksp (graph replay, B 1..4, 8..32
+// heads, S 128..4200): the choice is on average 0.7% slower than the best.
+struct Split {
+  int ksp, hpw;
+  bool pairs;
+};
+template <int DQK, int DV>
+static Split pick_split(int B, int Hq, int Hkv, int S, int causal) {
+  struct Cost {
+    int ksp;
+    double step, ends, fixed;
+  };
+  static constexpr Cost k64[] = {{1, 1.0, 4.0, 0.0}, {2, 1.08, 4.5, 1.0}, {4, 1.3, 3.5, 1.0}};
+  static constexpr Cost k128[] = {{1, 1.4, 4.0, 0.0}, {2, 1.6, 4.0, 0.5}};
+  const Cost* cost = DQK == 64 ? k64 : k128;
+  const int choices = DQK != DV ? 1 : DQK == 64 ? 3 : 2;
+  const int G = Hq / Hkv;
+  Split best{1, default_hpw(G), true};
+  double least = 0;
+  for (int c = 0; c < choices; ++c) {
+    const int ksp = cost[c].ksp;
+    const int rows = 32 * (choices == 1 ? default_waves<DQK, DV>() : 8) / ksp;  // query rows over all heads
+    const int hpw = default_hpw(G) > rows / 32 ? rows / 32 : default_hpw(G);
+    const long long QB = rows / hpw, nqb = (S + QB - 1) / QB, per = (long long)B * Hkv * (G / hpw);
+    auto steps = [&](long long keys) { return (double)(((keys + BN - 1) / BN + ksp - 1) / ksp) + cost[c].ends; };
+    const double longest = steps(S), shortest = steps(causal && nqb > 1 ? QB : S);
+    auto consider = [&](double m, bool pairs) {
+      const double t = cost[c].fixed + cost[c].step * m;
+      if ((c == 0 && pairs) || t < least) {
+        least = t;
+        best = Split{ksp, hpw, pairs};
+      }
+    };
+    if (causal) {
+      const double total = 0.5 * (longest + shortest) * (double)(nqb * per) / 256;
+      consider((double)(((nqb + 1) / 2 * per + 255) / 256) * (nqb > 1 ? longest + shortest : longest), true);
+      consider(total > longest ? total : longest, false);
+    } else {
+      consider((double)((nqb * per + 255) / 256) * longest, true);
+    }
+  }
+  return best;
+}
+
 template <int DQK, int DV, typename T>
 static int launch_default(const void* Q, const void* K, const void* V, void* O, int B, int Hq, int Hkv, int S,
                           float scale, int causal, hipStream_t s) {
-  constexpr int NW = default_waves<DQK, DV>();
-  const int hpw = default_hpw(Hq / Hkv);
-  return causal ? launch<DQK, DV, T, true, 1, NW>(Q, K, V, O, B, Hq, Hkv, S, scale, hpw, s)
-                : launch<DQK, DV, T, false, 1, NW>(Q, K, V, O, B, Hq, Hkv, S, scale, hpw, s);
+  const Split sp = pick_split<DQK, DV>(B, Hq, Hkv, S, causal);
+  auto go = [&](auto c, auto ksp) {
+    constexpr int KSP = decltype(ksp)::value, NW = KSP > 1 ? 8 : default_waves<DQK, DV>();
+    return launch<DQK, DV, T, decltype(c)::value, 1, NW, KSP>(Q, K, V, O, B, Hq, Hkv, S, scale, sp.hpw, sp.pairs, s);
+  };
+  auto by_ksp = [&](auto c) {
+    if constexpr (DQK == 64)
+      if (sp.ksp == 4) return go(c, std::integral_constant<int, 4>{});
+    if constexpr (DQK == DV)
+      if (sp.ksp == 2) return go(c, std::integral_constant<int, 2>{});
+    return go(c, std::integral_constant<int, 1>{});
+  };
+  return causal ? by_ksp(std::true_type{}) : by_ksp(std::false_type{});
 }
 
 // (qk head dim, v head dim) pairs with a kernel: the GQA head dims 64 and
@@ -642,9 +778,9 @@ namespace mx {
 namespace gqa {
 template <int D, typename T, bool C>
 static const void* tile_kernel(const Tile& t) {
-  if (t.qt == 2) return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 2, 4>);
-  if (t.nwaves == 4) return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 1, 4>);
-  return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 1, 8>);
+  if (t.qt == 2) return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 2, 4, 1>);
+  if (t.nwaves == 4) return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 1, 4, 1>);
+  return reinterpret_cast<const void*>(gqa_fwd_kernel<D, D, T, C, 1, 8, 1>);
 }
 template <int D, typename T>
 static const void* tile_kernel_c(const Tile& t, int causal) {

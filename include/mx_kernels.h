@@ -142,7 +142,9 @@ int mx_gqa_fwd(const void* Q, const void* K, const void* V, void* O, int B, int 
  * MFMAs).  A tile no kernel has returns MX_ERR_UNSUPPORTED before anything
  * is enqueued.  Any S is
  * accepted (ragged query and key tiles are masked).  mx_gqa_fwd runs
- * block_m = mx_gqa_fwd_default_block_m(Hq, Hkv, D), block_n 64, wave_m 32.
+ * block_m = mx_gqa_fwd_default_block_m(Hq, Hkv, D), block_n 64, wave_m 32
+ * where that fills the GPU; shorter problems run workgroups of fewer query
+ * rows whose waves split the keys.
  * Replaces: cutile-attn-gqa/main.py:202-230 (pick_blocks with the
  * --block-m / --block-n overrides, each pair compiled by make_gqa_kernel,
  * :64-66) and the launch at :249-252.

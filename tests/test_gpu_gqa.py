@@ -167,3 +167,47 @@ def test_tile_rejections_enqueue_nothing(ops):
             ops.gqa_fwd(q, k, v, causal=True, out=out, block_m=bm, block_n=bn, wave_m=wm)
     torch.cuda.synchronize()
     assert torch.isnan(out.float()).all()
+
+
+# Sizes at which the default launch splits the keys between 2 or 4 groups of waves: fewer key tiles than
+# groups (S <= 64), last tiles of 1 and 63 keys, query rows whose group's first tile is masked, one head and
+# several per workgroup, and the sizes around which the choice of one group takes over.
+KEY_GROUPS = [(1, 1, 8, 8, 64), (1, 63, 8, 2, 64), (1, 65, 8, 1, 64), (2, 129, 8, 8, 128), (1, 191, 16, 4, 64),
+              (1, 257, 8, 4, 64), (1, 320, 8, 1, 128), (2, 447, 8, 8, 64), (1, 1000, 8, 2, 64), (1, 1025, 8, 4, 128),
+              (2, 1001, 16, 4, 64), (1, 577, 32, 8, 128), (4, 640, 16, 16, 64)]
+
+
+@pytest.mark.parametrize("causal", [True, False], ids=["c", "n"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["b", "h"])
+@pytest.mark.parametrize("case", KEY_GROUPS, ids=lambda c: f"B{c[0]}S{c[1]}H{c[2]}/{c[3]}D{c[4]}")
+def test_key_groups(ops, case, dt, causal):
+    """Every output row against 64-bit attention.  Roundings on the way, each at
+    most u = 2^-9 (bf16) or 2^-12 (f16): Q with the scale folded in (moves a
+    score by u |s|, so a weight by about u log2-range; scores here stay below
+    12), the probabilities, the output; the bound allows 12 u per row's norm of
+    the values it mixes.  Scores drift along the keys so that the groups'
+    maxima differ, and K and V are followed by NaN in memory."""
+    B, S, Hq, Hkv, D = case
+    announce(f"gqa key groups B{B} S{S} Hq{Hq} Hkv{Hkv} D{D} causal={causal} {dt}")
+    g = torch.Generator().manual_seed(S * 7 + Hq + D)
+    q = torch.randn((B, Hq, S, D), generator=g).to(dt)
+    k = (torch.randn((B, Hkv, S, D), generator=g) * torch.linspace(1.0, 2.0, S)[:, None]).to(dt)
+    v = torch.randn((B, Hkv, S, D), generator=g).to(dt)
+
+    def padded(t):
+        buf = torch.full((t.numel() + 8192,), float("nan"), dtype=dt, device="cuda")
+        buf[:t.numel()].view(t.shape).copy_(t)
+        return buf[:t.numel()].view(t.shape)
+
+    o = ops.gqa_fwd(padded(q), padded(k), padded(v), causal=causal)
+    torch.cuda.synchronize()
+    kd, vd = (t.double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+    s = q.double() @ kd.transpose(-1, -2).contiguous() / D ** 0.5
+    if causal:
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool).triu(1), float("-inf"))
+    p = torch.softmax(s, dim=-1)
+    ref = p @ vd
+    u = 2.0 ** -9 if dt == torch.bfloat16 else 2.0 ** -12
+    err = (o.cpu().double() - ref).norm(dim=-1)
+    mixed = torch.sqrt((p ** 2) @ (vd.norm(dim=-1, keepdim=True) ** 2)).squeeze(-1) + ref.norm(dim=-1)
+    assert (err <= 12 * u * mixed).all(), (err / (u * mixed)).max()
