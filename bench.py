@@ -394,7 +394,7 @@ def case_gqa(c: Ctx) -> dict:
         "value": c.F.tflops(flops, ms),
         "tflops_reference_convention": c.F.tflops(c.F.gqa_attention_flops(shape), ms),
         "roofline": roofline("mfma", flops, ms, c.F.PEAK_BF16_TFLOPS, "TFLOP/s", wl,
-                             "gqa_fwd_kernel<128, 128, BF16, true, 1, 8>"),
+                             "gqa_fwd_kernel<128, 128, BF16, true, 1, 8, 1>"),
         "shape": shape,
     }
     if c.cpu:
@@ -799,7 +799,7 @@ def case_mla_prefill(c: Ctx) -> dict:
     rec = {"workload": wl, "unit": "TFLOPS", "mean_ms": ms, "wall_ms": wall,
            "value": c.F.tflops(fl, ms), "frac_mfma_peak": c.F.tflops(fl, ms) / c.F.PEAK_BF16_TFLOPS,
            "roofline": roofline("mfma", fl, ms, c.F.PEAK_BF16_TFLOPS, "TFLOP/s", wl,
-                                "gqa_fwd_kernel<192, 128, BF16, false, 1, 8>")}
+                                "gqa_fwd_kernel<192, 128, BF16, false, 1, 8, 1>")}
     if c.cpu:
         from oracle import mla as omla
 

@@ -165,16 +165,16 @@ GQA_PARTS = {
     # precomputed lane offsets (no row clamp, no address VALU, no branch);
     # the loop then waits for those loads before the ring is reused.
     "branch_free_loads": [
-        ("  auto issue = [&](int blk) {\n    const int kv0 = blk * BN;",
+        ("  auto issue = [&](int step) {\n    const int kv0 = (step * KSP + kgp) * BN;",
          "  auto issue_full = [&](int src, int slot, int n) {\n    const int ld = wave * L::LPW + n;\n"
          "    const bool vt = ld >= L::NLK;\n    const int kv0 = src * BN;\n"
          "    dma16((vt ? Vh + (size_t)kv0 * L::ROWV : Kh + (size_t)kv0 * L::ROWK), ld_off[n],\n"
          "          lds0 + slot * L::STAGE + ld * 1024);\n  };\n"
-         "  auto issue = [&](int blk) {\n    const int kv0 = blk * BN;"),
-        ("          if (dc == n * DC / L::LPW && load_next) issue_part(blk + NS - 1, n);",
-         "          if (dc == n * DC / L::LPW) issue_full(load_next ? blk + NS - 1 : nblk - 1, (blk + NS - 1) % NS, n);"),
-        ("      if (blk + 2 < nblk) tile(blk + 2, std::integral_constant<int, 2>{});\n  }\n",
-         "      if (blk + 2 < nblk) tile(blk + 2, std::integral_constant<int, 2>{});\n  }\n  wait_vmcnt<0>();\n"),
+         "  auto issue = [&](int step) {\n    const int kv0 = (step * KSP + kgp) * BN;"),
+        ("          if (dc == n * DC / L::LPW && load_next) issue_part(step + NS - 1, n);",
+         "          if (dc == n * DC / L::LPW)\n            issue_full(load_next ? (step + NS - 1) * KSP + kgp : nblk - 1, (step + NS - 1) % NS, n);"),
+        ("      if (step + 2 < nstep) tile(step + 2, std::integral_constant<int, 2>{});\n  }\n",
+         "      if (step + 2 < nstep) tile(step + 2, std::integral_constant<int, 2>{});\n  }\n  wait_vmcnt<0>();\n"),
     ],
     # K fragments read three k-steps ahead instead of two.
     "k_lookahead_3": [
