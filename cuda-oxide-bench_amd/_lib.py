@@ -111,6 +111,14 @@ def check(fn: str, code: int) -> None:
         raise MXError(fn, code, strerror(code))
 
 
+_FUNCTIONS: dict = {}  # entry points by name, once looked up
+
+
 def call(fn: str, *args) -> None:
     """Call a status-returning entry point and raise MXError on failure."""
-    check(fn, getattr(load(), fn)(*args))
+    f = _FUNCTIONS.get(fn)
+    if f is None:
+        f = _FUNCTIONS[fn] = getattr(load(), fn)
+    code = f(*args)
+    if code:
+        check(fn, code)

@@ -18,11 +18,22 @@ from . import _lib
 _IO_DTYPES = {torch.bfloat16: _lib.MX_DTYPE_BF16, torch.float16: _lib.MX_DTYPE_F16}
 
 
+_Tensor = torch.Tensor
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_current_device = torch._C._cuda_getDevice
+
+
+# The checks below run on every call, several per call, and most launches take
+# a few microseconds: their common path is one expression each, and the stream
+# handle comes without building a torch.cuda.Stream (2.8 us).
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def _require(t: torch.Tensor, name: str, dtypes, ndim: int | None = None) -> None:
+    if (type(t) is _Tensor and t.dtype in dtypes and t.is_cuda and (ndim is None or t.dim() == ndim)
+            and t.is_contiguous()):
+        return
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
     if t.dtype not in dtypes:
@@ -35,10 +46,12 @@ def _require(t: torch.Tensor, name: str, dtypes, ndim: int | None = None) -> Non
         raise ValueError(f"{name} must be contiguous")
 
 
-def _same_device(*ts: torch.Tensor) -> None:
-    devs = {t.device for t in ts}
-    if len(devs) != 1:
-        raise ValueError(f"all tensors must be on one device (got {sorted(map(str, devs))})")
+def _same_device(first: torch.Tensor, *others: torch.Tensor) -> None:
+    d = first.get_device()
+    for t in others:
+        if t.get_device() != d:
+            devs = {t.device for t in (first, *others)}
+            raise ValueError(f"all tensors must be on one device (got {sorted(map(str, devs))})")
 
 
 def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -54,9 +67,10 @@ def gemm_bf16(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None)
         raise ValueError(f"inner dimensions differ: a {tuple(a.shape)} vs b {tuple(b.shape)}")
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    _require(out, "out", (torch.bfloat16,), 2)
-    if tuple(out.shape) != (M, N):
-        raise ValueError(f"out must be {(M, N)}, got {tuple(out.shape)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 2)
+        if out.shape != (M, N):
+            raise ValueError(f"out must be {(M, N)}, got {tuple(out.shape)}")
     _same_device(a, b, out)
     _lib.call("mx_gemm_bf16", a.data_ptr(), b.data_ptr(), out.data_ptr(), M, N, K, K, N, N, _stream())
     return out
@@ -81,15 +95,16 @@ def gemm_fp8_bs(a: torch.Tensor, sa: torch.Tensor, b: torch.Tensor, sb: torch.Te
         raise ValueError(f"inner dimensions differ: a {tuple(a.shape)} vs b {tuple(b.shape)}")
     if K % 128:
         raise ValueError(f"K={K} must be a multiple of 128 (scale block depth)")
-    if tuple(sa.shape) != (M, K // 128):
+    if sa.shape != (M, K // 128):
         raise ValueError(f"sa must be {(M, K // 128)}, got {tuple(sa.shape)}")
-    if tuple(sb.shape) != (K // 128, (N + 127) // 128):
+    if sb.shape != (K // 128, (N + 127) // 128):
         raise ValueError(f"sb must be {(K // 128, (N + 127) // 128)}, got {tuple(sb.shape)}")
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=a.device)
-    _require(out, "out", (torch.bfloat16,), 2)
-    if tuple(out.shape) != (M, N):
-        raise ValueError(f"out must be {(M, N)}, got {tuple(out.shape)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 2)
+        if out.shape != (M, N):
+            raise ValueError(f"out must be {(M, N)}, got {tuple(out.shape)}")
     _same_device(a, sa, b, sb, out)
     _lib.call("mx_gemm_fp8_bs", a.data_ptr(), sa.data_ptr(), b.data_ptr(), sb.data_ptr(), out.data_ptr(),
               M, N, K, _stream())
@@ -112,7 +127,7 @@ def gqa_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
     _require(v, "v", (q.dtype,), 4)
     B, Hq, S, D = q.shape
     Bk, Hkv, Sk, Dk = k.shape
-    if (Bk, Sk, Dk) != (B, S, D) or tuple(v.shape) != tuple(k.shape):
+    if (Bk, Sk, Dk) != (B, S, D) or v.shape != tuple(k.shape):
         raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     if Hq % Hkv:
         raise ValueError(f"n_q ({Hq}) must be divisible by n_kv ({Hkv})")
@@ -120,9 +135,10 @@ def gqa_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool = Fa
         scale = 1.0 / math.sqrt(D)
     if out is None:
         out = torch.empty_like(q)
-    _require(out, "out", (q.dtype,), 4)
-    if out.shape != q.shape:
-        raise ValueError(f"out must be {tuple(q.shape)}")
+    else:
+        _require(out, "out", (q.dtype,), 4)
+        if out.shape != q.shape:
+            raise ValueError(f"out must be {tuple(q.shape)}")
     _same_device(q, k, v, out)
     if block_m is None and block_n is None and wave_m is None:
         _lib.call("mx_gqa_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, Hq, Hkv, S, D,
@@ -183,16 +199,17 @@ def mla_prefill_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
     if not (q.dtype == k.dtype == v.dtype):
         raise ValueError("q, k, v must share a dtype")
     B, H, S, Dqk = q.shape
-    if tuple(k.shape) != (B, H, S, Dqk) or tuple(v.shape[:3]) != (B, H, S):
+    if k.shape != (B, H, S, Dqk) or v.shape[:3] != (B, H, S):
         raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     Dv = v.shape[3]
     if scale is None:
         scale = 1.0 / math.sqrt(Dqk)
     if out is None:
         out = torch.empty((B, H, S, Dv), dtype=q.dtype, device=q.device)
-    _require(out, "out", (q.dtype,), 4)
-    if tuple(out.shape) != (B, H, S, Dv):
-        raise ValueError(f"out must be {(B, H, S, Dv)}")
+    else:
+        _require(out, "out", (q.dtype,), 4)
+        if out.shape != (B, H, S, Dv):
+            raise ValueError(f"out must be {(B, H, S, Dv)}")
     _same_device(q, k, v, out)
     _lib.call("mx_mla_prefill_fwd", q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, S, Dqk, Dv,
               float(scale), int(bool(causal)), _IO_DTYPES[q.dtype], _stream())
@@ -214,9 +231,10 @@ def mla_decode(q: torch.Tensor, kv: torch.Tensor, scale: float, d_latent: int = 
     d_rope = Dq - d_latent
     if out is None:
         out = torch.empty((B, H, d_latent), dtype=torch.bfloat16, device=q.device)
-    _require(out, "out", (torch.bfloat16,), 3)
-    if tuple(out.shape) != (B, H, d_latent):
-        raise ValueError(f"out must be {(B, H, d_latent)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 3)
+        if out.shape != (B, H, d_latent):
+            raise ValueError(f"out must be {(B, H, d_latent)}")
     need = mla_decode_workspace_bytes(B, H, T, d_latent)
     if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
         workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
@@ -245,24 +263,26 @@ def gdn_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, alpha: torch.T
     _require(S_in, "S_in", (torch.float32,), 4)
     B, Hk, dk = q.shape
     Bv, Hv, dv = v.shape
-    if tuple(k.shape) != (B, Hk, dk) or Bv != B:
+    if k.shape != (B, Hk, dk) or Bv != B:
         raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} v {tuple(v.shape)}")
     if Hv % Hk:
         raise ValueError(f"n_v_heads ({Hv}) must be a multiple of n_k_heads ({Hk})")
-    if tuple(alpha.shape) != (B, Hv) or tuple(beta.shape) != (B, Hv):
+    if alpha.shape != (B, Hv) or beta.shape != (B, Hv):
         raise ValueError(f"alpha/beta must be {(B, Hv)}")
-    if tuple(S_in.shape) != (B, Hv, dk, dv):
+    if S_in.shape != (B, Hv, dk, dv):
         raise ValueError(f"S_in must be {(B, Hv, dk, dv)}, got {tuple(S_in.shape)}")
     if S_out is None:
         S_out = torch.empty_like(S_in)
-    _require(S_out, "S_out", (torch.float32,), 4)
-    if S_out.shape != S_in.shape:
-        raise ValueError("S_out must match S_in")
+    else:
+        _require(S_out, "S_out", (torch.float32,), 4)
+        if S_out.shape != S_in.shape:
+            raise ValueError("S_out must match S_in")
     if o is None:
         o = torch.empty((B, Hv, dv), dtype=q.dtype, device=q.device)
-    _require(o, "o", (q.dtype,), 3)
-    if tuple(o.shape) != (B, Hv, dv):
-        raise ValueError(f"o must be {(B, Hv, dv)}")
+    else:
+        _require(o, "o", (q.dtype,), 3)
+        if o.shape != (B, Hv, dv):
+            raise ValueError(f"o must be {(B, Hv, dv)}")
     _same_device(q, k, v, alpha, beta, S_in, S_out, o)
     _lib.call("mx_gdn_decode", q.data_ptr(), k.data_ptr(), v.data_ptr(), alpha.data_ptr(), beta.data_ptr(),
               S_in.data_ptr(), S_out.data_ptr(), o.data_ptr(), B, Hk, Hv, dk, dv, _IO_DTYPES[q.dtype],
@@ -291,22 +311,24 @@ def kda_decode(q, k, v, g, beta, S_in, S_out=None, o=None):
     _require(S_in, "S_in", (torch.float32,), 4)
     B, Hh, dk = q.shape
     dv = v.shape[2]
-    if tuple(k.shape) != (B, Hh, dk) or tuple(g.shape) != (B, Hh, dk) or tuple(v.shape[:2]) != (B, Hh):
+    if k.shape != (B, Hh, dk) or g.shape != (B, Hh, dk) or v.shape[:2] != (B, Hh):
         raise ValueError(f"shape mismatch: q {tuple(q.shape)} k {tuple(k.shape)} g {tuple(g.shape)} v {tuple(v.shape)}")
-    if tuple(beta.shape) != (B, Hh):
+    if beta.shape != (B, Hh):
         raise ValueError(f"beta must be {(B, Hh)}")
-    if tuple(S_in.shape) != (B, Hh, dk, dv):
+    if S_in.shape != (B, Hh, dk, dv):
         raise ValueError(f"S_in must be {(B, Hh, dk, dv)}, got {tuple(S_in.shape)}")
     if S_out is None:
         S_out = torch.empty_like(S_in)
-    _require(S_out, "S_out", (torch.float32,), 4)
-    if S_out.shape != S_in.shape:
-        raise ValueError("S_out must match S_in")
+    else:
+        _require(S_out, "S_out", (torch.float32,), 4)
+        if S_out.shape != S_in.shape:
+            raise ValueError("S_out must match S_in")
     if o is None:
         o = torch.empty((B, Hh, dv), dtype=q.dtype, device=q.device)
-    _require(o, "o", (q.dtype,), 3)
-    if tuple(o.shape) != (B, Hh, dv):
-        raise ValueError(f"o must be {(B, Hh, dv)}")
+    else:
+        _require(o, "o", (q.dtype,), 3)
+        if o.shape != (B, Hh, dv):
+            raise ValueError(f"o must be {(B, Hh, dv)}")
     _same_device(q, k, v, g, beta, S_in, S_out, o)
     _lib.call("mx_kda_decode", q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(),
               S_in.data_ptr(), S_out.data_ptr(), o.data_ptr(), B, Hh, dk, dv, _IO_DTYPES[q.dtype], _stream())
@@ -327,7 +349,7 @@ def quant_fp8_act(x, q=None, scales=None):
     if scales is None:
         scales = torch.empty((M, K // 128), dtype=torch.float32, device=x.device)
     _require(scales, "scales", (torch.float32,), 2)
-    if tuple(q.shape) != (M, K) or tuple(scales.shape) != (M, K // 128):
+    if q.shape != (M, K) or scales.shape != (M, K // 128):
         raise ValueError(f"q must be {(M, K)} and scales {(M, K // 128)}")
     _same_device(x, q, scales)
     _lib.call("mx_quant_fp8_act", x.data_ptr(), q.data_ptr(), scales.data_ptr(), M, K, K, _IO_DTYPES[x.dtype],
@@ -345,9 +367,10 @@ def gemm_bf16_batched(a, b, out=None):
     N = b.shape[2]
     if out is None:
         out = torch.empty((nb, M, N), dtype=torch.bfloat16, device=a.device)
-    _require(out, "out", (torch.bfloat16,), 3)
-    if tuple(out.shape) != (nb, M, N):
-        raise ValueError(f"out must be {(nb, M, N)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 3)
+        if out.shape != (nb, M, N):
+            raise ValueError(f"out must be {(nb, M, N)}")
     _same_device(a, b, out)
     _lib.call("mx_gemm_bf16_batched", a.data_ptr(), b.data_ptr(), out.data_ptr(), nb, M, N, K, K, N, N,
               M * K, K * N, M * N, _stream())
@@ -375,9 +398,10 @@ def mla_absorb_q(q_nope, w_uk, out=None):
     dc = w_uk.shape[2]
     if out is None:
         out = torch.empty((B, Hh, dc), dtype=torch.bfloat16, device=q_nope.device)
-    _require(out, "out", (torch.bfloat16,), 3)
-    if tuple(out.shape) != (B, Hh, dc):
-        raise ValueError(f"out must be {(B, Hh, dc)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 3)
+        if out.shape != (B, Hh, dc):
+            raise ValueError(f"out must be {(B, Hh, dc)}")
     _same_device(q_nope, w_uk, out)
     _head_gemm(q_nope, w_uk, out, dc)
     return out
@@ -395,9 +419,10 @@ def mla_up_project(o_lat, w_uv, out=None):
     dv = w_uv.shape[2]
     if out is None:
         out = torch.empty((B, Hh, dv), dtype=torch.bfloat16, device=o_lat.device)
-    _require(out, "out", (torch.bfloat16,), 3)
-    if tuple(out.shape) != (B, Hh, dv):
-        raise ValueError(f"out must be {(B, Hh, dv)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 3)
+        if out.shape != (B, Hh, dv):
+            raise ValueError(f"out must be {(B, Hh, dv)}")
     _same_device(o_lat, w_uv, out)
     _head_gemm(o_lat, w_uv, out, dv)
     return out
@@ -418,16 +443,17 @@ def mla_decode_absorbed(q_nope, q_rope, kv, w_uk, w_uv, scale, out=None, workspa
         _require(t, n, (torch.bfloat16,), 3)
     B, Hh, dn = q_nope.shape
     T = kv.shape[1]
-    if tuple(q_rope.shape) != (B, Hh, 64) or kv.shape[0] != B or kv.shape[2] != 576:
+    if q_rope.shape != (B, Hh, 64) or kv.shape[0] != B or kv.shape[2] != 576:
         raise ValueError(f"q_rope must be {(B, Hh, 64)} and kv [B, T, 576]")
-    if tuple(w_uk.shape) != (Hh, dn, 512) or w_uv.shape[0] != Hh or w_uv.shape[1] != 512:
+    if w_uk.shape != (Hh, dn, 512) or w_uv.shape[0] != Hh or w_uv.shape[1] != 512:
         raise ValueError(f"w_uk must be {(Hh, dn, 512)} and w_uv [{Hh}, 512, dv]")
     dv = w_uv.shape[2]
     if out is None:
         out = torch.empty((B, Hh, dv), dtype=torch.bfloat16, device=q_nope.device)
-    _require(out, "out", (torch.bfloat16,), 3)
-    if tuple(out.shape) != (B, Hh, dv):
-        raise ValueError(f"out must be {(B, Hh, dv)}")
+    else:
+        _require(out, "out", (torch.bfloat16,), 3)
+        if out.shape != (B, Hh, dv):
+            raise ValueError(f"out must be {(B, Hh, dv)}")
     need = mla_decode_absorbed_workspace_bytes(B, Hh, T)
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(need + 256, dtype=torch.uint8, device=q_nope.device)

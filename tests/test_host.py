@@ -78,3 +78,26 @@ def test_missing_library_fails_loudly(tmp_path):
     proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, env=env, timeout=300)
     assert proc.returncode == 3, proc.stdout + proc.stderr
     assert "not found" in proc.stdout
+
+
+@pytest.mark.parametrize("make,error", [
+    (lambda: [1.0], TypeError),
+    (lambda: torch.zeros(2, 2), TypeError),                                    # dtype
+    (lambda: torch.zeros(2, 2, dtype=torch.bfloat16), ValueError),             # not on the device
+])
+def test_require_rejects(make, error):
+    with pytest.raises(error):
+        ops._require(make(), "x", (torch.bfloat16,), 2)
+
+
+def test_same_device_names_the_devices():
+    class On:
+        def __init__(self, d):
+            self.d, self.device = d, f"cuda:{d}"
+
+        def get_device(self):
+            return self.d
+
+    ops._same_device(On(0), On(0), On(0))
+    with pytest.raises(ValueError, match="cuda:0.*cuda:1"):
+        ops._same_device(On(0), On(0), On(1))
