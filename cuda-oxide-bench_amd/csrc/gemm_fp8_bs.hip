@@ -21,8 +21,8 @@
 //    follows them, so its FMAs run while those two MFMAs execute.
 //  * 256x256 tiles, 8 waves (2 in m x 4 in n, two per SIMD), each wave
 //    128(m) x 64(n): the fp32 accumulators stay in architectural VGPRs,
-//    where the promotion FMAs can reach them.  Grids under 256 such tiles
-//    use 128x128 tiles.
+//    where the promotion FMAs can reach them.  192x256, 128x256 and 128x128
+//    tiles where they fill the rounds of workgroups better (gemm_path).
 //  * A and B go HBM -> LDS with global_load_lds_dwordx4 (no VGPR staging),
 //    filling the 160 KB of LDS with two rings: A in whole scale blocks (BM
 //    rows of 128 bytes, so every load request is a full 128-byte line; rows
@@ -105,6 +105,19 @@ __device__ __forceinline__ void ld_scales_if(u32x2 (&x)[4], const float* sbase, 
       : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), [b] "s"(sbase), [go] "s"(go)
       : "memory", "scc");
 }
+__device__ __forceinline__ void ld_scales_if(u32x2 (&x)[3], const float* sbase, const uint32_t (&voff)[3],
+                                             uint32_t go) {
+  asm volatile(
+      "s_cmp_eq_u32 %[go], 0\n\t"
+      "s_cbranch_scc1 1f\n\t"
+      "global_load_dwordx2 %0, %3, %[b]\n\t"
+      "global_load_dwordx2 %1, %4, %[b]\n\t"
+      "global_load_dwordx2 %2, %5, %[b]\n"
+      "1:"
+      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2])
+      : "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), [b] "s"(sbase), [go] "s"(go)
+      : "memory", "scc");
+}
 __device__ __forceinline__ void ld_scales_if(u32x2 (&x)[2], const float* sbase, const uint32_t (&voff)[2],
                                              uint32_t go) {
   asm volatile(
@@ -122,10 +135,12 @@ __device__ __forceinline__ void ld_scales_if(u32x2 (&x)[2], const float* sbase, 
 template <int N, typename S, int FM>
 __device__ __forceinline__ void wait_scales(S (&sa)[FM], float& sb) {
   static_assert(N >= 0 && N < 16, "vmcnt immediate");
-  static_assert(FM == 2 || FM == 4, "scale registers");
+  static_assert(FM >= 2 && FM <= 4, "scale registers");
   if constexpr (FM == 4)
     asm volatile("s_waitcnt vmcnt(%5)" : "+v"(sa[0]), "+v"(sa[1]), "+v"(sa[2]), "+v"(sa[3]), "+v"(sb) : "i"(N)
                  : "memory");
+  else if constexpr (FM == 3)
+    asm volatile("s_waitcnt vmcnt(%4)" : "+v"(sa[0]), "+v"(sa[1]), "+v"(sa[2]), "+v"(sb) : "i"(N) : "memory");
   else
     asm volatile("s_waitcnt vmcnt(%3)" : "+v"(sa[0]), "+v"(sa[1]), "+v"(sb) : "i"(N) : "memory");
 }
@@ -464,31 +479,37 @@ static int launch(const void* A, const float* sA, const void* B, const float* sB
 // ---------------------------------------------------------------------------
 // Small M (decode batches) or few tiles: the product is a stream of the
 // weights B, and 128x128 tiles would leave most CUs idle.
-//  * A workgroup owns 32 columns x 32 MF rows of C, NW waves; wave w takes
+//  * A workgroup owns 32 NC columns x 32 MF rows of C, NW waves; wave w takes
 //    the scale blocks kb = w, w + NW, ... of K, so every workgroup streams
-//    its 32 columns of B once.  The row chunks of a column block and the
+//    its columns of B once.  The row chunks of a column block and the
 //    neighbouring column blocks run on one XCD, where they share B's
 //    128-byte lines in L2.
 //  * Each wave has a private ring of NSL slots, one scale block per slot:
-//    A (32 MF rows x 128 B), B (128 k-rows x 32 B) and the block's scales
+//    A (32 MF rows x 128 B), B (128 k-rows x 32 NC B) and the block's scales
 //    (one activation scale per row, the weight scale) by direct loads, so
 //    one vmcnt wait lands all of them and no register is written behind
 //    the compiler's back.  Slots are private, so the block loop has no
 //    barrier; the wave issues block i+NSL-1 before it waits for block i.
+//  * What bounds it is the CU's rate of line requests, about one per 3-4
+//    clocks, whether a request brings 32, 64 or 128 bytes: one row of B costs a
+//    workgroup the same at 32 columns as at 128 (probe, 64x4096x7168, 18 us:
+//    without B's loads 9 us, without the MFMAs and fragment reads 18, with B
+//    stored as dense 4 KB blocks 10).  So 64 columns where the grid still fills
+//    the CUs, and eight waves with shallow rings where it does not.
 //  * C^T = B^T . A^T on 32x32x64 fp8 MFMAs as in the main kernel: B^T
-//    fragments by ds_read_b64_tr_b8 from 32-byte rows (eight rows fill the
-//    256 banks' width, so a 32-lane phase is conflict free unswizzled), A^T
-//    fragments by two ds_read_b128 from 128-byte rows whose chunk c sits at
-//    c ^ ((m >> 1) & 7).  Two MFMAs build the block's partial, promoted with
-//    one FMA per element: acc += (sA sB) * partial.
-//  * The waves' accumulators meet in LDS at the end; wave i sums the four
-//    result registers of every wave that hold n = 8i + 4(l/32) + {0..3}
-//    and stores them (with 4 waves every register is summed once).
+//    fragments by ds_read_b64_tr_b8 (swz_sb), A^T fragments by two ds_read_b128
+//    from 128-byte rows whose chunk c sits at c ^ ((m >> 1) & 7).  Two MFMAs
+//    build the block's partial, promoted with one FMA per element: acc +=
+//    (sA sB) * partial.
+//  * The waves' accumulators meet in LDS at the end; four waves sum the result
+//    registers of every wave that hold n = 8i + 4(l/32) + {0..3}, i their
+//    number, and store them.
 // ---------------------------------------------------------------------------
-template <int MF, int NW, int NSL>
+template <int MF, int NC, int NW, int NSL>
 struct SmallCfg {
+  static constexpr int BN = 32 * NC;           // columns per workgroup
   static constexpr int A_B = 32 * MF * 128;   // A rows of one scale block
-  static constexpr int B_B = 128 * 32;         // B k-rows of one scale block
+  static constexpr int B_B = 128 * BN;         // B k-rows of one scale block
   static constexpr int SA_OFF = A_B + B_B, SB_OFF = SA_OFF + 256;  // 64 row scales, 64 copies of sB
   static constexpr int SLOT = SB_OFF + 256;
   static constexpr int A_L = A_B / 1024, B_L = B_B / 1024;
@@ -497,7 +518,8 @@ struct SmallCfg {
   static_assert(NW == 4 || NW == 8, "waves");
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert((NSL - 1) * VM < 64, "vmcnt range");
-  static_assert(NW * MF * 64 * 16 * 4 <= LDS, "reduction area");
+  static_assert(NW * MF * NC * 64 * 16 * 4 <= LDS, "reduction area");
+  static_assert(NC == 1 || NC == 2, "columns within one weight-scale block, row swizzle");
 };
 
 // f(integral_constant<int, I>) for I = 0 .. N-1, in order.
@@ -510,6 +532,13 @@ __device__ __forceinline__ void unroll_n(F&& f) {
 }
 
 __device__ __forceinline__ int swz_sa(int m) { return (m >> 1) & 7; }
+// B rows of 64 bytes: eight consecutive k-rows x 32 bytes (a transposing read
+// phase) span the 256-byte bank window twice, so rows 4..7 swap their halves;
+// rows of 32 bytes fill it once.
+template <int NC>
+__device__ __forceinline__ int swz_sb(int k) {
+  return NC == 1 ? 0 : ((k >> 2) & 1) << 1;
+}
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -527,24 +556,24 @@ __device__ __forceinline__ void wait_vmcnt_mem() {
 }
 #pragma clang diagnostic pop
 
-template <int MF, int NW, int NSL>
+template <int MF, int NC, int NW, int NSL>
 __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const uint8_t* __restrict__ A,
                                                                       const float* __restrict__ sA,
                                                                       const uint8_t* __restrict__ B,
                                                                       const float* __restrict__ sB,
                                                                       uint16_t* __restrict__ C, int M, int N,
                                                                       int K) {
-  using CF = SmallCfg<MF, NW, NSL>;
+  using CF = SmallCfg<MF, NC, NW, NSL>;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Workgroup -> (32-column block, chunk of 32 MF rows), the row chunks of a
+  // Workgroup -> (BN-column block, chunk of 32 MF rows), the row chunks of a
   // column block adjacent: consecutive column blocks share 128-byte lines
   // of B, and one XCD (one L2) then fetches each line from HBM once.
   const int kblocks = K / SBK;
   const int nmc = (M + 32 * MF - 1) / (32 * MF);
   const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
-  const int n0 = (wid / nmc) * 32, m0 = (wid % nmc) * 32 * MF;
+  const int n0 = (wid / nmc) * CF::BN, m0 = (wid % nmc) * 32 * MF;
   A += (size_t)m0 * K;
   sA += (size_t)m0 * kblocks;
   C += (size_t)m0 * N;
@@ -554,8 +583,9 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
   const uint32_t ring = lds_addr(smem) + wave * NSL * CF::SLOT;
 
   // Direct-load lane offsets.  A load n: rows 8n + l/8, LDS chunk l%8 taking
-  // global chunk (l%8) ^ swz(row); B load n: k-rows 32n + l/2, chunk l%2
-  // (columns past N re-read the last 16 valid ones; never stored).
+  // global chunk (l%8) ^ swz(row); B load n: its k-rows' chunks in lane order,
+  // chunk c of k-row k at c ^ swz_sb(k) (columns past N re-read the last 16
+  // valid ones; never stored).
   uint32_t a_off[CF::A_L], b_off[CF::B_L];
 #pragma unroll
   for (int n = 0; n < CF::A_L; ++n) {
@@ -564,8 +594,10 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
   }
 #pragma unroll
   for (int n = 0; n < CF::B_L; ++n) {
-    const int col = min(n0 + 16 * (lane & 1), N - 16) - n0;
-    b_off[n] = (uint32_t)(32 * n + (lane >> 1)) * (uint32_t)N + col;
+    constexpr int CH = CF::BN / 16;  // 16-byte chunks per k-row
+    const int row = (64 / CH) * n + lane / CH;
+    const int col = min(n0 + 16 * ((lane % CH) ^ swz_sb<NC>(row)), N - 16) - n0;
+    b_off[n] = (uint32_t)row * (uint32_t)N + col;
   }
   // scales: lane l loads the activation scale of row l (rows past M re-read
   // row M-1) and every lane the one weight scale of this column block
@@ -593,23 +625,31 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
 #pragma unroll
     for (int e = 0; e < 2; ++e) a_col[st][e] = am * 128 + 16 * ((4 * st + 2 * ah + e) ^ swz_sa(am));
   const int q = lane >> 4, jj = (lane & 15) >> 1, hh = lane & 1;
-  const uint32_t b_col = CF::A_B + (32 * (q >> 1) + jj) * 32 + 16 * (q & 1) + 8 * hh;
-
-  f32x16 acc[MF];
+  uint32_t b_col[NC];  // k-rows 8 apart share the swizzle
 #pragma unroll
-  for (int f = 0; f < MF; ++f) acc[f] = f32x16{};
+  for (int c = 0; c < NC; ++c)
+    b_col[c] = CF::A_B + (32 * (q >> 1) + jj) * CF::BN + 16 * ((2 * c + (q & 1)) ^ swz_sb<NC>(jj)) + 8 * hh;
+
+  f32x16 acc[NC][MF];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int f = 0; f < MF; ++f) acc[c][f] = f32x16{};
 
   auto compute = [&](auto slot_tag) {
     constexpr int I = decltype(slot_tag)::value;
     const uint32_t st = ring + I * CF::SLOT;
-    i32x8 bt[2], at[2][MF];
+    i32x8 bt[NC][2], at[2][MF];
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
-      u32x2 v[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = lds_read_tr8_at(st + b_col + 64 * s2 * 32 + 8 * r * 32);
-      bt[s2] = i32x8{(int)v[0][0], (int)v[0][1], (int)v[1][0], (int)v[1][1],
-                     (int)v[2][0], (int)v[2][1], (int)v[3][0], (int)v[3][1]};
+      for (int c = 0; c < NC; ++c) {
+        u32x2 v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = lds_read_tr8_at(st + b_col[c] + (64 * s2 + 8 * r) * CF::BN);
+        bt[c][s2] = i32x8{(int)v[0][0], (int)v[0][1], (int)v[1][0], (int)v[1][1],
+                          (int)v[2][0], (int)v[2][1], (int)v[3][0], (int)v[3][1]};
+      }
 #pragma unroll
       for (int f = 0; f < MF; ++f) {
         const uint32_t r = st + 32 * f * 128;
@@ -624,9 +664,12 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
     for (int f = 0; f < MF; ++f) {
       const float sav = *reinterpret_cast<const __attribute__((address_space(3))) float*>(
           (uintptr_t)(st + CF::SA_OFF + 4 * (32 * f + am)));
-      f32x16 p = mfma32_fp8(bt[0], at[0][f], f32x16{});
-      p = mfma32_fp8(bt[1], at[1][f], p);
-      acc[f] += (sav * sbv) * p;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        f32x16 p = mfma32_fp8(bt[c][0], at[0][f], f32x16{});
+        p = mfma32_fp8(bt[c][1], at[1][f], p);
+        acc[c][f] += (sav * sbv) * p;
+      }
     }
   };
 
@@ -652,23 +695,28 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
   });
   wait_vmcnt<0>();  // no DMA may land in the ring once it is reused below
 
-  // ---- accumulators meet in LDS: [wave][f][e][lane] floats ----
+  // ---- accumulators meet in LDS: [wave][c][f][e][lane] floats ----
   __syncthreads();
   float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
-  for (int f = 0; f < MF; ++f)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) red[((wave * MF + f) * 16 + e) * 64 + lane] = acc[f][e];
+    for (int f = 0; f < MF; ++f)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[(((wave * NC + c) * MF + f) * 16 + e) * 64 + lane] = acc[c][f][e];
   __syncthreads();
-  if (wave < 4) {
-    const int gn = n0 + 8 * wave + 4 * ah;
+  // result quad 4 i .. 4 i + 3 of column fragment c to wave i (and i + 4)
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if (wave / 4 != c % (NW / 4)) continue;
+    const int gn = n0 + 32 * c + 8 * (wave % 4) + 4 * ah;
 #pragma unroll
     for (int f = 0; f < MF; ++f) {
       float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < NW; ++w)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] += red[((w * MF + f) * 16 + 4 * wave + j) * 64 + lane];
+        for (int j = 0; j < 4; ++j) v[j] += red[(((w * NC + c) * MF + f) * 16 + 4 * (wave % 4) + j) * 64 + lane];
       const int gm = 32 * f + am;
       if (gm < M && gn < N)
         st64(C + (size_t)gm * N + gn, u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
@@ -676,18 +724,60 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_fp8_bs_smallm_kernel(const ui
   }
 }
 
-template <int MF, int NW, int NSL>
+template <int MF, int NC, int NW, int NSL>
 static int launch_smallm(const void* A, const float* sA, const void* B, const float* sB, void* C, int M, int N, int K,
                          hipStream_t stream) {
-  using CF = SmallCfg<MF, NW, NSL>;
-  constexpr auto kern = gemm_fp8_bs_smallm_kernel<MF, NW, NSL>;
+  using CF = SmallCfg<MF, NC, NW, NSL>;
+  constexpr auto kern = gemm_fp8_bs_smallm_kernel<MF, NC, NW, NSL>;
   MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
-  const long long grid = (long long)((N + 31) / 32) * ((M + 32 * MF - 1) / (32 * MF));
+  const long long grid = (long long)((N + CF::BN - 1) / CF::BN) * ((M + 32 * MF - 1) / (32 * MF));
   if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), CF::LDS, stream, (const uint8_t*)A, sA,
                      (const uint8_t*)B, sB, (uint16_t*)C, M, N, K);
   MX_RETURN_IF_HIP(hipGetLastError());
   return MX_OK;
+}
+
+// The kernels of mx_gemm_fp8_bs, and what one launch of each takes in
+// microseconds: fixed + rounds (round + step K/128) + fill (tiles / 256) K/128
+// with rounds = ceil(tiles / 256).  Fitted (relative least squares, no negative
+// term) to 180 random shapes, M 1..8192, N and K 512..8192, each timed on every
+// kernel by graph replay; the kernel picked is on average 0.7% slower than the
+// fastest.  Against 128x128 and 256x256 tiles and 32-column streams of four
+// waves, chosen by M and by rounds: 8% in geometric mean; 128x7168x2048 16.3 ->
+// 10.6 us, 256x4096x4096 26.1 -> 15.1 and 524x1536x8064 54 -> 23 (64x64
+// streams), 3072^3 44.8 -> 37.1 (192x256), 730x7120x2816 34.7 -> 29.0 (128x256),
+// 64x4096x7168 20.5 -> 18.5 (eight waves).  Not kept: 256x128 tiles, 32x64
+// streams and 32x32 streams of four waves were the fastest by up to 6, 8 and
+// 1% for 2 to 5 shapes in 180, and without them the mean is the same.
+enum class Path { Stream32, Stream64, Stream64x64, T128, T128x256, T192x256, T256 };
+struct Kernel {
+  Path path;
+  int bm, bn;
+  float fixed, round, step, fill;
+};
+constexpr Kernel kKernels[] = {
+    {Path::Stream32, 32, 32, 1.600f, 1.984f, 0.160f, 0.096f},
+    {Path::Stream64, 64, 32, 1.404f, 2.602f, 0.184f, 0.117f},
+    {Path::Stream64x64, 64, 64, 1.475f, 2.611f, 0.255f, 0.112f},
+    {Path::T128, 128, 128, 3.428f, 0.0f, 0.743f, 0.087f},
+    {Path::T128x256, 128, 256, 0.753f, 3.230f, 0.987f, 0.272f},
+    {Path::T192x256, 192, 256, 0.0f, 5.082f, 1.084f, 0.451f},
+    {Path::T256, 256, 256, 0.0f, 5.874f, 1.262f, 0.656f},
+};
+static Path gemm_path(int M, int N, int K) {
+  Path best = Path::T256;
+  double least = 0;
+  for (const Kernel& k : kKernels) {
+    const double tiles = (double)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
+    const double rounds = __builtin_ceil(tiles / 256), kb = K / 128.0;
+    const double t = k.fixed + rounds * (k.round + k.step * kb) + k.fill * kb * tiles / 256;
+    if (&k == kKernels || t < least) {
+      best = k.path;
+      least = t;
+    }
+  }
+  return best;
 }
 
 }  // namespace gemm8
@@ -706,29 +796,21 @@ extern "C" int mx_gemm_fp8_bs(const void* A, const float* sA, const void* B, con
   if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15) return MX_ERR_ALIGN;
   if (((uintptr_t)sA | (uintptr_t)sB) & 3) return MX_ERR_ALIGN;
   hipStream_t s = (hipStream_t)stream;
-  const long long tiles256 = (long long)((M + 255) / 256) * ((N + 255) / 256);
-  const long long tiles128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  // Rounds of 256 workgroups: a round of 256x256 tiles takes ~2.4 times a
-  // round of 128x128 ones at the same K (measured 1.95-2.55 at 2048-3072),
-  // so the big tile wins unless the small one needs fewer than 2.4 times
-  // its rounds (3072^3: 1 round against 3, 57 vs 72 us; 2560^3: 1 against
-  // 2, 44 vs 38 us).
-  constexpr int SMALLM_NW = 4;  // waves of the weight-streaming kernel (each takes every 4th scale block)
-  // Decode-sized M, or at most 64 tiles of 128x128 with M <= 512: stream
-  // the weights with 32-column workgroups (graph-replayed: 256x4096x4096
-  // 27.5 -> 22.5 us, 512x1024x4096 27.4 -> 12.3 us; 1024^3 stays tiled,
-  // 10.6 against 11.8 us).
-  if (M <= 32) return mx::gemm8::launch_smallm<1, SMALLM_NW, 4>(A, sA, B, sB, C, M, N, K, s);
-  const long long tiles128s = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  if (M <= 64 || (tiles128s <= 64 && M <= 512))
-    return mx::gemm8::launch_smallm<2, SMALLM_NW, 3>(A, sA, B, sB, C, M, N, K, s);
-  const long long r256 = (tiles256 + 255) / 256, r128 = (tiles128 + 255) / 256;
-  const bool big = tiles256 >= 256 || 12 * r256 < 5 * r128;
+  using namespace mx::gemm8;
+  const Path path = gemm_path(M, N, K);
   // activation scales four blocks per 8-byte load when the blocks come in
   // fours and sA is 8-byte aligned (the interface asks only for 4)
-  if (K % 512 == 0 && ((uintptr_t)sA & 7) == 0)
-    return big ? mx::gemm8::launch<256, 256, true>(A, sA, B, sB, C, M, N, K, s)
-               : mx::gemm8::launch<128, 128, true>(A, sA, B, sB, C, M, N, K, s);
-  return big ? mx::gemm8::launch<256, 256, false>(A, sA, B, sB, C, M, N, K, s)
-             : mx::gemm8::launch<128, 128, false>(A, sA, B, sB, C, M, N, K, s);
+  const bool gs = K % 512 == 0 && ((uintptr_t)sA & 7) == 0;
+#define MX_TILED(BM, BN) \
+  (gs ? launch<BM, BN, true>(A, sA, B, sB, C, M, N, K, s) : launch<BM, BN, false>(A, sA, B, sB, C, M, N, K, s))
+  switch (path) {
+    case Path::Stream32: return launch_smallm<1, 1, 8, 2>(A, sA, B, sB, C, M, N, K, s);
+    case Path::Stream64: return launch_smallm<2, 1, 4, 3>(A, sA, B, sB, C, M, N, K, s);
+    case Path::Stream64x64: return launch_smallm<2, 2, 4, 2>(A, sA, B, sB, C, M, N, K, s);
+    case Path::T128: return MX_TILED(128, 128);
+    case Path::T128x256: return MX_TILED(128, 256);
+    case Path::T192x256: return MX_TILED(192, 256);
+    default: return MX_TILED(256, 256);
+  }
+#undef MX_TILED
 }

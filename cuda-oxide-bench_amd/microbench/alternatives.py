@@ -101,19 +101,16 @@ FP8_PARTS = {
         ("s_m[mf] = sa_of(j & 3, mf) * sb_n;", "s_m[mf] = sa_of(j & (G - 1), mf) * sb_n;"),
         ("template <int BM, int BN, bool GS>\nstatic int launch(", "template <int BM, int BN, int G>\nstatic int launch("),
         ("  constexpr auto kern = gemm_fp8_bs_kernel<BM, BN, GS>;", "  constexpr auto kern = gemm_fp8_bs_kernel<BM, BN, G>;"),
-        ("  if (K % 512 == 0 && ((uintptr_t)sA & 7) == 0)\n"
-         "    return big ? mx::gemm8::launch<256, 256, true>(A, sA, B, sB, C, M, N, K, s)\n"
-         "               : mx::gemm8::launch<128, 128, true>(A, sA, B, sB, C, M, N, K, s);\n"
-         "  return big ? mx::gemm8::launch<256, 256, false>(A, sA, B, sB, C, M, N, K, s)\n"
-         "             : mx::gemm8::launch<128, 128, false>(A, sA, B, sB, C, M, N, K, s);",
-         "  if (K % 1024 == 0 && ((uintptr_t)sA & 15) == 0)\n"
-         "    return big ? mx::gemm8::launch<256, 256, 8>(A, sA, B, sB, C, M, N, K, s)\n"
-         "               : mx::gemm8::launch<128, 128, 8>(A, sA, B, sB, C, M, N, K, s);\n"
-         "  if (K % 512 == 0 && ((uintptr_t)sA & 7) == 0)\n"
-         "    return big ? mx::gemm8::launch<256, 256, 4>(A, sA, B, sB, C, M, N, K, s)\n"
-         "               : mx::gemm8::launch<128, 128, 4>(A, sA, B, sB, C, M, N, K, s);\n"
-         "  return big ? mx::gemm8::launch<256, 256, 1>(A, sA, B, sB, C, M, N, K, s)\n"
-         "             : mx::gemm8::launch<128, 128, 1>(A, sA, B, sB, C, M, N, K, s);"),
+        ("  switch (path) {\n    case Path::Stream32:",
+         "  if (path == Path::T256 || path == Path::T128) {\n"
+         "    const bool big = path == Path::T256;\n"
+         "    if (K % 1024 == 0 && ((uintptr_t)sA & 15) == 0)\n"
+         "      return big ? launch<256, 256, 8>(A, sA, B, sB, C, M, N, K, s) : launch<128, 128, 8>(A, sA, B, sB, C, M, N, K, s);\n"
+         "    if (gs) return big ? launch<256, 256, 4>(A, sA, B, sB, C, M, N, K, s) : launch<128, 128, 4>(A, sA, B, sB, C, M, N, K, s);\n"
+         "    return big ? launch<256, 256, 1>(A, sA, B, sB, C, M, N, K, s) : launch<128, 128, 1>(A, sA, B, sB, C, M, N, K, s);\n"
+         "  }\n  switch (path) {\n    case Path::Stream32:"),
+        ("  (gs ? launch<BM, BN, true>(A, sA, B, sB, C, M, N, K, s) : launch<BM, BN, false>(A, sA, B, sB, C, M, N, K, s))",
+         "  (gs ? launch<BM, BN, 4>(A, sA, B, sB, C, M, N, K, s) : launch<BM, BN, 1>(A, sA, B, sB, C, M, N, K, s))"),
     ],
     # Each block's LDS read bases (lane address + slot offset) computed once
     # and hidden from the compiler, so every fragment read carries its own

@@ -55,9 +55,9 @@ def test_parity_vs_oracle(ops, mnk):
                                  (64, 2048, 7168), (48, 272, 640), (20, 4112, 2944), (256, 512, 4096), (130, 1024, 2048),
                                  (500, 1008, 1024), (512, 1024, 384)])
 def test_small_m_path(ops, mnk):
-    """M <= 64 (decode batches), or at most 64 tiles of 128x128 with
-    M <= 512, runs the weight-streaming kernel: workgroups of 32 columns x
-    32 or 64 rows, scale blocks split over the waves.  Single rows, N not a
+    """Decode batches and products of few tiles run the weight-streaming
+    kernel: workgroups of 32 columns x 32 or 64 rows, scale blocks split over
+    the waves.  Single rows, N not a
     multiple of 32 (a last block 16 wide), fewer scale blocks than waves
     (K = 128), block counts that do not divide by the wave count, and both
     the one- and two-fragment (M > 32) variants."""
@@ -73,9 +73,8 @@ def test_small_m_path(ops, mnk):
 @pytest.mark.parametrize("mnk", [(4096, 4096, 128), (4096, 4096, 384), (4000, 4352, 640), (4096, 4112, 256),
                                  (3072, 3072, 1024), (3000, 3056, 640)])
 def test_large_tile_path(ops, mnk):
-    """Shapes on the 256x256 kernel: >= 256 such tiles, or fewer when 128x128
-    tiles would need more than 2.4 times the rounds of workgroups (3072^3:
-    144 tiles against 576).  One scale block (fewer stages than the ring
+    """Shapes of many tiles (256x256, 192x256 or 128x128, by the launch's
+    estimated time).  One scale block (fewer stages than the ring
     holds), an odd block count, ragged M and N (N = 4352 and 4112: a partial
     last column tile, and a last 128-column scale block only 16 wide)."""
     m, n, k = mnk
@@ -85,6 +84,31 @@ def test_large_tile_path(ops, mnk):
     ref = ofp8.gemm_fp8_bs_ref_torch(a8, sa, b8, sb)
     err = normwise_rel_err(c, ref)
     assert err <= TOL, f"normwise rel err {err:.3e}"
+
+
+@pytest.mark.parametrize("mnk", [(1000, 8208, 256), (2111, 4112, 256), (3000, 3088, 512), (2500, 4112, 640),
+                                 (385, 8208, 256), (2111, 2064, 256), (1601, 3088, 512), (1000, 4112, 640),
+                                 (1, 8208, 256), (191, 3088, 384), (193, 2064, 640), (2111, 272, 384),
+                                 (129, 3088, 640)])
+def test_wide_tiles_and_streams(ops, mnk):
+    """192x256 tiles (first four), 128x256 tiles (next four) and 64x64 streams,
+    with a last row tile of one to a few rows, a last column tile 16 wide, two
+    scale blocks (fewer than a ring or the waves hold), and K on both sides of
+    the grouped scale loads (512 and not), for sA on and off an 8-byte boundary.
+    Every partial sum is in float32: beside the bf16 result (8 significant bits: 2^-8
+    at most), both sides err by at most K 2^-24 of sum |a b|, under 4 times the
+    largest result here (K <= 640: 3e-4)."""
+    m, n, k = mnk
+    announce(f"fp8 wide tiles {m}x{n}x{k}")
+    a8, sa, b8, sb = inputs.fp8_gemm_inputs(shapes.FP8GemmShape("t", m, n, k))
+    ref = ofp8.gemm_fp8_bs_ref_torch(a8, sa, b8, sb)
+    off = torch.empty(sa.numel() + 1, dtype=torch.float32, device="cuda")[1:].view(sa.shape)
+    off.copy_(sa)
+    assert off.data_ptr() % 8 == 4
+    c = run(ops, a8, sa, b8, sb)
+    assert normwise_rel_err(c, ref) <= 2.0 ** -8 + 3e-4
+    c_off = run(ops, a8, off, b8, sb)
+    assert torch.equal(c.view(torch.int16), c_off.view(torch.int16))
 
 
 @pytest.mark.parametrize("mnk", [(4096, 4096, 512), (2048, 2048, 1024)])
