@@ -16,8 +16,8 @@
 // gemm_bf16_dma64_kernel: tiles of 64x64 to 128x192, single and batched.
 // gemm_bf16_stream_kernel: few rows or few tiles; workgroups of 32 columns x
 // 32 or 64 rows stream B, their waves splitting K.
-// gemm_bf16_smallm_kernel / gemm_bf16_smallm_sk_kernel (batched items with
-// M <= 32): single-wave or K-split 4-wave workgroups over the whole K.
+// gemm_bf16_smallm_kernel / gemm_bf16_smallm_sk_kernel (batched items of few
+// rows): single-wave or K-split 4-wave workgroups over the whole K.
 #include <type_traits>
 
 #include "mx_common.h"
@@ -669,15 +669,18 @@ static int launch_dma16s(const void* A, const void* B, void* C, int M, int N, in
 }
 
 // ---------------------------------------------------------------------------
-// Small-M batched kernel (M <= 32, e.g. one decode batch against one head's
-// weight): weight-streaming, so it needs enough bytes in flight per CU and
+// Small-M batched kernel (e.g. one decode batch against one head's weight; M >
+// 32 in chunks of 32 rows): weight-streaming, so it needs enough bytes in flight per CU and
 // few rounds of workgroups rather than big tiles.  A workgroup is one wave
 // computing a 32 x (32 NF) tile of C over the whole K; 64-deep chunks of A
 // [32][64] and B [64][32 NF] go HBM -> LDS by direct loads into an
 // NS-stage ring, NS-1 chunks ahead (6 stages for narrow tiles, 4 at NF = 4:
 // 48-80 KB of LDS, two workgroups per CU).  A single wave needs no barrier: the ring stage
 // it overwrites was consumed by its own MFMAs, which waited for those
-// reads.  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
+// reads.  The row chunks and column tiles of an item run on one XCD, whose L2
+// then holds its A and B once (against plain order: 16 items of 32 x 128 x 512
+// 3.95 -> 3.44 us, 64 items 6.33 -> 4.31, 128 items of 32 x 512 x 128 7.23 ->
+// 6.87).  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
 // B rows (64 NF bytes) put chunk c of k-row k at c ^ (((k & 3) << 2) mod
 // (4 NF)) so the 4 consecutive k-rows of a transposing read phase occupy
 // distinct 64-byte quarters of the bank sweep (no swizzle needed at NF = 1,
@@ -726,11 +729,14 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
   const int lane = threadIdx.x;
   const int g = lane >> 5;
   const int tiles_n = (N + TN - 1) / TN;
-  const int n0 = (int)(blockIdx.x % tiles_n) * TN;
-  const size_t item = blockIdx.x / tiles_n;
-  A += item * sA;
+  const int nmc = (M + 31) / 32;  // row chunks; those of a column tile, then an item's tiles, on one XCD
+  const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
+  const int n0 = wid / nmc % tiles_n * TN, m0 = wid % nmc * 32;
+  const size_t item = wid / nmc / tiles_n;
+  A += item * sA + (size_t)m0 * lda;
   B += item * sB;
-  C += item * sC;
+  C += item * sC + (size_t)m0 * ldc;
+  M -= m0;
   const int nk = K / SM_BK;
   const uint32_t lds0 = lds_addr(smem);
 
@@ -832,11 +838,14 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5;
   const int tiles_n = (N + TN - 1) / TN;
-  const int n0 = (int)(blockIdx.x % tiles_n) * TN;
-  const size_t item = blockIdx.x / tiles_n;
-  A += item * sA;
+  const int nmc = (M + 31) / 32;  // row chunks; those of a column tile, then an item's tiles, on one XCD
+  const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
+  const int n0 = wid / nmc % tiles_n * TN, m0 = wid % nmc * 32;
+  const size_t item = wid / nmc / tiles_n;
+  A += item * sA + (size_t)m0 * lda;
   B += item * sB;
-  C += item * sC;
+  C += item * sC + (size_t)m0 * ldc;
+  M -= m0;
   const int nkw = K / SM_BK / KW;  // chunks per wave (1..3)
   const int kc0 = wave * nkw;
   const uint32_t lds0 = lds_addr(smem) + wave * nkw * STAGE;
@@ -930,7 +939,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
 
 static int launch_smallm(const void* A, const void* B, void* C, int batch, int M, int N, int K, int lda, int ldb,
                          int ldc, long long sA, long long sB, long long sC, hipStream_t stream) {
-  auto groups = [&](int tn) { return (long long)batch * ((N + tn - 1) / tn); };
+  auto groups = [&](int tn) { return (long long)batch * ((M + 31) / 32) * ((N + tn - 1) / tn); };
   // 4..12 chunks of K, split among 4 waves: one workgroup per 32 x 64 tile
   // when that still gives >= 256 workgroups (one per CU), else 32 x 32.
   const int nkc = K / SM_BK;
@@ -1273,6 +1282,21 @@ static bool batched_small(int M, int K, int lda, int ldb) {
   return M <= 32 && K % 64 == 0 && (long long)lda * 2 * 32 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL;
 }
 
+// More rows take the same kernels, 32 at a time, where that beats 64-row tiles
+// (graph replay; the up-projections of an MLA step with 48 rows per head):
+// K split among four waves while a workgroup per CU is enough (N 128, K 512: 16
+// items 4.62 -> 3.49 us, 64 items 5.39 -> 5.22, but 128 items 7.3 -> 9.1), and
+// one or two chunks of K, which need a single round trip, up to 64 rows (N 512,
+// K 128: 16 items 3.64 -> 3.40, 64 items 6.46 -> 5.85, 32 items 4.14 -> 4.19;
+// 96 rows of 64 items 7.0 -> 9.7).
+static bool batched_rows(int batch, int M, int N, int K, int lda, int ldb) {
+  if (K % 64 || !strides_2g<64>(lda, ldb)) return false;
+  const int nkc = K / SM_BK;
+  const long long rows = (long long)batch * ((M + 31) / 32);
+  if (nkc % 4 == 0 && nkc <= 12) return rows * ((N + 63) / 64) <= 256;
+  return nkc <= 2 && M <= 64 && rows * ((N + 31) / 32) <= 0x7fffffffLL;
+}
+
 // Every check mx_gemm_bf16_batched makes before it launches, the grid
 // limits of the kernel it would pick included, so a caller that chains
 // several products can validate them all before enqueuing any.
@@ -1302,7 +1326,7 @@ extern "C" int mx_gemm_bf16_batched(const void* A, const void* B, void* C, int b
   using namespace mx::gemm;
   if (const int e = batched_check(A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC)) return e;
   hipStream_t s = (hipStream_t)stream;
-  if (batched_small(M, K, lda, ldb))
+  if (batched_small(M, K, lda, ldb) || batched_rows(batch, M, N, K, lda, ldb))
     return launch_smallm(A, B, C, batch, M, N, K, lda, ldb, ldc, strideA, strideB, strideC, s);
   return launch_tiled(gemm_path(M, N, K, lda, ldb, batch), A, B, C, M, N, K, lda, ldb, ldc, s, batch, strideA, strideB,
                       strideC);

@@ -334,10 +334,15 @@ def test_infinity_in_the_last_k_row(ops, mnk):
 
 
 @pytest.mark.parametrize("bmnk", [(5, 40, 1000, 72), (16, 48, 128, 512), (3, 300, 264, 136), (40, 200, 640, 136),
-                                  (30, 600, 400, 104), (2, 33, 8, 8), (70, 130, 200, 24)])
+                                  (30, 600, 400, 104), (2, 33, 8, 8), (70, 130, 200, 24),
+                                  # chunks of 32 rows: K split among the waves (last chunk 1 and 8 rows, ragged N,
+                                  # the most groups and one item more), and one and two chunks of K
+                                  (7, 65, 136, 768), (16, 200, 128, 512), (64, 64, 128, 256), (65, 64, 128, 256),
+                                  (16, 33, 512, 64), (37, 64, 264, 128), (128, 48, 512, 128), (3, 65, 72, 128)])
 def test_batched_larger_items(ops, bmnk):
     """Batched items with more than 32 rows, or a K that is no whole number of
-    64-deep chunks, run the tiled kernels over the batch."""
+    64-deep chunks, run the tiled kernels over the batch, or the small-row
+    kernels in chunks of 32 rows."""
     nb, m, n, k = bmnk
     announce(f"gemm_bf16_batched {nb}x{m}x{n}x{k}")
     g = torch.Generator().manual_seed(nb + m + n + k)
