@@ -14,8 +14,8 @@
 //
 // gemm_bf16_dma16s_kernel: 256x256 tiles, the large products.
 // gemm_bf16_dma64_kernel: tiles of 64x64 to 128x192, single and batched.
-// gemm_bf16_stream_kernel: few rows or few tiles; workgroups of 32 columns x
-// 32 or 64 rows stream B, their waves splitting K.
+// gemm_bf16_stream_kernel: few rows or few tiles; workgroups of 32 or 64
+// columns x 32 or 64 rows stream B, their waves splitting K.
 // gemm_bf16_smallm_kernel / gemm_bf16_smallm_sk_kernel (batched items of few
 // rows): single-wave or K-split 4-wave workgroups over the whole K.
 #include <type_traits>
@@ -984,34 +984,47 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
 // gemm_bf16_stream_kernel: products with few tiles (decode batches, small
 // M or N with a long K) stream the weights B.  Tiles of 64 or more rows
 // would leave most CUs idle.
-//  * A workgroup owns 32 columns x 32 MF rows of C, NW waves; wave w takes
+//  * A workgroup owns 32 NC columns x 32 MF rows of C, NW waves; wave w takes
 //    the 64-deep K blocks kb = w, w + NW, ..., so every workgroup streams its
-//    32 columns of B once.  The row chunks of a column block and the
+//    columns of B once.  The row chunks of a column block and the
 //    neighbouring column blocks run on one XCD, where they share B's
 //    128-byte lines in L2.
 //  * Each wave has a private ring of NSL slots, one K block per slot (A: 32 MF
-//    rows x 128 B, chunk c at c ^ ((m >> 1) & 7); B: 64 k-rows x 64 B), by
+//    rows x 128 B, chunk c at c ^ ((m >> 1) & 7); B: 64 k-rows x 64 NC B), by
 //    direct loads; slots are private, so the block loop has no barrier.
+//  * What bounds it is the CU's rate of line requests (about one per 3-4
+//    clocks, 64 or 128 bytes alike), so 64 columns where they still fill the
+//    CUs; eight waves with rings of two slots keep as many loads in flight as
+//    four with four and reach each block sooner (16x7168x4096 15.3 -> 15.1 us,
+//    1x696x1520 6.2 -> 5.2, 27x512x1280 4.96 -> 4.61).
 //  * C^T = B^T . A^T on 32x32x16 MFMAs: B^T fragments by transposing reads
-//    from the 64-byte B rows (a 32-lane phase covers 4 rows x 64 B, conflict
-//    free unswizzled), A^T fragments by ds_read_b128.
-//  * The waves' accumulators meet in LDS at the end; wave i sums and stores
-//    the four result registers holding n = 8i + 4(l/32) + {0..3}.
+//    from the B rows (swz_sb), A^T fragments by ds_read_b128.
+//  * The waves' accumulators meet in LDS at the end; four waves sum and store
+//    the result registers holding n = 8i + 4(l/32) + {0..3}, i their number.
 // ---------------------------------------------------------------------------
-template <int MF, int NW, int NSL>
+template <int MF, int NC, int NW, int NSL>
 struct StreamCfg {
+  static constexpr int BN = 32 * NC;          // columns per workgroup
   static constexpr int A_B = 32 * MF * 128;  // 64 k of 32 MF rows
-  static constexpr int B_B = 64 * 64;         // 64 k-rows of 32 columns
+  static constexpr int B_B = 64 * BN * 2;     // 64 k-rows
   static constexpr int SLOT = A_B + B_B;
   static constexpr int A_L = A_B / 1024, B_L = B_B / 1024;
   static constexpr int VM = A_L + B_L;
   static constexpr int LDS = NW * NSL * SLOT;
-  static_assert(NW == 4, "one reducing wave per result register quad");
+  static_assert(NW == 4 || NW == 8, "waves");
+  static_assert(NC == 1 || NC == 2, "B row swizzle");
   static_assert(LDS <= 160 * 1024, "LDS");
   static_assert((NSL - 1) * VM < 64, "vmcnt range");
-  static_assert(NW * MF * 64 * 16 * 4 <= LDS, "reduction area");
+  static_assert(NW * MF * NC * 64 * 16 * 4 <= LDS, "reduction area");
 };
 __device__ __forceinline__ int swz_s(int m) { return (m >> 1) & 7; }
+// B rows of 128 bytes: a transposing read phase (4 consecutive k-rows x 64
+// bytes) spans the 256-byte bank window twice, so k-rows 2 and 3 swap their
+// halves; rows of 64 bytes fill it once.
+template <int NC>
+__device__ __forceinline__ int swz_sb(int k) {
+  return NC == 1 ? 0 : ((k >> 1) & 1) << 2;
+}
 // f(integral_constant<int, I>) for I = 0 .. N-1, in order.
 template <int N, int I = 0, typename F>
 __device__ __forceinline__ void unroll_n(F&& f) {
@@ -1021,21 +1034,24 @@ __device__ __forceinline__ void unroll_n(F&& f) {
   }
 }
 
-template <int MF, int NW, int NSL, bool TAIL>
+template <int MF, int NC, int NW, int NSL, bool TAIL>
 __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint16_t* __restrict__ A,
                                                                     const uint16_t* __restrict__ B,
                                                                     uint16_t* __restrict__ C, int M, int N, int K,
                                                                     int lda, int ldb, int ldc) {
-  using CF = StreamCfg<MF, NW, NSL>;
+  using CF = StreamCfg<MF, NC, NW, NSL>;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // Workgroup -> (32-column block, chunk of 32 MF rows), the row chunks of a
+  // Workgroup -> (BN-column block, chunk of 32 MF rows), the row chunks of a
   // column block adjacent, so one XCD holds whole column blocks and their
-  // neighbours (which share B's lines in L2).
+  // neighbours (which share B's lines in L2); with more rows than columns the
+  // column blocks of a row chunk, so the XCDs share out A instead.
   const int nmc = (M + 32 * MF - 1) / (32 * MF);
   const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
-  const int n0 = (wid / nmc) * 32, m0 = (wid % nmc) * 32 * MF;
+  const int ncb = (N + CF::BN - 1) / CF::BN;
+  const bool tall = M > N;
+  const int n0 = (tall ? wid % ncb : wid / nmc) * CF::BN, m0 = (tall ? wid / ncb : wid % nmc) * 32 * MF;
   A += (size_t)m0 * lda;
   C += (size_t)m0 * ldc;
   M -= m0;  // rows of this chunk (more than 32 MF only past the last row read)
@@ -1044,39 +1060,49 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
   const uint32_t ring = lds_addr(smem) + wave * NSL * CF::SLOT;
 
   // A load n: rows 8n + l/8, LDS chunk l%8 taking global chunk (l%8) ^
-  // swz(row) (rows past M re-read row M-1); B load n: k-rows 16n + l/4,
-  // chunk l%4 (columns past N re-read the last 8 valid ones; never stored).
+  // swz(row) (rows past M re-read row M-1); B load n: its BR k-rows' chunks in
+  // lane order, chunk c of k-row k at c ^ swz_sb(k) (columns past N re-read
+  // the last 8 valid ones; never stored).
   uint32_t a_off[CF::A_L];
 #pragma unroll
   for (int n = 0; n < CF::A_L; ++n) {
     const int row = 8 * n + (lane >> 3);
     a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_s(row));
   }
-  const uint32_t b_col_off = 2u * (min(n0 + 8 * (lane & 3), N - 8) - n0);
-  const uint32_t b_off = (uint32_t)(lane >> 2) * (uint32_t)ldb * 2u + b_col_off;  // from k-row 16 n
+  constexpr int CH = CF::BN / 8, BR = 64 / CH;  // 16-byte chunks per k-row, k-rows per load
+  const int b_row = lane / CH;                   // from k-row BR n; BR n has no part in swz_sb
+  const uint32_t b_col_off = 2u * (min(n0 + 8 * ((lane % CH) ^ swz_sb<NC>(b_row)), N - 8) - n0);
+  const uint32_t b_off = (uint32_t)b_row * (uint32_t)ldb * 2u + b_col_off;
   auto issue = [&](int i, auto slot_tag) {
     constexpr int I = decltype(slot_tag)::value;
     const int kb = cnt > 0 ? wave + NW * min(i, cnt - 1) : 0;
     const uint32_t st = ring + I * CF::SLOT;
 #pragma unroll
     for (int n = 0; n < CF::A_L; ++n) dma16(A + (size_t)kb * 64, a_off[n], st + n * 1024);
+    const uint16_t* bb = B + (size_t)kb * 64 * ldb + n0;
 #pragma unroll
-    for (int n = 0; n < CF::B_L; ++n) dma16(B + ((size_t)kb * 64 + 16 * n) * ldb + n0, b_off, st + CF::A_B + n * 1024);
+    for (int n = 0; n < CF::B_L; ++n) dma16(bb + (size_t)BR * ldb * n, b_off, st + CF::A_B + n * 1024);
   };
 
   // fragment lane addresses within a slot.  A^T (B operand): row am, chunk
   // 2 ks + g.  B^T (A operand): lane 16G + 4j + a reads k-row 8 (G>>1) +
-  // 4 r + j (+16 ks), columns 16 (G&1) + 4a .. +3.
+  // 4 r + j (+16 ks), columns 32 c + 16 (G&1) + 4a .. +3.
   const int am = lane & 31, g = lane >> 5;
   uint32_t a_col[4];
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) a_col[ks] = am * 128 + 16 * ((2 * ks + g) ^ swz_s(am));
   const int G = lane >> 4, bj = (lane >> 2) & 3, ba = lane & 3;
-  const uint32_t b_col = CF::A_B + (8 * (G >> 1) + bj) * 64 + 32 * (G & 1) + 8 * ba;
-
-  f32x16 acc[MF];
+  uint32_t b_col[NC];
 #pragma unroll
-  for (int f = 0; f < MF; ++f) acc[f] = f32x16{};
+  for (int c = 0; c < NC; ++c)
+    b_col[c] = CF::A_B + (8 * (G >> 1) + bj) * (2 * CF::BN) +
+               16 * ((4 * c + 2 * (G & 1) + (ba >> 1)) ^ swz_sb<NC>(bj)) + 8 * (ba & 1);
+
+  f32x16 acc[NC][MF];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int f = 0; f < MF; ++f) acc[c][f] = f32x16{};
 
   // the first kr k values of a slot count (64: all of them)
   auto compute = [&](auto slot_tag, int kr) {
@@ -1084,13 +1110,20 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     const uint32_t st = ring + I * CF::SLOT;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      const u32x2 lo = lds_read_tr16_at(st + b_col + 16 * ks * 64);
-      const u32x2 hi = lds_read_tr16_at(st + b_col + 16 * ks * 64 + 4 * 64);
       const bool keep = 16 * ks + 8 * g < kr;
-      const u32x4 bt = keep_if(keep, u32x4{lo[0], lo[1], hi[0], hi[1]});
+      u32x4 bt[NC];
 #pragma unroll
-      for (int f = 0; f < MF; ++f)
-        acc[f] = mfma32<BF16>(bt, keep_if(keep, lds_ld128(st + 32 * f * 128 + a_col[ks])), acc[f]);
+      for (int c = 0; c < NC; ++c) {
+        const u32x2 lo = lds_read_tr16_at(st + b_col[c] + 16 * ks * (2 * CF::BN));
+        const u32x2 hi = lds_read_tr16_at(st + b_col[c] + (16 * ks + 4) * (2 * CF::BN));
+        bt[c] = keep_if(keep, u32x4{lo[0], lo[1], hi[0], hi[1]});
+      }
+#pragma unroll
+      for (int f = 0; f < MF; ++f) {
+        const u32x4 at = keep_if(keep, lds_ld128(st + 32 * f * 128 + a_col[ks]));
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[c][f] = mfma32<BF16>(bt[c], at, acc[c][f]);
+      }
     }
   };
 
@@ -1109,9 +1142,9 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     }
 #pragma unroll
     for (int n = 0; n < CF::B_L; ++n) {
-      const int r0 = min(16 * n, kr - 1);
+      const int r0 = min(BR * n, kr - 1);
       dma16(B + ((size_t)kblocks * 64 + r0) * ldb + n0,
-            (uint32_t)(min(16 * n + (lane >> 2), kr - 1) - r0) * (uint32_t)ldb * 2u + b_col_off, st + CF::A_B + n * 1024);
+            (uint32_t)(min(BR * n + b_row, kr - 1) - r0) * (uint32_t)ldb * 2u + b_col_off, st + CF::A_B + n * 1024);
     }
   }
   unroll_n<NSL - 1>([&](auto i_tag) { issue(decltype(i_tag)::value, i_tag); });
@@ -1135,38 +1168,45 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
   });
   wait_vmcnt<0>();  // no DMA may land in the ring once it is reused below
 
-  // ---- accumulators meet in LDS: [wave][f][e][lane] floats ----
+  // ---- accumulators meet in LDS: [wave][c][f][e][lane] floats ----
   __syncthreads();
   float* red = reinterpret_cast<float*>(smem);
 #pragma unroll
-  for (int f = 0; f < MF; ++f)
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) red[((wave * MF + f) * 16 + e) * 64 + lane] = acc[f][e];
+    for (int f = 0; f < MF; ++f)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) red[(((wave * NC + c) * MF + f) * 16 + e) * 64 + lane] = acc[c][f][e];
   __syncthreads();
-  const int gn = n0 + 8 * wave + 4 * g;
+  // result quad 4 i .. 4 i + 3 of column fragment c to wave i (with 8 waves, i or i + 4)
 #pragma unroll
-  for (int f = 0; f < MF; ++f) {
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int c = 0; c < NC; ++c) {
+    if (wave / 4 != c % (NW / 4)) continue;
+    const int gn = n0 + 32 * c + 8 * (wave % 4) + 4 * g;
 #pragma unroll
-    for (int w = 0; w < NW; ++w)
+    for (int f = 0; f < MF; ++f) {
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] += red[((w * MF + f) * 16 + 4 * wave + j) * 64 + lane];
-    const int gm = 32 * f + am;
-    if (gm < M && gn < N)
-      st64(C + (size_t)gm * ldc + gn, u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
+      for (int w = 0; w < NW; ++w)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] += red[(((w * NC + c) * MF + f) * 16 + 4 * (wave % 4) + j) * 64 + lane];
+      const int gm = 32 * f + am;
+      if (gm < M && gn < N)
+        st64(C + (size_t)gm * ldc + gn, u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])});
+    }
   }
 }
 
-template <int MF, int NSL>
+template <int MF, int NC, int NW, int NSL>
 static int launch_stream(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
                          hipStream_t stream) {
-  using CF = StreamCfg<MF, 4, NSL>;
-  const long long grid = (long long)((N + 31) / 32) * ((M + 32 * MF - 1) / (32 * MF));
+  using CF = StreamCfg<MF, NC, NW, NSL>;
+  const long long grid = (long long)((N + CF::BN - 1) / CF::BN) * ((M + 32 * MF - 1) / (32 * MF));
   if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
   auto go = [&](auto tail) {
-    constexpr auto kern = gemm_bf16_stream_kernel<MF, 4, NSL, decltype(tail)::value>;
+    constexpr auto kern = gemm_bf16_stream_kernel<MF, NC, NW, NSL, decltype(tail)::value>;
     MX_RETURN_IF_HIP(lds_limit_once<kern>(CF::LDS));
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), CF::LDS, stream, (const uint16_t*)A,
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(64 * NW), CF::LDS, stream, (const uint16_t*)A,
                        (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc);
     MX_RETURN_IF_HIP(hipGetLastError());
     return MX_OK;
@@ -1178,24 +1218,31 @@ static int launch_stream(const void* A, const void* B, void* C, int M, int N, in
 // microseconds: fixed + rounds (round + step K/64) + fill (tiles / slots) K/64
 // with rounds = ceil(tiles / slots).  A round of workgroups costs its slowest
 // one (round, step), and more workgroups at once share the L2 and the clock
-// (fill).  Fitted (relative least squares, no negative term) to 228 random
+// (fill).  Fitted (relative least squares, no negative term) to 450 random
 // shapes, M 1..8192, N and K 512..8192, ragged and whole, each timed on every
-// kernel by graph replay; the kernel picked is on average 0.8% slower than
-// the fastest of the seven, at worst 26% (a single shape, 94x6904x6368).
-enum class Path { None, Stream32, Stream64, T64, T64x128, T128, T128x192, T256 };
+// kernel by graph replay; the kernel picked is on average about 1% slower than
+// the fastest.  The 64-column streams against the four-wave 32-column ones and
+// the tiles alone: 260x3008x6080 30.2 -> 21.8 us, 524x1536x8064 42 -> 27 (64
+// rows), 158x1664x6512 25.3 -> 20.4, 142x3032x2408 14.4 -> 12.6 (32 rows); below
+// 48 K blocks the 64-row one is 5-10% behind 64x64 tiles (763x1280x1024 8.55
+// against 7.91), which its min_k keeps.
+enum class Path { None, Stream32, Stream32x64, Stream64, Stream64x64, T64, T64x128, T128, T128x192, T256 };
 struct Kernel {
   Path path;
   int bm, bn, slots;  // tile, workgroups resident at once
   float fixed, round, step, fill;
+  int min_k;
 };
 constexpr Kernel kKernels[] = {
-    {Path::Stream32, 32, 32, 256, 1.393f, 1.922f, 0.097f, 0.064f},
-    {Path::Stream64, 64, 32, 256, 1.048f, 2.553f, 0.121f, 0.095f},
-    {Path::T64, 64, 64, 512, 2.301f, 1.117f, 0.184f, 0.298f},
-    {Path::T64x128, 64, 128, 256, 2.332f, 1.946f, 0.254f, 0.111f},
-    {Path::T128, 128, 128, 256, 1.749f, 2.956f, 0.353f, 0.187f},
-    {Path::T128x192, 128, 192, 256, 1.803f, 3.855f, 0.499f, 0.225f},
-    {Path::T256, 256, 256, 256, 2.082f, 6.139f, 0.977f, 0.532f},
+    {Path::Stream32, 32, 32, 256, 2.206f, 1.142f, 0.089f, 0.082f, 64},
+    {Path::Stream32x64, 32, 64, 256, 2.471f, 1.142f, 0.133f, 0.081f, 64},
+    {Path::Stream64, 64, 32, 256, 1.048f, 2.553f, 0.121f, 0.095f, 64},
+    {Path::Stream64x64, 64, 64, 256, 1.455f, 2.880f, 0.167f, 0.076f, 48 * 64},
+    {Path::T64, 64, 64, 512, 2.301f, 1.117f, 0.184f, 0.298f, 0},
+    {Path::T64x128, 64, 128, 256, 2.332f, 1.946f, 0.254f, 0.111f, 0},
+    {Path::T128, 128, 128, 256, 1.749f, 2.956f, 0.353f, 0.187f, 0},
+    {Path::T128x192, 128, 192, 256, 1.803f, 3.855f, 0.499f, 0.225f, 0},
+    {Path::T256, 256, 256, 256, 2.082f, 6.139f, 0.977f, 0.532f, 64},
 };
 
 // batch items of a strided-batched product (the tiled kernels only), or 0 for
@@ -1204,12 +1251,11 @@ static Path gemm_path(int M, int N, int K, int lda, int ldb, int batch) {
   Path best = Path::None;
   double least = 0;
   for (const Kernel& k : kKernels) {
-    const bool stream = k.bn == 32;
-    const bool plain = stream || k.path == Path::T256;  // no batch, and at least one whole 64-deep K block
-    if (plain && (K < 64 || batch > 0)) continue;
+    const bool stream = k.path < Path::T64;
+    if (K < k.min_k || (batch > 0 && (stream || k.path == Path::T256))) continue;
     // The lane offsets of the direct loads are 32-bit: bm rows of A, and the
-    // k-rows of B that share a base (16, 32 or 64), span less than 4 GiB.
-    const long long brows = stream ? 16 : k.path == Path::T256 ? 32 : K < 64 ? K : 64;
+    // k-rows of B that share a base (8 to 64), span less than 4 GiB.
+    const long long brows = stream ? 512 / k.bn : k.path == Path::T256 ? 32 : K < 64 ? K : 64;
     if ((long long)lda * 2 * k.bm > 0xffffffffLL || (long long)ldb * 2 * (brows - 1) + 2 * k.bn > 0xffffffffLL) continue;
     const double tiles = (double)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn) * (batch > 0 ? batch : 1);
     const double rounds = __builtin_ceil(tiles / k.slots), kb = K / 64.0;
@@ -1266,8 +1312,10 @@ extern "C" int mx_gemm_bf16(const void* A, const void* B, void* C, int M, int N,
   if (!strides_ok(M, N, K, lda, ldb)) return MX_ERR_SHAPE;
   const Path path = gemm_path(M, N, K, lda, ldb, 0);
   switch (path) {
-    case Path::Stream32: return launch_stream<1, 4>(A, B, C, M, N, K, lda, ldb, ldc, s);
-    case Path::Stream64: return launch_stream<2, 3>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::Stream32: return launch_stream<1, 1, 8, 2>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::Stream32x64: return launch_stream<1, 2, 4, 3>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::Stream64: return launch_stream<2, 1, 4, 3>(A, B, C, M, N, K, lda, ldb, ldc, s);
+    case Path::Stream64x64: return launch_stream<2, 2, 4, 2>(A, B, C, M, N, K, lda, ldb, ldc, s);
     case Path::T256: return launch_dma16s(A, B, C, M, N, K, lda, ldb, ldc, s);
     default: return launch_tiled(path, A, B, C, M, N, K, lda, ldb, ldc, s, 1, 0, 0, 0);
   }

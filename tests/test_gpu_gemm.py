@@ -288,13 +288,17 @@ def _check_elementwise(c, a, b):
     assert worst <= 1.0, f"{worst:.2f} times the bound"
 
 
-# every kernel of the dispatch: 32- and 64-row streams, 64x64, 64x128,
-# 128x128, 128x192 and 256x256 tiles, with K tails on both sides of 32, K
+# every kernel of the dispatch: streams of 32 and 64 rows and of 32 and 64
+# columns, 64x64, 64x128, 128x128, 128x192 and 256x256 tiles, with K tails on both sides of 32, K
 # below one 64-deep block, a single block, and edges off the tiles
 RAGGED_K = [(1, 8, 8), (16, 520, 72), (33, 264, 520), (1, 1024, 2056), (50, 5288, 2168), (100, 3200, 1800),
             (129, 200, 24), (300, 1104, 656), (129, 136, 40), (500, 1496, 1048), (1315, 840, 1128),
             (777, 3592, 200), (2000, 2040, 264), (554, 7384, 136), (607, 7040, 104), (3500, 1032, 16),
-            (1937, 7024, 104), (4000, 4040, 72), (4096, 4096, 152)]
+            (1937, 7024, 104), (4000, 4040, 72), (4096, 4096, 152),
+            # 64-column streams: 32 rows (K tails of 8, a last column block 8 wide, a last row of its own), 64
+            # rows (from K 3072; wide and tall)
+            (65, 4104, 200), (257, 1032, 1032), (130, 2056, 520), (500, 1032, 3080), (1000, 520, 3080),
+            (129, 4104, 3072), (3000, 264, 3136)]
 
 
 @pytest.mark.parametrize("mnk", RAGGED_K)
@@ -317,7 +321,8 @@ def test_any_k_on_every_kernel(ops, mnk):
     assert torch.equal(c, cw[:m, :n])
 
 
-@pytest.mark.parametrize("mnk", [(40, 600, 328), (300, 1104, 264), (700, 1400, 520), (2000, 2040, 264), (4000, 4040, 104)])
+@pytest.mark.parametrize("mnk", [(40, 600, 328), (300, 1104, 264), (130, 2056, 520), (500, 1032, 3080),
+                                 (700, 1400, 520), (2000, 2040, 264), (4000, 4040, 104)])
 def test_infinity_in_the_last_k_row(ops, mnk):
     """The K tail re-reads the last k-row for the missing ones: an infinity
     there counts once, against zeros it gives NaN only where A holds a zero."""
