@@ -996,7 +996,8 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
 //    clocks, 64 or 128 bytes alike), so 64 columns where they still fill the
 //    CUs; eight waves with rings of two slots keep as many loads in flight as
 //    four with four and reach each block sooner (16x7168x4096 15.3 -> 15.1 us,
-//    1x696x1520 6.2 -> 5.2, 27x512x1280 4.96 -> 4.61).
+//    1x696x1520 6.2 -> 5.2, 27x512x1280 4.96 -> 4.61; the other way at 5x712x6272,
+//    15.6 -> 15.9, which neither tiles nor K tells from the rest).
 //  * C^T = B^T . A^T on 32x32x16 MFMAs: B^T fragments by transposing reads
 //    from the B rows (swz_sb), A^T fragments by ds_read_b128.
 //  * The waves' accumulators meet in LDS at the end; four waves sum and store

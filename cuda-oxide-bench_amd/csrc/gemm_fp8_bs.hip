@@ -747,7 +747,9 @@ static int launch_smallm(const void* A, const float* sA, const void* B, const fl
 // waves, chosen by M and by rounds: 8% in geometric mean; 128x7168x2048 16.3 ->
 // 10.6 us, 256x4096x4096 26.1 -> 15.1 and 524x1536x8064 54 -> 23 (64x64
 // streams), 3072^3 44.8 -> 37.1 (192x256), 730x7120x2816 34.7 -> 29.0 (128x256),
-// 64x4096x7168 20.5 -> 18.5 (eight waves).  Not kept: 256x128 tiles, 32x64
+// 64x4096x7168 20.5 -> 18.5 (eight waves); a few near ties lose 1-4%
+// (4096x4096x128 11.8 -> 12.3, 1539x4992x2560 with the quantiser 33.9 -> 34.3).
+// Not kept: 256x128 tiles, 32x64
 // streams and 32x32 streams of four waves were the fastest by up to 6, 8 and
 // 1% for 2 to 5 shapes in 180, and without them the mean is the same.
 enum class Path { Stream32, Stream64, Stream64x64, T128, T128x256, T192x256, T256 };
