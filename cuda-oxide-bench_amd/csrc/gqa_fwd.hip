@@ -401,17 +401,21 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
           // sees no key of its group's first tile sees none of the later ones
           // either: its max stays 0, its sums 0.
           const float shift = !first ? fmaxf(mx, 0.f) : KSP > 1 && mx == -INFINITY ? 0.f : mx;
-          const float corr = __builtin_amdgcn_exp2f(-shift);
           m_run[qt] += shift;
-          l_run[qt] *= corr;
+          // nothing to rescale at the first tile, where a max below -128
+          // would make the factor infinite and 0 * inf a NaN
+          if (!first) {
+            const float corr = __builtin_amdgcn_exp2f(-shift);
+            l_run[qt] *= corr;
 #pragma unroll
-          for (int i = 0; i < DT; ++i) {
-            if constexpr (QT == 1) {
-              acc_o[qt][i] *= corr;
-            } else {
-              agpr_settle(acc_o[qt][i]);
-              scale_acc(acc_o[qt][i], corr);
-              agpr_settle(acc_o[qt][i]);  // before the next asm MFMA reads it
+            for (int i = 0; i < DT; ++i) {
+              if constexpr (QT == 1) {
+                acc_o[qt][i] *= corr;
+              } else {
+                agpr_settle(acc_o[qt][i]);
+                scale_acc(acc_o[qt][i], corr);
+                agpr_settle(acc_o[qt][i]);  // before the next asm MFMA reads it
+              }
             }
           }
 #pragma unroll

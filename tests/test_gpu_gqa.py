@@ -211,3 +211,54 @@ def test_key_groups(ops, case, dt, causal):
     err = (o.cpu().double() - ref).norm(dim=-1)
     mixed = torch.sqrt((p ** 2) @ (vd.norm(dim=-1, keepdim=True) ** 2)).squeeze(-1) + ref.norm(dim=-1)
     assert (err <= 12 * u * mixed).all(), (err / (u * mixed)).max()
+
+
+def _assert_rows(o, q, k, v, causal):
+    """Every output row within test_key_groups' bound of 64-bit attention."""
+    S, G = q.shape[2], q.shape[1] // k.shape[1]
+    kd, vd = (t.double().repeat_interleave(G, 1) for t in (k, v))
+    s = q.double() @ kd.transpose(-1, -2).contiguous() / q.shape[3] ** 0.5
+    if causal:
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool).triu(1), float("-inf"))
+    p = torch.softmax(s, dim=-1)
+    ref = p @ vd
+    u = 2.0 ** -9 if q.dtype == torch.bfloat16 else 2.0 ** -12
+    err = (o.double() - ref).norm(dim=-1)
+    mixed = torch.sqrt((p ** 2) @ (vd.norm(dim=-1, keepdim=True) ** 2)).squeeze(-1) + ref.norm(dim=-1)
+    assert (err <= 12 * u * mixed).all(), (err / (u * mixed)).max()
+
+
+# (S, Hq, Hkv, d_qk, d_v, tile): 4 and 2 key groups, one group, the explicit tiles of both kernels, MLA prefill
+FAR_BELOW = [(129, 8, 8, 64, 64, None), (193, 8, 2, 64, 64, None), (257, 8, 2, 64, 64, None),
+             (193, 8, 8, 128, 128, None), (321, 8, 2, 128, 128, None), (65, 8, 2, 128, 128, None),
+             (193, 8, 2, 64, 64, (256, 32)), (193, 8, 2, 128, 128, (256, 64)), (193, 8, 2, 64, 64, (128, 64)),
+             (193, 4, 4, 192, 128, None), (193, 4, 4, 96, 64, None)]
+
+
+@pytest.mark.parametrize("causal", [True, False], ids=["c", "n"])
+@pytest.mark.parametrize("low", ["last", "first tile", "tile starts", "all"])
+@pytest.mark.parametrize("case", FAR_BELOW, ids=lambda c: f"S{c[0]}H{c[1]}/{c[2]}D{c[3]}-{c[4]}{'t%d-%d' % c[5] if c[5] else ''}")
+def test_scores_far_below_the_rest(ops, case, low, causal):
+    """Keys that score 240 to 420 powers of two below the others, where a tile
+    of them is all that a row has met so far: the last key alone in a key
+    group's tile, the whole first tile, the first key of every tile (a causal
+    row's only key there), every key."""
+    S, Hq, Hkv, dqk, dv, tile = case
+    announce(f"gqa far below: {low} S{S} Hq{Hq} Hkv{Hkv} D{dqk}/{dv} tile={tile} causal={causal}")
+    g = torch.Generator().manual_seed(S + dqk)
+    dt = torch.bfloat16
+    q = torch.randn((1, Hq, S, dqk), generator=g).to(dt)
+    k = torch.randn((1, Hkv, S, dqk), generator=g).to(dt)
+    v = torch.randn((1, Hkv, S, dv), generator=g).to(dt)
+    rows = {"last": slice(S - 1, S), "first tile": slice(0, 64), "tile starts": slice(0, S, 64), "all": slice(0, S)}[low]
+    q[..., 0], k[..., 0] = 32.0, 0.0
+    k[:, :, rows, 0] = -72.0
+    args = [t.cuda() for t in (q, k, v)]
+    if dqk != dv:
+        o = ops.mla_prefill_fwd(*args, causal=causal)
+    elif tile is None:
+        o = ops.gqa_fwd(*args, causal=causal)
+    else:
+        o = ops.gqa_fwd(*args, causal=causal, block_m=tile[0], wave_m=tile[1])
+    torch.cuda.synchronize()
+    _assert_rows(o.cpu(), q, k, v, causal)
