@@ -49,6 +49,13 @@ static_assert(RING <= 160 * 1024 && NW * VT * 64 * 16 <= RING, "LDS");
 __device__ __forceinline__ int swz_l(int t) { return (t & 7) << 1; }
 __device__ __forceinline__ int swz_r(int t) { return (t >> 1) & 7; }
 
+// Byte offset, from the first row of the block at token tok0, of the last row
+// of it that the sequence has.  Counted in rows first: the rest of a sequence
+// of more than 3.7 million tokens is over 2^32 bytes.
+__host__ __device__ __forceinline__ uint32_t last_row(int T, int tok0) {
+  return (uint32_t)(T - tok0 < BT ? T - tok0 - 1 : BT - 1) * ROW_B;
+}
+
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4 mfma_k16(const u32x2& a, const u32x2& b, const f32x4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0,
@@ -84,7 +91,7 @@ __global__ __launch_bounds__(64 * NW, 1) void mla_decode_few_kernel(const uint16
   auto issue = [&](int i) {
     const int tok0 = t0 + (wave + NW * i) * BT;
     const unsigned char* base = kvb + (size_t)tok0 * ROW_B;
-    const uint32_t last = (uint32_t)(T - 1 - tok0) * ROW_B;  // offset of the sequence's last row
+    const uint32_t last = last_row(T, tok0);
     const uint32_t st = ring + (i & 1) * SLOT;
 #pragma unroll 1
     for (int h = 0; h < 2; ++h) {

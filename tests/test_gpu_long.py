@@ -104,3 +104,27 @@ def test_gemm_bf16_batched_many(ops):
     c = ops.gemm_bf16_batched(a.cuda(), b.cuda()).cpu()
     ref = torch.stack([torch.as_tensor(ogemm.gemm_ref(a[i], b[i])) for i in range(nb)])
     assert normwise_rel_err(c, ref) <= TOL
+
+
+@pytest.mark.parametrize("T,t0", [(3_728_300, 16), (3_900_000, 171_728)])
+def test_mla_few_heads_past_4_gib(ops, T, t0):
+    """A cache of more than 2^32 bytes per sequence, with up to 16 heads: the
+    attention sits on the block of 16 tokens that lies a little more than 2^32
+    bytes before the end.  The other tokens score 90 (natural units) below and
+    together weigh less than 2^-100."""
+    announce(f"long mla few heads T{T}, attention on tokens {t0}..{t0 + 15}")
+    g = torch.Generator(device="cuda").manual_seed(T)
+    kv = torch.randn((1, T, 576), generator=g, device="cuda", dtype=torch.bfloat16)
+    kv[0, :, 0] = 0
+    hot = kv[0, t0:t0 + 16]
+    hot[:, 0] = 8
+    hot[:, 1] = torch.linspace(-1, 1, 16)
+    q = torch.zeros((1, 4, 576), device="cuda", dtype=torch.bfloat16)
+    q[..., 0] = 12.5
+    q[0, :, 1] = torch.tensor([0.0, 1.0, -1.0, 0.5])
+    o = ops.mla_decode(q, kv, 1.0)
+    torch.cuda.synchronize()
+    p = torch.softmax(q[0].double() @ hot.double().t().contiguous(), dim=-1)
+    ref = p @ hot[:, :512].double()
+    # probabilities, partial result and output rounded to bf16, as in test_few_heads
+    assert ((o[0].double() - ref).norm() / ref.norm()).item() <= 3 * 2.0 ** -9
