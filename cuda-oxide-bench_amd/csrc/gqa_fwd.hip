@@ -274,6 +274,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
   // neg_m = -m_run instead of zero, so they return s - m_run directly.
   f32x16 acc_o[QT][DT];
   float m_run[QT], l_run[QT];
+  float lim[QT];  // a block max above this moves m_run: -inf while the row has met no key, then kLazy
   f32x16 neg_m[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -281,6 +282,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
     for (int i = 0; i < DT; ++i) acc_o[qt][i] = f32x16{};
     m_run[qt] = 0.f;
     l_run[qt] = 0.f;
+    lim[qt] = -INFINITY;
     neg_m[qt] = f32x16{};
   }
 
@@ -372,7 +374,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
       __builtin_amdgcn_s_setprio(0);
       // ---- mask, online softmax (lane-local + one lane^32 exchange) ----
       // s holds s - m_run (log2 units).  The running max is set from the
-      // first tile and afterwards only raised when some lane's block max
+      // first keys met and afterwards only raised when some lane's block max
       // exceeds it by more than 2^kLazy: below that, p = 2^(s - m_run)
       // stays <= 2^kLazy and neither O, l nor the scores are touched.  The
       // decision is a wave-wide vote.
@@ -395,17 +397,18 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[qt][t][e]);
         mx = max_xor32(mx);
-        const bool first = step == 0;  // every wave with a tile has one at step 0
-        if (first || __any(mx > kLazy)) {
-          // first tile: the max itself; later: only upward moves.  A row that
-          // sees no key of its group's first tile sees none of the later ones
-          // either: its max stays 0, its sums 0.
-          const float shift = !first ? fmaxf(mx, 0.f) : KSP > 1 && mx == -INFINITY ? 0.f : mx;
+        if (__any(mx > lim[qt])) {
+          // the first keys a row meets: their max itself; later: only upward
+          // moves.  Keys that are masked or score -inf are not met: the row
+          // stays empty (max and sums 0) until one is.
+          const bool empty = lim[qt] == -INFINITY, met = mx > -INFINITY;
+          const float shift = empty && met ? mx : fmaxf(mx, 0.f);
+          lim[qt] = met ? kLazy : lim[qt];
           m_run[qt] += shift;
-          // nothing to rescale at the first tile, where a max below -128
-          // would make the factor infinite and 0 * inf a NaN
-          if (!first) {
-            const float corr = __builtin_amdgcn_exp2f(-shift);
+          // An empty row has nothing to rescale: with a max below -128 the
+          // factor would be infinite and 0 * inf a NaN.
+          if (step > 0) {
+            const float corr = empty ? 1.f : __builtin_amdgcn_exp2f(-shift);
             l_run[qt] *= corr;
 #pragma unroll
             for (int i = 0; i < DT; ++i) {
@@ -517,7 +520,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
         const f32x16& a = acc_o[0][dt];
         red[(wv * NQ + 4 * dt + i) * 64 + lane] = f32x4{a[4 * i], a[4 * i + 1], a[4 * i + 2], a[4 * i + 3]};
       }
-    if (g == 0) ml[wv * 32 + ql] = float2{l_tot > 0.f ? m_run[0] : -INFINITY, l_tot};
+    if (g == 0) ml[wv * 32 + ql] = float2{l_tot == 0.f ? -INFINITY : m_run[0], l_tot};
     __syncthreads();
     float mx = -INFINITY, w[KSP], l = 0.f;
 #pragma unroll
@@ -525,10 +528,10 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 #pragma unroll
     for (int k = 0; k < KSP; ++k) {
       const float2 x = ml[(k * QS + wave) * 32 + ql];
-      w[k] = x.y > 0.f ? __builtin_amdgcn_exp2f(x.x - mx) : 0.f;
+      w[k] = __builtin_amdgcn_exp2f(x.x - mx);
       l += w[k] * x.y;
     }
-    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    const float inv = 1.0f / l;  // NaN for a row whose scores are all -inf, as softmax gives
     uint16_t* orow = O + (q_head + qrow[0]) * DV;
 #pragma unroll
     for (int u = 0; u < QPW; ++u) {
@@ -552,7 +555,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     const float l_tot = sum_xor32(l_run[qt]);
-    const float inv = (l_tot > 0.f) ? 1.0f / l_tot : 0.f;
+    const float inv = 1.0f / l_tot;  // inf, and 0 * inf = NaN, for a row whose scores are all -inf
     if (qrow[qt] < S) {
       uint16_t* orow = O + (q_head + qrow[qt]) * DV;
 #pragma unroll

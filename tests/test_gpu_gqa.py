@@ -262,3 +262,52 @@ def test_scores_far_below_the_rest(ops, case, low, causal):
         o = ops.gqa_fwd(*args, causal=causal, block_m=tile[0], wave_m=tile[1])
     torch.cuda.synchronize()
     _assert_rows(o.cpu(), q, k, v, causal)
+
+
+@pytest.mark.parametrize("causal", [True, False], ids=["c", "n"])
+@pytest.mark.parametrize("low", [0.0, -72.0], ids=["", "low"])
+@pytest.mark.parametrize("hidden", ["first tile", "all but last", "first half", "last half", "all"])
+@pytest.mark.parametrize("case", FAR_BELOW, ids=lambda c: f"S{c[0]}H{c[1]}/{c[2]}D{c[3]}-{c[4]}{'t%d-%d' % c[5] if c[5] else ''}")
+def test_scores_of_minus_infinity(ops, case, hidden, low, causal):
+    """Keys hidden by a component of -inf (q > 0 there): the same rows as
+    softmax, NaN where a row sees hidden keys only, whether or not the keys are
+    split between groups; with the visible keys at the others' level or 240 to
+    420 powers of two below zero."""
+    S, Hq, Hkv, dqk, dv, tile = case
+    announce(f"gqa -inf: {hidden} {low} S{S} Hq{Hq} Hkv{Hkv} D{dqk}/{dv} tile={tile} causal={causal}")
+    g = torch.Generator().manual_seed(S + dqk)
+    dt = torch.bfloat16
+    q = torch.randn((1, Hq, S, dqk), generator=g).to(dt)
+    k = torch.randn((1, Hkv, S, dqk), generator=g).to(dt)
+    v = torch.randn((1, Hkv, S, dv), generator=g).to(dt)
+    rows = {"first tile": slice(0, 64), "all but last": slice(0, S - 1), "first half": slice(0, S // 2),
+            "last half": slice(S // 2, S), "all": slice(0, S)}[hidden]
+    q[..., 0], k[..., 0] = 32.0, low
+    k[:, :, rows, 0] = float("-inf")
+    args = [t.cuda() for t in (q, k, v)]
+    if dqk != dv:
+        o = ops.mla_prefill_fwd(*args, causal=causal)
+    elif tile is None:
+        o = ops.gqa_fwd(*args, causal=causal)
+    else:
+        o = ops.gqa_fwd(*args, causal=causal, block_m=tile[0], wave_m=tile[1])
+    torch.cuda.synchronize()
+    o = o.cpu()
+    visible = torch.ones(S, dtype=torch.bool)
+    visible[rows] = False
+    seen = visible.cumsum(0) > 0 if causal else visible.any().expand(S)  # rows that see a key
+    assert torch.isnan(o[:, :, ~seen]).all()
+    # the rows that see a key, over the visible keys alone
+    S1, G = int(seen.sum()), Hq // Hkv
+    if S1 == 0:
+        return
+    kd, vd = (t.double().repeat_interleave(G, 1) for t in (k[:, :, visible], v[:, :, visible]))
+    s = q[:, :, seen].double() @ kd.transpose(-1, -2).contiguous() / dqk ** 0.5
+    if causal:
+        at = torch.arange(S)
+        s = s.masked_fill(at[visible][None, :] > at[seen][:, None], float("-inf"))
+    p = torch.softmax(s, dim=-1)
+    ref = p @ vd
+    err = (o[:, :, seen].double() - ref).norm(dim=-1)
+    mixed = torch.sqrt((p ** 2) @ (vd.norm(dim=-1, keepdim=True) ** 2)).squeeze(-1) + ref.norm(dim=-1)
+    assert (err <= 12 * 2.0 ** -9 * mixed).all(), (err / (2.0 ** -9 * mixed)).max()
