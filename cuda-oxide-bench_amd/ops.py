@@ -19,15 +19,15 @@ _IO_DTYPES = {torch.bfloat16: _lib.MX_DTYPE_BF16, torch.float16: _lib.MX_DTYPE_F
 
 
 _Tensor = torch.Tensor
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_current_device = torch._C._cuda_getDevice
+_C = torch._C
 
 
 # The checks below run on every call, several per call, and most launches take
 # a few microseconds: their common path is one expression each, and the stream
-# handle comes without building a torch.cuda.Stream (2.8 us).
+# handle comes without building a torch.cuda.Stream (2.8 us).  The device
+# bindings are looked up by the call: a CPU-only torch has none, and imports.
 def _stream() -> int:
-    return _raw_stream(_current_device())
+    return _C._cuda_getCurrentRawStream(_C._cuda_getDevice())
 
 
 def _require(t: torch.Tensor, name: str, dtypes, ndim: int | None = None) -> None:

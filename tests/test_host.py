@@ -101,3 +101,26 @@ def test_same_device_names_the_devices():
     ops._same_device(On(0), On(0), On(0))
     with pytest.raises(ValueError, match="cuda:0.*cuda:1"):
         ops._same_device(On(0), On(0), On(1))
+
+
+def test_operators_import_without_a_gpu_build_of_torch():
+    """The operator module imports where torch has no device bindings (a
+    CPU-only build); only a call needs them."""
+    import subprocess
+    import sys
+
+    from conftest import REPO_ROOT
+
+    code = (
+        "import importlib, torch\n"
+        "for name in [n for n in dir(torch._C) if n.startswith('_cuda_')]:\n"
+        "    delattr(torch._C, name)\n"
+        "ops = importlib.import_module('cuda-oxide-bench_amd.ops')\n"
+        "try:\n"
+        "    ops.gemm_bf16(torch.zeros(8, 8, dtype=torch.bfloat16), torch.zeros(8, 8, dtype=torch.bfloat16))\n"
+        "except ValueError as e:\n"
+        "    print(e)\n"
+    )
+    proc = subprocess.run([sys.executable, "-c", code], cwd=REPO_ROOT, capture_output=True, text=True, timeout=300)
+    assert proc.returncode == 0, proc.stderr
+    assert "must be on a HIP device" in proc.stdout
