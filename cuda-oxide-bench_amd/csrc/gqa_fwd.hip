@@ -274,7 +274,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
   // neg_m = -m_run instead of zero, so they return s - m_run directly.
   f32x16 acc_o[QT][DT];
   float m_run[QT], l_run[QT];
-  float lim[QT];  // a block max above this moves m_run: -inf while the row has met no key, then kLazy
+  bool open[QT];  // some row of the wave has met no key (uniform: a scalar)
   f32x16 neg_m[QT];
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
@@ -282,7 +282,7 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
     for (int i = 0; i < DT; ++i) acc_o[qt][i] = f32x16{};
     m_run[qt] = 0.f;
     l_run[qt] = 0.f;
-    lim[qt] = -INFINITY;
+    open[qt] = true;
     neg_m[qt] = f32x16{};
   }
 
@@ -397,13 +397,14 @@ __global__ __launch_bounds__(64 * NWAVES, QT == 1 ? 2 : 1) void gqa_fwd_kernel(c
 #pragma unroll
           for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[qt][t][e]);
         mx = max_xor32(mx);
-        if (__any(mx > lim[qt])) {
+        const bool moved = __any(mx > kLazy);
+        if (moved || open[qt]) {
           // the first keys a row meets: their max itself; later: only upward
           // moves.  Keys that are masked or score -inf are not met: the row
           // stays empty (max and sums 0) until one is.
-          const bool empty = lim[qt] == -INFINITY, met = mx > -INFINITY;
-          const float shift = empty && met ? mx : fmaxf(mx, 0.f);
-          lim[qt] = met ? kLazy : lim[qt];
+          const bool empty = open[qt] && sum_xor32(l_run[qt]) == 0.f, met = mx > -INFINITY;
+          const float shift = empty ? (met ? mx : 0.f) : moved ? fmaxf(mx, 0.f) : 0.f;
+          open[qt] = __any(empty && !met);
           m_run[qt] += shift;
           // An empty row has nothing to rescale: with a max below -128 the
           // factor would be infinite and 0 * inf a NaN.
