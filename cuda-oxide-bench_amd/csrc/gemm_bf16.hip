@@ -13,7 +13,8 @@
 // slot that the prologue leaves free.
 //
 // gemm_bf16_dma16s_kernel: 256x256 tiles, the large products.
-// gemm_bf16_dma64_kernel: tiles of 64x64 to 128x192, single and batched.
+// gemm_bf16_dma64_kernel: tiles of 64x64 to 128x192, single and batched;
+// gemm_bf16_short_kernel: the smaller ones for K < 128.
 // gemm_bf16_stream_kernel: few rows or few tiles; workgroups of 32 or 64
 // columns x 32 or 64 rows stream B, their waves splitting K.
 // gemm_bf16_smallm_kernel / gemm_bf16_smallm_sk_kernel (batched items of few
@@ -26,6 +27,24 @@ namespace mx {
 namespace gemm {
 
 constexpr int GROUP_M = 8;
+
+// First row and column of this workgroup's C tile: tiles grouped for L2 reuse
+// (GROUP_M tile rows share their columns of B), XCD-aware.
+struct Origin {
+  int m0, n0;
+};
+template <int BM, int BN>
+__device__ __forceinline__ Origin tile_origin(int M, int N) {
+  const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+  const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
+  const int per_group = GROUP_M * tiles_n;
+  const int group = id / per_group;
+  const int first_m = group * GROUP_M;
+  const int gsz = min(tiles_m - first_m, GROUP_M);
+  const int tm = first_m + (id % per_group) % gsz;
+  const int tn = (id % per_group) / gsz;
+  return Origin{tm * BM, tn * BN};
+}
 
 // The interface's bound on the leading dimensions of shapes with K % 32 != 0,
 // of small grids and of batched items with more than 32 rows: BM rows of A
@@ -43,6 +62,9 @@ template <int BK>
 __device__ __forceinline__ int swz_a(int m) {
   return BK == 64 ? ((m >> 1) & 7) : ((m >> 2) & 3);
 }
+
+// Below this K a tile takes the whole K to LDS at once (gemm_bf16_short_kernel).
+constexpr int kShortK = 128;
 
 // A fragment whose k values lie past K counts as zero on both sides, so
 // whatever was loaded in their place (an infinity too) adds nothing.
@@ -196,16 +218,8 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
   const int wm = wave / WN_, wn = wave % WN_;
   const int kg = lane >> 4;  // k-group of the lane's operand and row quad of its result
 
-  // ---- tile -> (tm, tn), grouped for L2 reuse, XCD-aware ----
-  const int tiles_m = (M + CF::BM - 1) / CF::BM, tiles_n = (N + CF::BN - 1) / CF::BN;
-  const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
-  const int per_group = GROUP_M * tiles_n;
-  const int group = id / per_group;
-  const int first_m = group * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int tm = first_m + (id % per_group) % gsz;
-  const int tn = (id % per_group) / gsz;
-  const int m0 = tm * CF::BM, n0 = tn * CF::BN;
+  const Origin org = tile_origin<CF::BM, CF::BN>(M, N);
+  const int m0 = org.m0, n0 = org.n0;
   const int nk = K / BK;
 
   // ---- direct loads: load ld = wave * LPW + n of a stage fills its bytes
@@ -339,15 +353,10 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
   }
   // Prologue: tiles 0 .. NS-2 in flight (tiles past the end re-load the
   // last one), wait for tile 0, read its fragments.
-  if (!TAIL || nk > 0) {
 #pragma unroll
-    for (int p = 0; p < NS - 1; ++p) issue(min(p, nk - 1), p);
-  }
+  for (int p = 0; p < NS - 1; ++p) issue(min(p, nk - 1), p);
   if constexpr (TAIL) {
-    if (nk > 0)
-      wait_vmcnt<(NS - 1) * CF::LPW>();
-    else
-      wait_vmcnt<0>();
+    wait_vmcnt<(NS - 1) * CF::LPW>();
     lds_barrier();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -365,21 +374,156 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage's reads are done before the next barrier frees it
   }
-  if (!TAIL || nk > 0) {
-    wait_vmcnt<(NS - 2) * CF::LPW>();
-    lds_barrier();
-    read_b(0, 0);
+  wait_vmcnt<(NS - 2) * CF::LPW>();
+  lds_barrier();
+  read_b(0, 0);
 #pragma unroll
-    for (int mf = 0; mf < FM; ++mf) read_a(0, 0, mf);
-    int kt = 0;
-    for (; kt + NS <= nk; kt += NS) step_period<NS>(step, kt);
-    step_tail<NS>(step, kt, nk - kt);
-  }
+  for (int mf = 0; mf < FM; ++mf) read_a(0, 0, mf);
+  int kt = 0;
+  for (; kt + NS <= nk; kt += NS) step_period<NS>(step, kt);
+  step_tail<NS>(step, kt, nk - kt);
   wait_vmcnt<0>();  // no DMA may land in LDS after the workgroup ends
 
   // ---- epilogue: lane holds m = am + 16 mf, n = wn*TN + 16 nf + 4 kg + {0..3}
   // of the tile ----
   store_tile_lds<CF::BM, CF::BN, CF::NT, FM, FN>(smem, acc, am, wn * CF::TN + 4 * kg, C, m0, n0, M, N, ldc);
+}
+
+// ---------------------------------------------------------------------------
+// gemm_bf16_short_kernel: the tiles of the kernel above for K < 128, which it
+// would spend in its prologue: its ring leaves room for one or two workgroups
+// per CU, and its constant waits load the last K tile again into every stage
+// that has none of its own.  Here the whole K goes to LDS at once (one wait,
+// one barrier, then fragments and MFMAs without another), only what the
+// product has of it (no k-rows past K, no rows past M in blocks of eight), in
+// one or two stages, so that the workgroups of a CU hide each other's loads
+// and stores.  What bounds it is the C tiles' way to memory, or a launch.
+// Ring -> this, same tile choice aside: 8192x8192x32 68.6 -> 23.8 us,
+// 16121x1672x8 32.1 -> 19, 170 items of 3x992x40 13.7 -> 8.6.  From K = 128 on
+// the ring is the faster one (64x64 tiles: by 8% at 128, 16% at 200 to 256).
+// ---------------------------------------------------------------------------
+template <int BM_, int BN_, int WM_, int WN_>
+__global__ __launch_bounds__(64 * WM_ * WN_) void gemm_bf16_short_kernel(
+    const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, uint16_t* __restrict__ C, int M, int N, int K,
+    int lda, int ldb, int ldc, long long sA, long long sB, long long sC) {
+  using CF = D64Cfg<BM_, BN_, WM_, WN_, 4>;
+  constexpr int FM = CF::FM, FN = CF::FN, BK = CF::BK;
+  extern __shared__ __align__(1024) unsigned char smem[];
+  A += (size_t)blockIdx.y * sA;
+  B += (size_t)blockIdx.y * sB;
+  C += (size_t)blockIdx.y * sC;
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN_, wn = wave % WN_;
+  const int kg = lane >> 4;
+  const Origin org = tile_origin<CF::BM, CF::BN>(M, N);
+  const int m0 = org.m0, n0 = org.n0;
+  const uint32_t lds0 = lds_addr(smem);
+
+  // ---- direct loads, laid out as in the kernel above.  Loads without a row of
+  // the product are left out: what LDS holds there reaches only results that
+  // are not stored, and k values that are set to zero. ----
+  for (int k0 = 0, st = lds0; k0 < K; k0 += BK, st += CF::STAGE) {
+    const int kr = min(K - k0, BK);
+    const uint16_t* abase = A + (size_t)m0 * lda + k0;
+    const uint16_t* bbase = B + (size_t)k0 * ldb + n0;
+#pragma unroll
+    for (int n = 0; n < CF::LPW; ++n) {
+      const int ld = wave * CF::LPW + n;
+      if (ld < CF::A_L) {
+        const int row = CF::A_RPL * ld + lane / 8;
+        const int chunk = min(8 * ((lane % 8) ^ swz_a16w(row)), kr - 8);  // elements
+        if (CF::A_RPL * ld < M - m0)
+          dma16(abase, (uint32_t)(min(m0 + row, M - 1) - m0) * (uint32_t)lda * 2u + 2u * chunk, st + ld * 1024);
+      } else {
+        const int byte = 1024 * (ld - CF::A_L) + 16 * lane;
+        const int row = byte / CF::RB;
+        const int col = 8 * (((byte % CF::RB) / 16) ^ swz_b16n<CF::BN>(row));
+        if (1024 * (ld - CF::A_L) / CF::RB < kr)
+          dma16(bbase, (uint32_t)min(row, kr - 1) * (uint32_t)ldb * 2u + 2u * (min(n0 + col, N - 8) - n0),
+                st + ld * 1024);
+      }
+    }
+  }
+
+  // Fragment lane addresses of the first half, as in the kernel above; the
+  // second half of a stage is 64 bytes (one bit) across in A and 32 k-rows on
+  // in B.
+  const int am = wm * CF::TM + (lane & 15);
+  uint32_t a_col = lds0 + am * CF::RA + 16 * (kg ^ swz_a16w(am));
+  const int b_j = (lane >> 2) & 3, b_a = lane & 3;
+  const int bk = 8 * kg + b_j;
+  uint32_t b_col[FN];
+#pragma unroll
+  for (int nf = 0; nf < FN; ++nf) {
+    const int chunk = (wn * CF::TN + 16 * nf + 4 * b_a) >> 3;
+    b_col[nf] = lds0 + CF::A_B + bk * CF::RB + 16 * (chunk ^ swz_b16n<CF::BN>(bk)) + 8 * (b_a & 1);
+  }
+
+  f32x4 acc[FM][FN];
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{};
+
+  land_args(C);
+  wait_vmcnt<0>();
+  lds_barrier();
+  // A loop and not unrolled further: the kernel's code is fetched anew for
+  // every short launch.
+#pragma unroll 1
+  for (int k0 = 0, so = 0; k0 < K; k0 += 32) {
+    const bool keep = k0 + 8 * kg < K;
+    u32x4 bf[FN], af[FM];
+#pragma unroll
+    for (int nf = 0; nf < FN; ++nf) {
+      const u32x2 lo = lds_read_tr16_at(b_col[nf] + so);
+      const u32x2 hi = lds_read_tr16_at(b_col[nf] + so + 4 * CF::RB);
+      bf[nf] = keep_if(keep, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    }
+#pragma unroll
+    for (int mf = 0; mf < FM; ++mf) af[mf] = keep_if(keep, lds_ld128(a_col + 16 * mf * CF::RA));
+#pragma unroll
+    for (int mf = 0; mf < FM; ++mf)
+#pragma unroll
+      for (int nf = 0; nf < FN; ++nf) acc[mf][nf] = mfma16<BF16>(bf[nf], af[mf], acc[mf][nf]);
+    const bool second = k0 & 32;
+    a_col = (a_col ^ 64) + (second ? CF::STAGE : 0);
+    so += second ? CF::STAGE - 32 * CF::RB : 32 * CF::RB;
+  }
+  // 64 rows per tile are taken for small grids, where the way of the C tile
+  // through LDS is latency (10 items of 62x8x40: 2.85 us, 3.0 through LDS).
+  if constexpr (BM_ == 64) {
+#pragma unroll
+    for (int mf = 0; mf < FM; ++mf) {
+      const int gm = m0 + am + 16 * mf;
+#pragma unroll
+      for (int nf = 0; nf < FN; ++nf) {
+        const int gn = n0 + wn * CF::TN + 16 * nf + 4 * kg;
+        const f32x4& a = acc[mf][nf];
+        if (gm < M && gn < N) st64(C + (size_t)gm * ldc + gn, u32x2{pack_bf16x2(a[0], a[1]), pack_bf16x2(a[2], a[3])});
+      }
+    }
+  } else {
+    store_tile_lds<CF::BM, CF::BN, CF::NT, FM, FN>(smem, acc, am, wn * CF::TN + 4 * kg, C, m0, n0, M, N, ldc);
+  }
+}
+
+template <int BM, int BN, int WM, int WN>
+static int launch_short(const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb, int ldc,
+                        hipStream_t stream, int batch, long long sA, long long sB, long long sC) {
+  using CF = D64Cfg<BM, BN, WM, WN, 4>;
+  const long long tiles = (long long)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
+  if (tiles > 0x7fffffffLL || batch > 65535) return MX_ERR_SHAPE;
+  constexpr auto kern = gemm_bf16_short_kernel<BM, BN, WM, WN>;
+  constexpr int c_tile = BM == 64 ? 0 : BM * (BN * 2 + 16), most = kShortK / CF::BK * CF::STAGE;
+  MX_RETURN_IF_HIP(lds_limit_once<kern>(most > c_tile ? most : c_tile));
+  const int stages = (K + CF::BK - 1) / CF::BK * CF::STAGE;
+  hipLaunchKernelGGL(kern, dim3((unsigned)tiles, (unsigned)batch), dim3(CF::NT), stages > c_tile ? stages : c_tile,
+                     stream, (const uint16_t*)A, (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
+  MX_RETURN_IF_HIP(hipGetLastError());
+  return MX_OK;
 }
 
 template <int BM, int BN, int WM, int WN, int NS>
@@ -466,16 +610,8 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   const int wm = wave / WN, wn = wave % WN;
   const int kg = lane >> 4;  // k-group of the lane's operand and row quad of its result
 
-  // ---- tile -> (tm, tn), grouped for L2 reuse, XCD-aware ----
-  const int tiles_m = (M + CF::BM - 1) / CF::BM, tiles_n = (N + CF::BN - 1) / CF::BN;
-  const int id = xcd_remap(blockIdx.x, tiles_m * tiles_n);
-  const int per_group = GROUP_M * tiles_n;
-  const int group = id / per_group;
-  const int first_m = group * GROUP_M;
-  const int gsz = min(tiles_m - first_m, GROUP_M);
-  const int tm = first_m + (id % per_group) % gsz;
-  const int tn = (id % per_group) / gsz;
-  const int m0 = tm * CF::BM, n0 = tn * CF::BN;
+  const Origin org = tile_origin<CF::BM, CF::BN>(M, N);
+  const int m0 = org.m0, n0 = org.n0;
   const int nka = K / CF::BKA, nk = 2 * nka;
 
   // ---- direct-load lane offsets (bytes from the tile's first element).
@@ -1246,31 +1382,71 @@ constexpr Kernel kKernels[] = {
     {Path::T256, 256, 256, 256, 2.082f, 6.139f, 0.977f, 0.532f, 64},
 };
 
+// The same below K = 128, where tiles take gemm_bf16_short_kernel: fixed +
+// first K/64 + round ceil(x) + (tile + fill K/64) x with x = tiles / 256, since
+// a CU holds several workgroups of these.  Fitted to 440 random shapes, single
+// and batched, M 1..20000, N 8..16384, K 8..120, operands cached and not; the
+// kernel picked is on average 0.4% slower than the fastest of all.  256x256
+// tiles are there for B strides whose 64 k-rows pass 4 GiB.
+struct ShortKernel {
+  Path path;
+  int bm, bn;
+  float fixed, first, round, tile, fill;
+  int min_k;
+};
+constexpr ShortKernel kShortKernels[] = {
+    {Path::T64, 64, 64, 2.316f, 0.502f, 0.070f, 0.531f, 0.184f, 0},
+    {Path::T64x128, 64, 128, 2.119f, 0.478f, 0.451f, 0.701f, 0.336f, 0},
+    {Path::T128, 128, 128, 2.392f, 0.648f, 0.624f, 0.811f, 0.517f, 0},
+    {Path::Stream32, 32, 32, 1.256f, 0.103f, 1.427f, 0.270f, 0.166f, 64},
+    {Path::T256, 256, 256, 0.0f, 1.490f, 5.060f, 7.154f, 0.0f, 64},
+};
+
 // batch items of a strided-batched product (the tiled kernels only), or 0 for
 // a single one.
 static Path gemm_path(int M, int N, int K, int lda, int ldb, int batch) {
   Path best = Path::None;
   double least = 0;
-  for (const Kernel& k : kKernels) {
+  auto consider = [&](const auto& k, auto&& cost) {
     const bool stream = k.path < Path::T64;
-    if (K < k.min_k || (batch > 0 && (stream || k.path == Path::T256))) continue;
+    if (K < k.min_k || (batch > 0 && (stream || k.path == Path::T256))) return;
     // The lane offsets of the direct loads are 32-bit: bm rows of A, and the
     // k-rows of B that share a base (8 to 64), span less than 4 GiB.
     const long long brows = stream ? 512 / k.bn : k.path == Path::T256 ? 32 : K < 64 ? K : 64;
-    if ((long long)lda * 2 * k.bm > 0xffffffffLL || (long long)ldb * 2 * (brows - 1) + 2 * k.bn > 0xffffffffLL) continue;
+    if ((long long)lda * 2 * k.bm > 0xffffffffLL || (long long)ldb * 2 * (brows - 1) + 2 * k.bn > 0xffffffffLL) return;
     const double tiles = (double)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn) * (batch > 0 ? batch : 1);
-    const double rounds = __builtin_ceil(tiles / k.slots), kb = K / 64.0;
-    const double t = k.fixed + rounds * (k.round + k.step * kb) + k.fill * kb * tiles / k.slots;
+    const double t = cost(k, tiles);
     if (best == Path::None || t < least) {
       best = k.path;
       least = t;
     }
+  };
+  const double kb = K / 64.0;
+  if (K < kShortK) {
+    for (const ShortKernel& k : kShortKernels)
+      consider(k, [&](const ShortKernel& c, double tiles) {
+        const double x = tiles / 256;
+        return c.fixed + c.first * kb + c.round * __builtin_ceil(x) + (c.tile + c.fill * kb) * x;
+      });
+  } else {
+    for (const Kernel& k : kKernels)
+      consider(k, [&](const Kernel& c, double tiles) {
+        return c.fixed + __builtin_ceil(tiles / c.slots) * (c.round + c.step * kb) + c.fill * kb * tiles / c.slots;
+      });
   }
   return best;
 }
 
 static int launch_tiled(Path path, const void* A, const void* B, void* C, int M, int N, int K, int lda, int ldb,
                         int ldc, hipStream_t s, int batch, long long sA, long long sB, long long sC) {
+  if (K < kShortK) {
+    switch (path) {
+      case Path::T64: return launch_short<64, 64, 2, 2>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+      case Path::T64x128: return launch_short<64, 128, 2, 4>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+      case Path::T128: return launch_short<128, 128, 2, 4>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
+      default: return MX_ERR_SHAPE;
+    }
+  }
   switch (path) {
     case Path::T64: return launch_dma64<64, 64, 2, 2, 4>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);
     case Path::T64x128: return launch_dma64<64, 128, 2, 4, 6>(A, B, C, M, N, K, lda, ldb, ldc, s, batch, sA, sB, sC);

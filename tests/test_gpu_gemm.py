@@ -321,8 +321,28 @@ def test_any_k_on_every_kernel(ops, mnk):
     assert torch.equal(c, cw[:m, :n])
 
 
+# K below 128, where tiles take the whole K to LDS at once, and the 32-row stream: every K chunk count up to
+# 32 and beside 64, one and two stages, blocks of eight rows without a row, edges on and off the tiles
+SHORT_K = [(1, 8, 8), (64, 64, 64), (65, 72, 120), (152, 392, 40), (7, 3984, 24), (63, 56, 32), (9, 136, 56), (130, 64, 16),
+           (816, 1360, 8), (1837, 600, 96), (508, 2720, 40), (797, 2072, 104), (530, 3216, 64), (2268, 1672, 120),
+           (3052, 2256, 32), (1215, 3840, 8), (1506, 2752, 48), (4096, 4096, 64), (12, 968, 88), (782, 128, 104)]
+
+
+@pytest.mark.parametrize("mnk", SHORT_K)
+def test_short_k(ops, mnk):
+    test_any_k_on_every_kernel(ops, mnk)
+
+
+@pytest.mark.parametrize("bmnk", [(1, 1, 8, 8), (3, 9, 64, 40), (7, 65, 72, 120), (57, 2, 392, 48), (24, 3, 912, 72),
+                                  (15, 244, 504, 32), (34, 273, 928, 8), (36, 228, 224, 104), (7, 554, 776, 120)])
+def test_batched_short_k(ops, bmnk):
+    """Batched items with K below 128: the 64x64, 64x128 and 128x128 tiles."""
+    test_batched_larger_items(ops, bmnk)
+
+
 @pytest.mark.parametrize("mnk", [(40, 600, 328), (300, 1104, 264), (130, 2056, 520), (500, 1032, 3080),
-                                 (700, 1400, 520), (2000, 2040, 264), (4000, 4040, 104)])
+                                 (700, 1400, 520), (2000, 2040, 264), (4000, 4040, 104), (130, 200, 40), (65, 72, 8),
+                                 (900, 1360, 24)])
 def test_infinity_in_the_last_k_row(ops, mnk):
     """The K tail re-reads the last k-row for the missing ones: an infinity
     there counts once, against zeros it gives NaN only where A holds a zero."""
