@@ -66,6 +66,18 @@ __device__ __forceinline__ int swz_a(int m) {
 // Below this K a tile takes the whole K to LDS at once (gemm_bf16_short_kernel).
 constexpr int kShortK = 128;
 
+// s_waitcnt for "at most min(MAXC, after) chunks of LPC loads in flight".
+template <int LPC, int MAXC>
+__device__ __forceinline__ void wait_chunks(int after) {
+  if constexpr (MAXC > 0) {
+    if (after < MAXC) {
+      wait_chunks<LPC, MAXC - 1>(after);
+      return;
+    }
+  }
+  wait_vmcnt<MAXC * LPC>();
+}
+
 // A fragment whose k values lie past K counts as zero on both sides, so
 // whatever was loaded in their place (an infinity too) adds nothing.
 __device__ __forceinline__ u32x4 keep_if(bool keep, const u32x4& x) { return keep ? x : u32x4{0, 0, 0, 0}; }
@@ -311,21 +323,19 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     __builtin_amdgcn_sched_barrier(0);
   };
 
-  // One K tile: the fragments of its first half are in af and bf[0].  Every
-  // step issues exactly one tile of loads (near the end the last tile again,
-  // into stages nobody reads), so the ring accounting is the same in every
-  // step.
+  // One K tile: the fragments of its first half are in af and bf[0].
   auto step = [&](int kt, auto stg_tag) {
     constexpr int STG = decltype(stg_tag)::value;
     constexpr int NXT = (STG + 1) % NS;
     half(0, STG, 1);
     // This wave's loads of tile kt+1 have landed (at most the NS-3 tiles
-    // issued after it are in flight): after the barrier tile kt+1 is
-    // readable, and stage (kt-1)%NS, whose last reads every wave waited for
-    // before its first half's MFMAs, takes tile kt+NS-1.
-    wait_vmcnt<(NS - 3) * CF::LPW>();
+    // issued after it, fewer near the end, are in flight): after the barrier
+    // tile kt+1 is readable, and stage (kt-1)%NS, whose last reads every wave
+    // waited for before its first half's MFMAs, takes tile kt+NS-1.  After
+    // the last tile the reads for a next one get stale fragments nobody uses.
+    wait_chunks<CF::LPW, NS - 3>(nk - 2 - kt);
     lds_barrier();
-    issue(min(kt + NS - 1, nk - 1), (STG + NS - 1) % NS);
+    if (kt + NS - 1 < nk) issue(kt + NS - 1, (STG + NS - 1) % NS);
     half(1, NXT, 0);
   };
 
@@ -351,12 +361,13 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
       }
     }
   }
-  // Prologue: tiles 0 .. NS-2 in flight (tiles past the end re-load the
-  // last one), wait for tile 0, read its fragments.
+  // Prologue: tiles 0 .. NS-2 in flight (two at least: K >= 128), wait for
+  // tile 0, read its fragments.
 #pragma unroll
-  for (int p = 0; p < NS - 1; ++p) issue(min(p, nk - 1), p);
+  for (int p = 0; p < NS - 1; ++p)
+    if (p < 2 || p < nk) issue(p, p);
   if constexpr (TAIL) {
-    wait_vmcnt<(NS - 1) * CF::LPW>();
+    wait_chunks<CF::LPW, NS - 1>(nk);
     lds_barrier();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -374,7 +385,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the stage's reads are done before the next barrier frees it
   }
-  wait_vmcnt<(NS - 2) * CF::LPW>();
+  wait_chunks<CF::LPW, NS - 2>(nk - 1);
   lds_barrier();
   read_b(0, 0);
 #pragma unroll
@@ -828,22 +839,6 @@ constexpr int SM_A_B = 32 * SM_BK * 2;  // 4 KB
 template <int NF>
 __device__ __forceinline__ int sm_swz(int k) {
   return NF == 1 ? 0 : (((k & 3) << 2) & (4 * NF - 1));
-}
-
-// s_waitcnt for "at most min(MAXC, after) chunks of LPC loads in flight".
-template <int LPC, int MAXC>
-__device__ __forceinline__ void wait_chunks(int after) {
-  if constexpr (MAXC >= 4) {
-    if (after >= 4) { wait_vmcnt<4 * LPC>(); return; }
-  }
-  if constexpr (MAXC >= 3) {
-    if (after == 3) { wait_vmcnt<3 * LPC>(); return; }
-  }
-  if constexpr (MAXC >= 2) {
-    if (after == 2) { wait_vmcnt<2 * LPC>(); return; }
-  }
-  if (after >= 1) { wait_vmcnt<LPC>(); return; }
-  wait_vmcnt<0>();
 }
 
 template <int NF>
