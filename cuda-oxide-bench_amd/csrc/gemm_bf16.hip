@@ -824,10 +824,11 @@ static int launch_dma16s(const void* A, const void* B, void* C, int M, int N, in
 // NS-stage ring, NS-1 chunks ahead (6 stages for narrow tiles, 4 at NF = 4:
 // 48-80 KB of LDS, two workgroups per CU).  A single wave needs no barrier: the ring stage
 // it overwrites was consumed by its own MFMAs, which waited for those
-// reads.  The row chunks and column tiles of an item run on one XCD, whose L2
-// then holds its A and B once (against plain order: 16 items of 32 x 128 x 512
-// 3.95 -> 3.44 us, 64 items 6.33 -> 4.31, 128 items of 32 x 512 x 128 7.23 ->
-// 6.87).  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
+// reads.  With items first in the grid (by_item) the row chunks and column tiles
+// of an item run on one XCD, whose L2 then holds its A and B once: 64 items of
+// 32 x 128 x 512 6.33 -> 4.31 us, items with three and more chunks of K 5%
+// faster; one or two chunks gain nothing and keep the column tiles first (182
+// items of 2 x 512 x 128 7.5 us against 8.8).  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
 // B rows (64 NF bytes) put chunk c of k-row k at c ^ (((k & 3) << 2) mod
 // (4 NF)) so the 4 consecutive k-rows of a transposing read phase occupy
 // distinct 64-byte quarters of the bank sweep (no swizzle needed at NF = 1,
@@ -841,12 +842,22 @@ __device__ __forceinline__ int sm_swz(int k) {
   return NF == 1 ? 0 : (((k & 3) << 2) & (4 * NF - 1));
 }
 
+// The tile of a workgroup: the grid's dimensions are the indices, since the
+// divisions of a flat one take 0.1 to 0.15 us of these 3 us launches.
+struct SmallTile {
+  int item, ct, mc;  // batch item, column tile, row chunk
+};
+__device__ __forceinline__ SmallTile small_tile(bool by_item) {
+  return by_item ? SmallTile{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z}
+                 : SmallTile{(int)blockIdx.y, (int)blockIdx.x, (int)blockIdx.z};
+}
+
 template <int NF>
 __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __restrict__ A,
                                                               const uint16_t* __restrict__ B,
-                                                              uint16_t* __restrict__ C, int M, int N, int K, int lda,
-                                                              int ldb, int ldc, long long sA, long long sB,
-                                                              long long sC) {
+                                                              uint16_t* __restrict__ C, int batch, int M, int N, int K,
+                                                              int lda, int ldb, int ldc, long long sA, long long sB,
+                                                              long long sC, bool by_item) {
   constexpr int TN = 32 * NF;                 // columns per workgroup
   constexpr int RB = TN * 2;                  // B row bytes in LDS
   constexpr int B_B = SM_BK * RB;             // B chunk bytes
@@ -859,11 +870,10 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
   __shared__ __align__(1024) unsigned char smem[SM_NS * STAGE];
   const int lane = threadIdx.x;
   const int g = lane >> 5;
-  const int tiles_n = (N + TN - 1) / TN;
-  const int nmc = (M + 31) / 32;  // row chunks; those of a column tile, then an item's tiles, on one XCD
-  const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
-  const int n0 = wid / nmc % tiles_n * TN, m0 = wid % nmc * 32;
-  const size_t item = wid / nmc / tiles_n;
+  const SmallTile t = small_tile(by_item);
+  const size_t item = t.item;
+  const int n0 = t.ct * TN, m0 = t.mc * 32;
+  if (t.item >= batch) return;
   A += item * sA + (size_t)m0 * lda;
   B += item * sB;
   C += item * sC + (size_t)m0 * ldc;
@@ -959,20 +969,19 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
 template <int NF, int KW>
 __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint16_t* __restrict__ A,
                                                                      const uint16_t* __restrict__ B,
-                                                                     uint16_t* __restrict__ C, int M, int N, int K,
-                                                                     int lda, int ldb, int ldc, long long sA,
-                                                                     long long sB, long long sC) {
+                                                                     uint16_t* __restrict__ C, int batch, int M, int N,
+                                                                     int K, int lda, int ldb, int ldc, long long sA,
+                                                                     long long sB, long long sC, bool by_item) {
   constexpr int TN = 32 * NF, RB = TN * 2, B_B = SM_BK * RB, STAGE = SM_A_B + B_B;
   constexpr int BL = B_B / 1024, BCH = RB / 16, BRPL = 1024 / RB;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5;
-  const int tiles_n = (N + TN - 1) / TN;
-  const int nmc = (M + 31) / 32;  // row chunks; those of a column tile, then an item's tiles, on one XCD
-  const int wid = xcd_remap(blockIdx.x, (int)gridDim.x);
-  const int n0 = wid / nmc % tiles_n * TN, m0 = wid % nmc * 32;
-  const size_t item = wid / nmc / tiles_n;
+  const SmallTile t = small_tile(by_item);
+  const size_t item = t.item;
+  const int n0 = t.ct * TN, m0 = t.mc * 32;
+  if (t.item >= batch) return;
   A += item * sA + (size_t)m0 * lda;
   B += item * sB;
   C += item * sC + (size_t)m0 * ldc;
@@ -1070,44 +1079,40 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
 
 static int launch_smallm(const void* A, const void* B, void* C, int batch, int M, int N, int K, int lda, int ldb,
                          int ldc, long long sA, long long sB, long long sC, hipStream_t stream) {
-  auto groups = [&](int tn) { return (long long)batch * ((M + 31) / 32) * ((N + tn - 1) / tn); };
+  const long long chunks = (M + 31) / 32;
+  auto groups = [&](int tn) { return batch * chunks * ((N + tn - 1) / tn); };
+  // Grid: items (rounded up to whole XCDs; the extra workgroups return at
+  // once), column tiles, row chunks; with by_item off, column tiles, items, row
+  // chunks.  One launch covers the 65535 column tiles of a grid's second dimension.
+  auto go = [&](auto kern, int threads, int smem, int tn, bool by_item) {
+    const int most = 65535 * tn;
+    for (long long n0 = 0; n0 < N; n0 += most) {
+      const int n = (int)(N - n0 < most ? N - n0 : most);
+      const unsigned nt = (unsigned)((n + tn - 1) / tn), nb = (unsigned)(batch + 7) / 8 * 8, nm = (unsigned)chunks;
+      hipLaunchKernelGGL(kern, by_item ? dim3(nb, nt, nm) : dim3(nt, (unsigned)batch, nm), dim3(threads), smem, stream,
+                         (const uint16_t*)A, (const uint16_t*)B + n0, (uint16_t*)C + n0, batch, M, n, K, lda, ldb, ldc,
+                         sA, sB, sC, by_item);
+      MX_RETURN_IF_HIP(hipGetLastError());
+    }
+    return MX_OK;
+  };
   // 4..12 chunks of K, split among 4 waves: one workgroup per 32 x 64 tile
   // when that still gives >= 256 workgroups (one per CU), else 32 x 32.
   const int nkc = K / SM_BK;
   if (nkc % 4 == 0 && nkc >= 4 && nkc <= 12) {
-    const int nfs = groups(64) >= 256 ? 2 : 1;
-    const long long gsk = groups(32 * nfs);
-    if (gsk > 0x7fffffffLL) return MX_ERR_SHAPE;
-    const int smem = nkc * (SM_A_B + SM_BK * 64 * nfs);
-    if (nfs == 2) {
-      constexpr auto kern = gemm_bf16_smallm_sk_kernel<2, 4>;
-      MX_RETURN_IF_HIP(lds_limit_once<kern>(12 * (SM_A_B + SM_BK * 128)));
-      hipLaunchKernelGGL(kern, dim3((unsigned)gsk), dim3(256), smem, stream, (const uint16_t*)A, (const uint16_t*)B,
-                         (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-    } else {
-      constexpr auto kern = gemm_bf16_smallm_sk_kernel<1, 4>;
-      MX_RETURN_IF_HIP(lds_limit_once<kern>(12 * (SM_A_B + SM_BK * 64)));
-      hipLaunchKernelGGL(kern, dim3((unsigned)gsk), dim3(256), smem, stream, (const uint16_t*)A, (const uint16_t*)B,
-                         (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-    }
-    MX_RETURN_IF_HIP(hipGetLastError());
-    return MX_OK;
+    auto split_k = [&](auto nf) {
+      constexpr int NF = decltype(nf)::value, STAGE = SM_A_B + SM_BK * 64 * NF;
+      constexpr auto kern = gemm_bf16_smallm_sk_kernel<NF, 4>;
+      MX_RETURN_IF_HIP(lds_limit_once<kern>(12 * STAGE));
+      return go(kern, 256, nkc * STAGE, 32 * NF, true);
+    };
+    return groups(64) >= 256 ? split_k(std::integral_constant<int, 2>{}) : split_k(std::integral_constant<int, 1>{});
   }
   // Widest column tile that still leaves >= 512 workgroups (two per CU).
-  const int nf = groups(128) >= 512 ? 4 : (groups(64) >= 512 ? 2 : 1);
-  const long long grid = groups(32 * nf);
-  if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
-  if (nf == 4)
-    hipLaunchKernelGGL(gemm_bf16_smallm_kernel<4>, dim3((unsigned)grid), dim3(64), 0, stream, (const uint16_t*)A,
-                       (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-  else if (nf == 2)
-    hipLaunchKernelGGL(gemm_bf16_smallm_kernel<2>, dim3((unsigned)grid), dim3(64), 0, stream, (const uint16_t*)A,
-                       (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-  else
-    hipLaunchKernelGGL(gemm_bf16_smallm_kernel<1>, dim3((unsigned)grid), dim3(64), 0, stream, (const uint16_t*)A,
-                       (const uint16_t*)B, (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC);
-  MX_RETURN_IF_HIP(hipGetLastError());
-  return MX_OK;
+  const bool by_item = nkc > 2;
+  if (groups(128) >= 512) return go(gemm_bf16_smallm_kernel<4>, 64, 0, 128, by_item);
+  if (groups(64) >= 512) return go(gemm_bf16_smallm_kernel<2>, 64, 0, 64, by_item);
+  return go(gemm_bf16_smallm_kernel<1>, 64, 0, 32, by_item);
 }
 
 
@@ -1502,19 +1507,20 @@ static bool batched_small(int M, int K, int lda, int ldb) {
   return M <= 32 && K % 64 == 0 && (long long)lda * 2 * 32 <= 0xffffffffLL && (long long)ldb * 2 * 64 <= 0xffffffffLL;
 }
 
-// More rows take the same kernels, 32 at a time, where that beats 64-row tiles
-// (graph replay; the up-projections of an MLA step with 48 rows per head):
-// K split among four waves while a workgroup per CU is enough (N 128, K 512: 16
-// items 4.62 -> 3.49 us, 64 items 5.39 -> 5.22, but 128 items 7.3 -> 9.1), and
-// one or two chunks of K, which need a single round trip, up to 64 rows (N 512,
-// K 128: 16 items 3.64 -> 3.40, 64 items 6.46 -> 5.85, 32 items 4.14 -> 4.19;
-// 96 rows of 64 items 7.0 -> 9.7).
+// More rows take the same kernels, 32 at a time, where that beats the tiles
+// (graph replay; 800 random items, contiguous and strided by head):  K split
+// among four waves while a workgroup per CU is enough (N 128, K 512: 16 items
+// of 48 rows 4.62 -> 3.49 us, 64 items 5.39 -> 5.22, but 128 items 7.3 -> 9.1),
+// and one or two chunks of K, which need a single round trip, while all
+// workgroups run at once (K 128: 14 items of 46 x 512 3.19 against 3.34 us with
+// tiles, 18 of 62 x 512 3.53 against 3.41, 75 of 38 x 512 8.1 against 5.4; K 64:
+// 51 of 55 x 88 2.73 against 3.26, 133 of 58 x 88 4.10 against 3.55).
 static bool batched_rows(int batch, int M, int N, int K, int lda, int ldb) {
   if (K % 64 || !strides_2g<64>(lda, ldb)) return false;
   const int nkc = K / SM_BK;
   const long long rows = (long long)batch * ((M + 31) / 32);
   if (nkc % 4 == 0 && nkc <= 12) return rows * ((N + 63) / 64) <= 256;
-  return nkc <= 2 && M <= 64 && rows * ((N + 31) / 32) <= 0x7fffffffLL;
+  return nkc <= 2 && rows * ((N + 31) / 32) <= 512;
 }
 
 // Every check mx_gemm_bf16_batched makes before it launches, the grid

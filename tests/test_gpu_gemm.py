@@ -363,7 +363,9 @@ def test_infinity_in_the_last_k_row(ops, mnk):
                                   # chunks of 32 rows: K split among the waves (last chunk 1 and 8 rows, ragged N,
                                   # the most groups and one item more), and one and two chunks of K
                                   (7, 65, 136, 768), (16, 200, 128, 512), (64, 64, 128, 256), (65, 64, 128, 256),
-                                  (16, 33, 512, 64), (37, 64, 264, 128), (128, 48, 512, 128), (3, 65, 72, 128)])
+                                  (16, 33, 512, 64), (37, 64, 264, 128), (128, 48, 512, 128), (3, 65, 72, 128),
+                                  # ... up to 512 workgroups of 32 x 32 at any M, and one item more
+                                  (32, 128, 128, 64), (33, 128, 128, 64), (9, 96, 520, 128), (5, 1000, 72, 128)])
 def test_batched_larger_items(ops, bmnk):
     """Batched items with more than 32 rows, or a K that is no whole number of
     64-deep chunks, run the tiled kernels over the batch, or the small-row
@@ -377,3 +379,23 @@ def test_batched_larger_items(ops, bmnk):
     torch.cuda.synchronize()
     for i in range(nb):
         _check_elementwise(c[i], a[i], b[i])
+
+
+@pytest.mark.parametrize("bmnk", [(1, 3, 65535 * 64 + 72, 256), (2, 2, 65535 * 128 + 8, 192)])
+def test_batched_more_column_tiles_than_a_grid_dimension(ops, bmnk):
+    """Small-row kernels whose grid has items first take the column tiles in
+    slices of 65535: every column is written, those around the seam and at both
+    ends are right."""
+    nb, m, n, k = bmnk
+    announce(f"gemm_bf16_batched {nb}x{m}x{n}x{k}")
+    g = torch.Generator(device="cuda").manual_seed(k)
+    a = (torch.rand((nb, m, k), generator=g, device="cuda") * 2 - 1).to(torch.bfloat16)
+    b = torch.empty((nb, k, n), dtype=torch.bfloat16, device="cuda").uniform_(-1, 1, generator=g)
+    c = torch.full((nb, m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    ops.gemm_bf16_batched(a, b, out=c)
+    torch.cuda.synchronize()
+    assert not torch.isnan(c).any()
+    seam = 65535 * (64 if k % 256 == 0 else 128)
+    for lo, hi in ((0, 512), (seam - 512, min(n, seam + 512)), (n - 512, n)):
+        for i in range(nb):
+            _check_elementwise(c[i, :, lo:hi], a[i], b[i, :, lo:hi])
