@@ -343,7 +343,8 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
   // The K % 64 tail is computed first, from stage NS-1, which the ring fills
   // only after step 0's barrier: its loads share the prologue's latency
   // instead of adding a round trip at the end.  Chunks and k-rows past K
-  // re-read the last valid ones.
+  // re-read the last valid ones or are left out, and so is the second half of
+  // the stage when K ends in the first.
   if constexpr (TAIL) {
     const int kr = K - nk * BK;
     const uint32_t st = lds0 + (NS - 1) * CF::STAGE;
@@ -357,7 +358,8 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
         dma16(abase, off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), st + ld * 1024);
       } else {
         const int row = (1024 * (ld - CF::A_L) + 16 * lane) / CF::RB;
-        dma16(bbase, off[n] - (uint32_t)(row - min(row, kr - 1)) * (uint32_t)ldb * 2u, st + ld * 1024);
+        if (1024 * (ld - CF::A_L) / CF::RB < kr)
+          dma16(bbase, off[n] - (uint32_t)(row - min(row, kr - 1)) * (uint32_t)ldb * 2u, st + ld * 1024);
       }
     }
   }
@@ -371,6 +373,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     lds_barrier();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (32 * h >= K - nk * BK) break;
       const bool keep = 32 * h + 8 * kg < K - nk * BK;
       read_b(NS - 1, h);
 #pragma unroll
@@ -746,14 +749,15 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
       dma16(abase, a_off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), lds0 + 2 * CF::A_B + (wave * CF::A_LPW + n) * 1024);
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < 2; ++h) {
+      if (32 * h >= kr) break;
 #pragma unroll
       for (int n = 0; n < CF::B_LPW; ++n) {
         const int row = CF::B_RPL * (wave * CF::B_LPW + n) + lane / CF::B_CH;
-        const int r0 = h && kr > 32 ? 32 : 0;  // first k-row of the half, if it has any
-        dma16(bbase + (size_t)r0 * ldb, b_off[n] - (uint32_t)(row - min(row, kr - 1 - r0)) * (uint32_t)ldb * 2u,
+        dma16(bbase + (size_t)32 * h * ldb, b_off[n] - (uint32_t)(row - min(row, kr - 1 - 32 * h)) * (uint32_t)ldb * 2u,
               lds0 + CF::B_OFF + (3 - h) * CF::B_B + (wave * CF::B_LPW + n) * 1024);
       }
+    }
   }
   // Prologue, in the order the waits need: A block 0, B stages 0 and 1,
   // A block 1, B stage 2; then tile 0's fragments.
@@ -768,6 +772,7 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
     lds_barrier();
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
+      if (32 * h >= kr) break;
       const bool keep = 32 * h + 8 * kg < kr;
       read_b(3 - h, h);
 #pragma unroll
@@ -1247,6 +1252,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     const uint32_t st = ring + I * CF::SLOT;
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
+      if (16 * ks >= kr) break;
       const bool keep = 16 * ks + 8 * g < kr;
       u32x4 bt[NC];
 #pragma unroll
@@ -1279,9 +1285,9 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     }
 #pragma unroll
     for (int n = 0; n < CF::B_L; ++n) {
-      const int r0 = min(BR * n, kr - 1);
-      dma16(B + ((size_t)kblocks * 64 + r0) * ldb + n0,
-            (uint32_t)(min(BR * n + b_row, kr - 1) - r0) * (uint32_t)ldb * 2u + b_col_off, st + CF::A_B + n * 1024);
+      if (BR * n >= kr) break;
+      dma16(B + ((size_t)kblocks * 64 + BR * n) * ldb + n0,
+            (uint32_t)min(b_row, kr - 1 - BR * n) * (uint32_t)ldb * 2u + b_col_off, st + CF::A_B + n * 1024);
     }
   }
   unroll_n<NSL - 1>([&](auto i_tag) { issue(decltype(i_tag)::value, i_tag); });
