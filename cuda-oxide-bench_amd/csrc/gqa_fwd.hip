@@ -660,8 +660,12 @@ static int dispatch_tile(const void* Q, const void* K, const void* V, void* O, i
 // The estimate, in units of a step with one group: a workgroup costs its steps
 // plus a start and end per query block, 256 run at once; single causal
 // workgroups, of all lengths, fill the CUs evenly after the first round.
-// Fitted to 70 random shapes timed with every ksp (graph replay, B 1..4, 8..32
-// heads, S 128..4200): the choice is on average 0.7% slower than the best.
+// Head dim 64 is fitted to 70 random shapes timed with every ksp (graph replay,
+// B 1..4, 8..32 heads, S 128..4200), head dim 128 to 120 with more heads and
+// shorter prompts (up to 64 x 96 heads, S 16..20000), where the first fit split
+// keys that fill the CUs unsplit (B10 with 64 heads, S99: 24.4 us with one group,
+// 29.1 with two).  The choice is on average 0.8% slower than the best; B39 with
+// 4 heads, S288, takes 27.5 us in two groups against 24.6.
 struct Split {
   int ksp, hpw;
   bool pairs;
@@ -673,7 +677,7 @@ static Split pick_split(int B, int Hq, int Hkv, int S, int causal) {
     double step, ends, fixed;
   };
   static constexpr Cost k64[] = {{1, 1.0, 4.0, 0.0}, {2, 1.08, 4.5, 1.0}, {4, 1.3, 3.5, 1.0}};
-  static constexpr Cost k128[] = {{1, 1.4, 4.0, 0.0}, {2, 1.6, 4.0, 0.5}};
+  static constexpr Cost k128[] = {{1, 1.4, 5.75, 0.0}, {2, 1.72, 5.4, 0.15}};
   const Cost* cost = DQK == 64 ? k64 : k128;
   const int choices = DQK != DV ? 1 : DQK == 64 ? 3 : 2;
   const int G = Hq / Hkv;
