@@ -1082,10 +1082,19 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
   }
 }
 
+// Batched items of few rows: four to twelve 64-deep chunks of K are split among
+// four waves, one workgroup per 32 x 64 tile when that still gives >= 256
+// workgroups (one per CU), else 32 x 32; other K run one wave per tile, the
+// widest that still leaves >= 512 workgroups (two per CU).
+static bool small_split_k(int K) { return K / SM_BK % 4 == 0 && K / SM_BK <= 12; }
+static int small_width(int batch, int M, int N, int K) {  // 32-column fragments of a tile
+  auto groups = [&](int tn) { return (long long)batch * ((M + 31) / 32) * ((N + tn - 1) / tn); };
+  if (small_split_k(K)) return groups(64) >= 256 ? 2 : 1;
+  return groups(128) >= 512 ? 4 : groups(64) >= 512 ? 2 : 1;
+}
+
 static int launch_smallm(const void* A, const void* B, void* C, int batch, int M, int N, int K, int lda, int ldb,
                          int ldc, long long sA, long long sB, long long sC, hipStream_t stream) {
-  const long long chunks = (M + 31) / 32;
-  auto groups = [&](int tn) { return batch * chunks * ((N + tn - 1) / tn); };
   // Grid: items (rounded up to whole XCDs; the extra workgroups return at
   // once), column tiles, row chunks; with by_item off, column tiles, items, row
   // chunks.  One launch covers the 65535 column tiles of a grid's second dimension.
@@ -1093,7 +1102,8 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
     const int most = 65535 * tn;
     for (long long n0 = 0; n0 < N; n0 += most) {
       const int n = (int)(N - n0 < most ? N - n0 : most);
-      const unsigned nt = (unsigned)((n + tn - 1) / tn), nb = (unsigned)(batch + 7) / 8 * 8, nm = (unsigned)chunks;
+      const unsigned nt = (unsigned)((n + tn - 1) / tn), nb = (unsigned)(batch + 7) / 8 * 8,
+                     nm = (unsigned)((M + 31) / 32);
       hipLaunchKernelGGL(kern, by_item ? dim3(nb, nt, nm) : dim3(nt, (unsigned)batch, nm), dim3(threads), smem, stream,
                          (const uint16_t*)A, (const uint16_t*)B + n0, (uint16_t*)C + n0, batch, M, n, K, lda, ldb, ldc,
                          sA, sB, sC, by_item);
@@ -1101,22 +1111,19 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
     }
     return MX_OK;
   };
-  // 4..12 chunks of K, split among 4 waves: one workgroup per 32 x 64 tile
-  // when that still gives >= 256 workgroups (one per CU), else 32 x 32.
-  const int nkc = K / SM_BK;
-  if (nkc % 4 == 0 && nkc >= 4 && nkc <= 12) {
-    auto split_k = [&](auto nf) {
-      constexpr int NF = decltype(nf)::value, STAGE = SM_A_B + SM_BK * 64 * NF;
+  const int nkc = K / SM_BK, nf = small_width(batch, M, N, K);
+  if (small_split_k(K)) {
+    auto split_k = [&](auto nf_tag) {
+      constexpr int NF = decltype(nf_tag)::value, STAGE = SM_A_B + SM_BK * 64 * NF;
       constexpr auto kern = gemm_bf16_smallm_sk_kernel<NF, 4>;
       MX_RETURN_IF_HIP(lds_limit_once<kern>(12 * STAGE));
       return go(kern, 256, nkc * STAGE, 32 * NF, true);
     };
-    return groups(64) >= 256 ? split_k(std::integral_constant<int, 2>{}) : split_k(std::integral_constant<int, 1>{});
+    return nf == 2 ? split_k(std::integral_constant<int, 2>{}) : split_k(std::integral_constant<int, 1>{});
   }
-  // Widest column tile that still leaves >= 512 workgroups (two per CU).
   const bool by_item = nkc > 2;
-  if (groups(128) >= 512) return go(gemm_bf16_smallm_kernel<4>, 64, 0, 128, by_item);
-  if (groups(64) >= 512) return go(gemm_bf16_smallm_kernel<2>, 64, 0, 64, by_item);
+  if (nf == 4) return go(gemm_bf16_smallm_kernel<4>, 64, 0, 128, by_item);
+  if (nf == 2) return go(gemm_bf16_smallm_kernel<2>, 64, 0, 64, by_item);
   return go(gemm_bf16_smallm_kernel<1>, 64, 0, 32, by_item);
 }
 

@@ -58,7 +58,7 @@ P = ctypes.c_void_p(0x10000)  # never dereferenced: every call below fails valid
     ((P, P, P, 64, 64, 60, 60, 64, 64, None), _lib.MX_ERR_ALIGN),
     ((P, P, P, 64, 64, 64, 32, 64, 64, None), _lib.MX_ERR_SHAPE),
     ((ctypes.c_void_p(0x10008), P, P, 64, 64, 64, 64, 64, 64, None), _lib.MX_ERR_ALIGN),
-    # register-staged kernel: 64 rows of A at this stride pass its 2^31-byte buffer range
+    # 64 rows of A at this stride pass the 2^31 bytes that the interface takes for such a shape
     ((P, P, P, 64, 64, 64, 20971520, 64, 64, None), _lib.MX_ERR_SHAPE),
 ])
 def test_gemm_bf16_validation(args, code):

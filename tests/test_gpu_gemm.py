@@ -47,23 +47,21 @@ def test_parity_vs_oracle(ops, mnk):
     assert torch.all((c.float() - ref).abs() <= 0.2 + 0.05 * ref.abs())
 
 
-@pytest.mark.parametrize("mnk,path", [((64, 64, 4096), "one tile: weight streaming"),
-                                      ((256, 1024, 2048), "64 tiles: weight streaming"),
-                                      ((1024, 1024, 1024), "direct-load ring, 256 tiles (BASELINE configs[0])"),
-                                      ((1024, 1024, 576), "K % 128 != 0: register-staged split-K path"),
-                                      ((960, 1024, 512), "M % 64 == 0, 240 tiles: direct-load ring"),
-                                      ((1024, 1024, 512), "direct-load ring, 4 K tiles per group"),
-                                      ((768, 1024, 640), "direct-load ring, 5 K tiles per group, 192 tiles"),
-                                      ((1024, 960, 768), "direct-load ring, 6 K tiles per group, 240 tiles"),
-                                      ((512, 2048, 896), "direct-load ring, 7 K tiles per group"),
-                                      ((1024, 1024, 1536), "direct-load ring, 12 K tiles per group"),
-                                      ((512, 1024, 4096), "128 tiles, long K: direct-load ring")])
+@pytest.mark.parametrize("mnk,path", [((64, 64, 4096), "32-column streams"),
+                                      ((256, 1024, 2048), "32-column streams"),
+                                      ((1024, 1024, 1024), "256 tiles, 16 K tiles"),
+                                      ((1024, 1024, 576), "9 K tiles"),
+                                      ((960, 1024, 512), "240 tiles, 8 K tiles"),
+                                      ((1024, 1024, 512), "256 tiles, 8 K tiles"),
+                                      ((768, 1024, 640), "192 tiles, 10 K tiles"),
+                                      ((1024, 960, 768), "240 tiles, 12 K tiles"),
+                                      ((512, 2048, 896), "256 tiles, 14 K tiles"),
+                                      ((1024, 1024, 1536), "256 tiles, 24 K tiles"),
+                                      ((512, 1024, 4096), "64-column streams")])
 def test_small_grid_paths(ops, mnk, path):
-    """Grids of at most one 64x64 tile per CU with K >= 512: at most 64
-    tiles stream the weights; more, with whole tiles and 128-deep K chunks,
-    run the direct-load ring (two K groups per workgroup summed through
-    LDS; K tiles per group from fewer than the ring's 4 slots in flight to
-    many more), other shapes the register-staged split-K kernel."""
+    """Grids of at most one 64x64 tile per CU with K >= 512: streams of B for
+    the fewest tiles, else 64x64 tiles through a ring of four K tiles, with
+    K tile counts around whole periods of the ring."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} ({path})")
     a, b = inputs.gemm_inputs(shapes.GemmShape("t", m, n, k))
@@ -77,8 +75,7 @@ def test_small_grid_paths(ops, mnk, path):
 @pytest.mark.parametrize("mnk", [(1024, 1024, 1024), (768, 1024, 640), (1024, 1024, 1536)])
 def test_small_grid_strided(ops, mnk):
     """Leading dimensions beyond the row lengths (lda > K, ldb > N,
-    ldc > N) on the direct-load ring; C's padding columns are left
-    untouched."""
+    ldc > N) on 64x64 tiles; C's padding columns are left untouched."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} strided")
     lib = import_submodule("_lib")
@@ -141,10 +138,10 @@ def test_kat_pattern(ops):
 @pytest.mark.parametrize("mnk", [(4096, 4096, 32), (4096, 4096, 96), (4000, 4040, 4128), (4096, 4352, 2048),
                                  (4096, 4096, 64), (4096, 4096, 192), (4000, 4040, 4096), (4096, 4096, 1600)])
 def test_direct_load_path(ops, mnk):
-    """Shapes that take the large-problem kernels (>= 256 tiles of 256x256):
-    with K % 64 == 0 the split-ring kernel (whole 128-byte A lines), else
-    the single ring (K % 32 == 0).  A single K tile or A block, fewer K
-    tiles than ring slots, ragged M and N, and K-tile counts that are not a
+    """About one 256x256 tile per CU and more: 256x256 tiles (A and B rings of
+    their own) from K 192 on, 128x192 where their rounds fill the CUs better,
+    128x128 with the whole K at once below K 128.  Fewer K tiles than ring
+    slots, a K tail of 32, ragged M and N, and K-tile counts that are no
     multiple of either ring's period."""
     m, n, k = mnk
     announce(f"gemm_bf16 direct-load {m}x{n}x{k}")
@@ -176,14 +173,13 @@ def test_target_size_sampled(ops):
 @pytest.mark.parametrize("mnk,path", [((2048, 2048, 2048), "128x128 tiles, 64 K tiles"),
                                       ((2000, 2040, 2048), "ragged M and N"),
                                       ((2560, 2560, 1024), "400 tiles: two rounds of workgroups"),
-                                      ((2048, 2048, 32), "one K tile, fewer than the ring's stages"),
-                                      ((2048, 2048, 160), "five K tiles: only the loop tail"),
-                                      ((2048, 4096, 1056), "33 K tiles: five ring periods and a tail of three"),
+                                      ((2048, 2048, 32), "half a K tile, the whole K at once"),
+                                      ((2048, 2048, 160), "two K tiles and a tail of 32, fewer than the ring's stages"),
+                                      ((2048, 4096, 1056), "16 K tiles and a tail of 32: three ring periods and one"),
                                       ((4080, 2056, 256), "ragged, 544 tiles")])
 def test_direct_load_128_paths(ops, mnk, path):
-    """Mid-size GEMMs (at least one 128x128 tile per CU, fewer than one
-    256x256 tile per CU, K % 32 == 0) run the direct-load 16x16x32 kernel on
-    128x128 tiles with a 6-stage ring.  2048^3 is a size of the reference's
+    """Mid-size GEMMs: 128x128 tiles through a ring of five K tiles, or the
+    whole K at once (K 32); 256x256 tiles for the last shape.  2048^3 is a size of the reference's
     mixed-dtype harness sweep (cutile-matmul-tiled-mixed/main.py:60)."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} direct-load 128x128 ({path})")
@@ -199,12 +195,10 @@ def test_direct_load_128_paths(ops, mnk, path):
                                  (7, 296, 640), (48, 3000, 1344), (256, 512, 4096), (130, 1024, 2048),
                                  (1000, 96, 1024), (2048, 128, 4096), (96, 512, 8192)])
 def test_weight_streaming_small_m(ops, mnk):
-    """M <= 64 against at least 256 columns, or at most 64 tiles of 64x64
-    with K >= 512, with whole 64-deep K blocks runs the weight-streaming
-    kernel: single rows, one K block (fewer than the waves), the
-    two-fragment variant (M > 32) and its chunks of 64 rows (a last chunk of
-    2 or 40 rows), a last column block 8 or 24 wide, block counts that do
-    not divide by the wave count."""
+    """Few rows or few tiles run the streams of B, here the 32x32 one: single
+    rows, one K block (fewer than the waves), a last chunk of 1, 2 or 8 rows, a
+    last column block 8 or 24 wide, block counts that do not divide by the
+    wave count, more rows than columns."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} weight streaming")
     a, b = inputs.gemm_inputs(shapes.GemmShape("t", m, n, k))
@@ -219,9 +213,8 @@ def test_weight_streaming_small_m(ops, mnk):
                                       ((3000, 3064, 512), "ragged, 144 tiles"),
                                       ((3584, 3584, 2048), "196 tiles against 784")])
 def test_direct_load_256_below_one_tile_per_cu(ops, mnk, path):
-    """Fewer than one 256x256 tile per CU still runs the 256x256 direct-load
-    kernel when 128x128 tiles would need more than 2.6 times the rounds of
-    workgroups."""
+    """Fewer than one 256x256 tile per CU still runs 256x256 tiles where the
+    rounds of 128x128 ones would cost more."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} direct-load 256x256 ({path})")
     a, b = inputs.gemm_inputs(shapes.GemmShape("t", m, n, k))
@@ -232,12 +225,11 @@ def test_direct_load_256_below_one_tile_per_cu(ops, mnk, path):
     assert torch.all((c.float() - ref).abs() <= 0.2 + 0.05 * ref.abs())
 
 
-@pytest.mark.parametrize("mnk,path", [((2048, 2048, 2056), "register-staged 128x128 (tiles128 >= 256, K % 32 != 0)"),
-                                      ((4096, 8192, 264), "register-staged 256x256 (tiles256 >= 512, K % 32 != 0)"),
-                                      ((2048, 2048, 72), "register-staged 128x128, K tail of 8")])
-def test_register_staged_paths(ops, mnk, path):
-    """Single GEMMs whose K is not a multiple of 32 land on the
-    register-staged 128x128 and 256x256 kernels (zero-filled K tail)."""
+@pytest.mark.parametrize("mnk,path", [((2048, 2048, 2056), "128x128 tiles, K tail of 8"),
+                                      ((4096, 8192, 264), "256x256 tiles, K tail of 8"),
+                                      ((2048, 2048, 72), "128x128 tiles, whole K at once")])
+def test_k_tail_of_eight(ops, mnk, path):
+    """Large products whose K is 8 past a multiple of 64."""
     m, n, k = mnk
     announce(f"gemm_bf16 {m}x{n}x{k} {path}")
     a, b = inputs.gemm_inputs(shapes.GemmShape("t", m, n, k))
@@ -257,13 +249,13 @@ def test_rejects_bad_arguments(ops):
 
 @pytest.mark.parametrize("bmnk", [(1, 64, 64, 64), (7, 100, 136, 72), (128, 32, 512, 128), (128, 32, 128, 512), (16, 5, 40, 192),
                                   (3, 300, 264, 520), (4, 1024, 1024, 256),
-                                  # split-K small-M kernel: 4, 8 and 12 chunks of K, 32 x 64 and 32 x 32
+                                  # K split among the waves: 4, 8 and 12 chunks of K, 32 x 64 and 32 x 32
                                   # tiles, ragged M and N
                                   (8, 17, 72, 256), (64, 32, 136, 768), (200, 32, 128, 512), (3, 1, 8, 512)])
 def test_batched_vs_oracle(ops, bmnk):
-    """Strided-batched GEMM: every item against the fp32 oracle (small-M,
-    its split-K variant for 4..12 chunks of K, 64x64 and, at 4 x
-    1024x1024x256, the 128x128 register-staged kernel)."""
+    """Strided-batched GEMM: every item against the fp32 oracle (small-row
+    kernels with and without K split among the waves, 64x64 tiles and, at 4 x
+    1024x1024x256, 128x128 ones)."""
     nb, m, n, k = bmnk
     announce(f"gemm_bf16_batched {nb}x{m}x{n}x{k}")
     g = torch.Generator().manual_seed(nb * 131 + m)
@@ -298,7 +290,11 @@ RAGGED_K = [(1, 8, 8), (16, 520, 72), (33, 264, 520), (1, 1024, 2056), (50, 5288
             # 64-column streams: 32 rows (K tails of 8, a last column block 8 wide, a last row of its own), 64
             # rows (from K 3072; wide and tall)
             (65, 4104, 200), (257, 1032, 1032), (130, 2056, 520), (500, 1032, 3080), (1000, 520, 3080),
-            (129, 4104, 3072), (3000, 264, 3136)]
+            (129, 4104, 3072), (3000, 264, 3136),
+            # tails that the sizes above leave out: 64x128 (both sides of 32), 128x128, 128x192 and 256x256 tiles,
+            # 32-row streams of 32 and 64 columns, 64x64 streams; 64-row streams without one
+            (1067, 1136, 1488), (782, 2160, 808), (403, 5136, 168), (1214, 4400, 168), (2330, 4104, 176), (1, 64, 304),
+            (92, 4088, 304), (395, 1472, 3896), (436, 856, 384)]
 
 
 @pytest.mark.parametrize("mnk", RAGGED_K)
@@ -325,7 +321,8 @@ def test_any_k_on_every_kernel(ops, mnk):
 # 32 and beside 64, one and two stages, blocks of eight rows without a row, edges on and off the tiles
 SHORT_K = [(1, 8, 8), (64, 64, 64), (65, 72, 120), (152, 392, 40), (7, 3984, 24), (63, 56, 32), (9, 136, 56), (130, 64, 16),
            (816, 1360, 8), (1837, 600, 96), (508, 2720, 40), (797, 2072, 104), (530, 3216, 64), (2268, 1672, 120),
-           (3052, 2256, 32), (1215, 3840, 8), (1506, 2752, 48), (4096, 4096, 64), (12, 968, 88), (782, 128, 104)]
+           (3052, 2256, 32), (1215, 3840, 8), (1506, 2752, 48), (4096, 4096, 64), (12, 968, 88), (782, 128, 104),
+           (65, 2184, 72), (794, 1016, 104)]
 
 
 @pytest.mark.parametrize("mnk", SHORT_K)
@@ -334,7 +331,8 @@ def test_short_k(ops, mnk):
 
 
 @pytest.mark.parametrize("bmnk", [(1, 1, 8, 8), (3, 9, 64, 40), (7, 65, 72, 120), (57, 2, 392, 48), (24, 3, 912, 72),
-                                  (15, 244, 504, 32), (34, 273, 928, 8), (36, 228, 224, 104), (7, 554, 776, 120)])
+                                  (15, 244, 504, 32), (34, 273, 928, 8), (36, 228, 224, 104), (7, 554, 776, 120),
+                                  (28, 1, 504, 120), (18, 331, 288, 40)])
 def test_batched_short_k(ops, bmnk):
     """Batched items with K below 128: the 64x64, 64x128 and 128x128 tiles."""
     test_batched_larger_items(ops, bmnk)
@@ -365,7 +363,12 @@ def test_infinity_in_the_last_k_row(ops, mnk):
                                   (7, 65, 136, 768), (16, 200, 128, 512), (64, 64, 128, 256), (65, 64, 128, 256),
                                   (16, 33, 512, 64), (37, 64, 264, 128), (128, 48, 512, 128), (3, 65, 72, 128),
                                   # ... up to 512 workgroups of 32 x 32 at any M, and one item more
-                                  (32, 128, 128, 64), (33, 128, 128, 64), (9, 96, 520, 128), (5, 1000, 72, 128)])
+                                  (32, 128, 128, 64), (33, 128, 128, 64), (9, 96, 520, 128), (5, 1000, 72, 128),
+                                  # 64x64 to 128x192 tiles from K 128 on, K tails on both sides of 32 and none
+                                  (1, 1, 8, 152), (1, 104, 8, 240), (12, 542, 232, 800), (9, 815, 248, 888),
+                                  (18, 222, 792, 176), (56, 374, 432, 216), (16, 563, 400, 296),
+                                  # small-row tiles of 64 and 128 columns, column tiles or items first in the grid
+                                  (64, 2, 496, 64), (137, 1, 232, 192), (119, 1, 616, 320)])
 def test_batched_larger_items(ops, bmnk):
     """Batched items with more than 32 rows, or a K that is no whole number of
     64-deep chunks, run the tiled kernels over the batch, or the small-row

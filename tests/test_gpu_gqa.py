@@ -169,12 +169,14 @@ def test_tile_rejections_enqueue_nothing(ops):
     assert torch.isnan(out.float()).all()
 
 
-# Sizes at which the default launch splits the keys between 2 or 4 groups of waves: fewer key tiles than
-# groups (S <= 64), last tiles of 1 and 63 keys, query rows whose group's first tile is masked, one head and
-# several per workgroup, and the sizes around which the choice of one group takes over.
-KEY_GROUPS = [(1, 1, 8, 8, 64), (1, 63, 8, 2, 64), (1, 65, 8, 1, 64), (2, 129, 8, 8, 128), (1, 191, 16, 4, 64),
-              (1, 257, 8, 4, 64), (1, 320, 8, 1, 128), (2, 447, 8, 8, 64), (1, 1000, 8, 2, 64), (1, 1025, 8, 4, 128),
-              (2, 1001, 16, 4, 64), (1, 577, 32, 8, 128), (4, 640, 16, 16, 64)]
+# Sizes at which the default launch splits the keys between 2 or 4 groups of waves: last tiles of 1, 2 and 63
+# keys, a group whose only tile has one key (S 129 and 193), query rows whose group's first tile is masked, one head
+# and several per workgroup; and sizes that one group takes, the shortest and one where the choice turns.
+ONE_GROUP = [(1, 1, 8, 8, 64), (1, 63, 8, 2, 64), (1, 65, 8, 1, 64), (2, 129, 8, 8, 128), (4, 640, 16, 16, 64)]
+KEY_GROUPS = ONE_GROUP + [(1, 191, 16, 4, 64), (1, 257, 8, 4, 64), (1, 320, 8, 1, 128), (2, 447, 8, 8, 64),
+                          (1, 1000, 8, 2, 64), (1, 1025, 8, 4, 128), (2, 1001, 16, 4, 64), (1, 577, 32, 8, 128),
+                          (1, 129, 8, 8, 64), (1, 130, 8, 2, 64), (1, 193, 8, 1, 64), (1, 193, 8, 8, 128),
+                          (1, 257, 8, 2, 128)]
 
 
 @pytest.mark.parametrize("causal", [True, False], ids=["c", "n"])

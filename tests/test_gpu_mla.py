@@ -126,9 +126,9 @@ def test_absorbed_pipeline(ops):
 
 @pytest.mark.parametrize("b,h,t,dv", [(32, 128, 4096, 128), (40, 16, 300, 64), (1, 128, 64, 128)])
 def test_absorbed_step_shapes(ops, b, h, t, dv):
-    """The one-call absorbed step at the BASELINE shape (split decode,
-    small-M projections), a batch above 32 (register-staged projections)
-    and a single sequence (unsplit decode)."""
+    """The one-call absorbed step at 32 sequences of 4096 tokens (split decode,
+    one row chunk per head in the projections), a batch above 32 (two row
+    chunks) and a single sequence of 64 tokens (unsplit decode)."""
     announce(f"mla absorbed step B{b} H{h} T{t} dv{dv}")
     s = shapes.MLADecodeShape("t", batch=b, n_h=h, ctx=t)
     _, kv = inputs.mla_inputs(s)
