@@ -658,10 +658,8 @@ static int dispatch_tile(const void* Q, const void* K, const void* V, void* O, i
 //    elsewhere (MLA prefill, 64 heads, S2199: 128 against 116; D 128, 64 heads
 //    in all, S647: 32.6 against 22.1).
 // The estimate, in units of a step with one group: a workgroup costs its steps
-// plus a start and end per query block, 256 run at once (512 of the four-wave
-// ones of head dims 96 / 64; with 256, B4 with 64 heads, S584, ran singly in 38.7
-// us, and in pairs takes 35.5); single causal workgroups, of all lengths, fill
-// the CUs evenly after the first round.
+// plus a start and end per query block, 256 run at once; single causal
+// workgroups, of all lengths, fill the CUs evenly after the first round.
 // Head dim 64 is fitted to 70 random shapes timed with every ksp (graph replay,
 // B 1..4, 8..32 heads, S 128..4200), head dim 128 to 120 with more heads and
 // shorter prompts (up to 64 x 96 heads, S 16..20000), where the first fit split
@@ -682,7 +680,6 @@ static Split pick_split(int B, int Hq, int Hkv, int S, int causal) {
   static constexpr Cost k128[] = {{1, 1.4, 5.75, 0.0}, {2, 1.72, 5.4, 0.15}};
   const Cost* cost = DQK == 64 ? k64 : k128;
   const int choices = DQK != DV ? 1 : DQK == 64 ? 3 : 2;
-  constexpr int slots = default_waves<DQK, DV>() == 4 ? 512 : 256;  // workgroups at once
   const int G = Hq / Hkv;
   Split best{1, default_hpw(G), true};
   double least = 0;
@@ -701,11 +698,11 @@ static Split pick_split(int B, int Hq, int Hkv, int S, int causal) {
       }
     };
     if (causal) {
-      const double total = 0.5 * (longest + shortest) * (double)(nqb * per) / slots;
-      consider((double)(((nqb + 1) / 2 * per + slots - 1) / slots) * (nqb > 1 ? longest + shortest : longest), true);
+      const double total = 0.5 * (longest + shortest) * (double)(nqb * per) / 256;
+      consider((double)(((nqb + 1) / 2 * per + 255) / 256) * (nqb > 1 ? longest + shortest : longest), true);
       consider(total > longest ? total : longest, false);
     } else {
-      consider((double)((nqb * per + slots - 1) / slots) * longest, true);
+      consider((double)((nqb * per + 255) / 256) * longest, true);
     }
   }
   return best;
