@@ -54,14 +54,11 @@ inline bool strides_2g(int lda, int ldb) {
   return (long long)lda * 2 * BM < 0x7ffffff0LL && (long long)ldb * 2 * 64 < 0x7ffffff0LL;
 }
 
-// A-row chunk swizzle of the small-M kernels' LDS rows: a 16-lane
-// ds_read_b128 phase reads one chunk of 16 consecutive rows, and chunk ^
-// swz_a(m) puts them in 16 distinct 16-byte slots of the 256-byte bank
-// window (64-byte rows: (m >> 2) & 3; 128-byte rows: (m >> 1) & 7).
-template <int BK>
-__device__ __forceinline__ int swz_a(int m) {
-  return BK == 64 ? ((m >> 1) & 7) : ((m >> 2) & 3);
-}
+// A-row chunk swizzle of every kernel here: rows of 128 bytes, whose chunk c
+// sits at c ^ swz_a(row).  A 16-lane ds_read_b128 phase reads one chunk of 16
+// consecutive rows, which this puts in 16 distinct 16-byte slots of the 256-byte
+// bank window.
+__device__ __forceinline__ int swz_a(int m) { return (m >> 1) & 7; }
 
 // Below this K a tile takes the whole K to LDS at once (gemm_bf16_short_kernel).
 constexpr int kShortK = 128;
@@ -110,7 +107,6 @@ __device__ __forceinline__ u32x4 keep_if(bool keep, const u32x4& x) { return kee
 //    start, each A^T one in place right after the MFMAs that consumed the
 //    previous one's.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ int swz_a16w(int m) { return (m >> 1) & 7; }
 __device__ __forceinline__ int swz_b16(int k) { return 2 * ((k & 3) | (((k >> 3) & 1) << 2)); }
 template <int BM_, int BN_, int WM, int WN, int NS_>
 struct D64Cfg {
@@ -244,7 +240,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     const int ld = wave * CF::LPW + n;
     if (ld < CF::A_L) {
       const int row = CF::A_RPL * ld + lane / 8;
-      off[n] = (uint32_t)(min(m0 + row, M - 1) - m0) * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_a16w(row));
+      off[n] = (uint32_t)(min(m0 + row, M - 1) - m0) * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_a(row));
     } else {
       const int byte = 1024 * (ld - CF::A_L) + 16 * lane;
       const int row = byte / CF::RB;
@@ -273,7 +269,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
   for (int st = 0; st < NS; ++st)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      a_col[st][h] = lds0 + st * CF::STAGE + am * CF::RA + 16 * ((4 * h + kg) ^ swz_a16w(am));
+      a_col[st][h] = lds0 + st * CF::STAGE + am * CF::RA + 16 * ((4 * h + kg) ^ swz_a(am));
       asm volatile("" : "+v"(a_col[st][h]));  // keep it a base register
     }
   // B^T (A operand): lane (kg, j, a) reads k-rows 32h + 8kg + 4r + j, columns
@@ -354,7 +350,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_, 1) void gemm_bf16_dma64_kernel(
     for (int n = 0; n < CF::LPW; ++n) {
       const int ld = wave * CF::LPW + n;
       if (ld < CF::A_L) {
-        const uint32_t swz = 16u * ((lane % 8) ^ swz_a16w(CF::A_RPL * ld + lane / 8));
+        const uint32_t swz = 16u * ((lane % 8) ^ swz_a(CF::A_RPL * ld + lane / 8));
         dma16(abase, off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), st + ld * 1024);
       } else {
         const int row = (1024 * (ld - CF::A_L) + 16 * lane) / CF::RB;
@@ -447,7 +443,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_) void gemm_bf16_short_kernel(
       const int ld = wave * CF::LPW + n;
       if (ld < CF::A_L) {
         const int row = CF::A_RPL * ld + lane / 8;
-        const int chunk = min(8 * ((lane % 8) ^ swz_a16w(row)), kr - 8);  // elements
+        const int chunk = min(8 * ((lane % 8) ^ swz_a(row)), kr - 8);  // elements
         if (CF::A_RPL * ld < M - m0)
           dma16(abase, (uint32_t)(min(m0 + row, M - 1) - m0) * (uint32_t)lda * 2u + 2u * chunk, st + ld * 1024);
       } else {
@@ -465,7 +461,7 @@ __global__ __launch_bounds__(64 * WM_ * WN_) void gemm_bf16_short_kernel(
   // second half of a stage is 64 bytes (one bit) across in A and 32 k-rows on
   // in B.
   const int am = wm * CF::TM + (lane & 15);
-  uint32_t a_col = lds0 + am * CF::RA + 16 * (kg ^ swz_a16w(am));
+  uint32_t a_col = lds0 + am * CF::RA + 16 * (kg ^ swz_a(am));
   const int b_j = (lane >> 2) & 3, b_a = lane & 3;
   const int bk = 8 * kg + b_j;
   uint32_t b_col[FN];
@@ -558,21 +554,22 @@ static int launch_dma64(const void* A, const void* B, void* C, int M, int N, int
 }
 
 // ---------------------------------------------------------------------------
-// gemm_bf16_dma16s_kernel: gemm_bf16_dma16_kernel's 256x256 tiles and
-// fragment schedule with whole 128-byte A lines.  In the single ring, a
-// 32-deep stage holds 64 bytes of each A row, so every A line is fetched as
-// two half-line requests; the L1 then holds up the address unit (the fp8
-// GEMM measured the same).  Here A goes through its own ring of 64-deep
-// blocks (256 rows x 128 B, 3 slots) beside a ring of 32-deep B stages
-// (32 k-rows x 512 B, 4 slots), 160 KB in all:
+// gemm_bf16_dma16s_kernel: 256x256 tiles, eight waves of 128x64 on 16x16x32
+// MFMAs, the fragments of the next 32-deep K tile read during the current one's
+// MFMAs as in the kernel above.  A single ring of 32-deep stages would hold 64
+// bytes of each A row and fetch every 128-byte line of A as two half-line
+// requests, which hold up the L1's address unit; 64-deep stages of both would
+// leave room for two.  So A goes through its own ring of 64-deep blocks (256
+// rows x 128 B, 3 slots) beside a ring of 32-deep B stages (32 k-rows x 512 B,
+// 4 slots), 160 KB in all:
 //  * step kt computes K tile kt (B stage kt, half kt % 2 of A block kt / 2)
 //    and reads tile kt+1's fragments; it issues B stage kt+3 and half kt % 2
 //    of A block kt/2 + 2, each into the slot of the stage / block that the
 //    barrier just freed, so every step issues the same 4 loads per wave and
 //    waits for all but the 4 of the step before.
-//  * A rows of 8 chunks: chunk c ^ ((m >> 1) & 7) keeps the 16-lane phases
-//    of the A^T reads on distinct bank slots.
-// Shapes: K % 64 == 0 (whole A blocks).
+//  * A rows (128 B) and B rows (512 B) are swizzled by swz_a and swz_b16.
+// Shapes: any K of at least 64.  The K % 64 tail is computed before the K loop,
+// from A slot 2 and B slots 3 and 2.
 // ---------------------------------------------------------------------------
 struct S16Cfg {
   static constexpr int BM = 256, BN = 256, BK = 32, BKA = 64;
@@ -592,23 +589,6 @@ struct S16Cfg {
   static constexpr int P = 12;                        // steps until slots and parity repeat
   static_assert(LDS <= 160 * 1024 && A_LPW % 2 == 0 && A_LPW >= 2 && B_LPW >= 1, "rings");
 };
-
-template <int P, int I = 0, typename Step>
-__device__ __forceinline__ void steps_s(Step& step, int kt) {
-  if constexpr (I < P) {
-    step(kt + I, std::integral_constant<int, I>{});
-    steps_s<P, I + 1>(step, kt);
-  }
-}
-template <int P, int I = 0, typename Step>
-__device__ __forceinline__ void steps_tail_s(Step& step, int kt, int n) {
-  if constexpr (I < P - 1) {
-    if (I < n) {
-      step(kt + I, std::integral_constant<int, I>{});
-      steps_tail_s<P, I + 1>(step, kt, n);
-    }
-  }
-}
 
 template <bool TAIL>
 __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const uint16_t* __restrict__ A,
@@ -638,7 +618,7 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   for (int n = 0; n < CF::A_LPW; ++n) {
     const int row = CF::A_RPL * (wave * CF::A_LPW + n) + lane / 8;
     const int gm = full_m ? m0 + row : min(m0 + row, M - 1);
-    a_off[n] = (uint32_t)(gm - m0) * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_a16w(row));
+    a_off[n] = (uint32_t)(gm - m0) * (uint32_t)lda * 2u + 16u * ((lane % 8) ^ swz_a(row));
   }
 #pragma unroll
   for (int n = 0; n < CF::B_LPW; ++n) {
@@ -673,7 +653,7 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
   for (int st = 0; st < CF::NSA; ++st)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      a_col[st][h] = lds0 + st * CF::A_B + am * CF::RA + 16 * ((4 * h + kg) ^ swz_a16w(am));
+      a_col[st][h] = lds0 + st * CF::A_B + am * CF::RA + 16 * ((4 * h + kg) ^ swz_a(am));
       asm volatile("" : "+v"(a_col[st][h]));  // keep it a base register
     }
   // B^T (A operand): lane (kg, j, a) reads k-rows 8kg + 4r + j, columns
@@ -745,7 +725,7 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
     const uint16_t* bbase = B + (size_t)nka * CF::BKA * ldb + n0;
 #pragma unroll
     for (int n = 0; n < CF::A_LPW; ++n) {
-      const uint32_t swz = 16u * ((lane % 8) ^ swz_a16w(CF::A_RPL * (wave * CF::A_LPW + n) + lane / 8));
+      const uint32_t swz = 16u * ((lane % 8) ^ swz_a(CF::A_RPL * (wave * CF::A_LPW + n) + lane / 8));
       dma16(abase, a_off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), lds0 + 2 * CF::A_B + (wave * CF::A_LPW + n) * 1024);
     }
 #pragma unroll
@@ -795,8 +775,8 @@ __global__ __launch_bounds__(S16Cfg::NT, 1) void gemm_bf16_dma16s_kernel(const u
 #pragma unroll
   for (int mf = 0; mf < FM; ++mf) read_a(0, 0, mf);
   int kt = 0;
-  for (; kt + CF::P <= nk; kt += CF::P) steps_s<CF::P>(step, kt);
-  steps_tail_s<CF::P>(step, kt, nk - kt);
+  for (; kt + CF::P <= nk; kt += CF::P) step_period<CF::P>(step, kt);
+  step_tail<CF::P>(step, kt, nk - kt);
   wait_vmcnt<0>();  // no DMA may land in LDS after the workgroup ends
 
   // ---- epilogue: lane holds m = am + 16 mf, n = wn*TN + 16 nf + 4 kg + {0..3} ----
@@ -887,14 +867,14 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
   const uint32_t lds0 = lds_addr(smem);
 
   // Direct-load lane offsets.  A load n (0..3): rows 8n + lane/8, chunk
-  // (lane%8) ^ swz_a<64>(row); rows past M re-read row M-1.  B load n:
+  // (lane%8) ^ swz_a(row); rows past M re-read row M-1.  B load n:
   // k-rows BRPL n + lane/BCH, chunk (lane%BCH) ^ sm_swz(k-row); columns
   // past N re-read the last valid 8.
   uint32_t a_off[4], b_off[BL];
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int row = 8 * n + (lane >> 3);
-    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_a<64>(row));
+    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_a(row));
   }
 #pragma unroll
   for (int n = 0; n < BL; ++n) {
@@ -918,7 +898,7 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
   const int am = lane & 31;
   const int b_sg = (lane >> 4) & 1, b_j = (lane >> 2) & 3, b_a = lane & 3;
   const uint32_t a_base = lds0 + am * 128;
-  const int ax = swz_a<64>(am);
+  const int ax = swz_a(am);
   uint32_t b_base[NF];
 #pragma unroll
   for (int nf = 0; nf < NF; ++nf) {
@@ -1000,7 +980,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
 #pragma unroll
   for (int n = 0; n < 4; ++n) {
     const int row = 8 * n + (lane >> 3);
-    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_a<64>(row));
+    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_a(row));
   }
 #pragma unroll
   for (int n = 0; n < BL; ++n) {
@@ -1021,7 +1001,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint
   const int am = lane & 31;
   const int b_sg = (lane >> 4) & 1, b_j = (lane >> 2) & 3, b_a = lane & 3;
   const uint32_t a_base = lds0 + am * 128;
-  const int ax = swz_a<64>(am);
+  const int ax = swz_a(am);
   uint32_t b_base[NF];
 #pragma unroll
   for (int nf = 0; nf < NF; ++nf) {
@@ -1136,16 +1116,17 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
 //    the 64-deep K blocks kb = w, w + NW, ..., so every workgroup streams its
 //    columns of B once.  The row chunks of a column block and the
 //    neighbouring column blocks run on one XCD, where they share B's
-//    128-byte lines in L2.
+//    128-byte lines in L2; with more rows than columns, the column blocks of a
+//    row chunk.
 //  * Each wave has a private ring of NSL slots, one K block per slot (A: 32 MF
 //    rows x 128 B, chunk c at c ^ ((m >> 1) & 7); B: 64 k-rows x 64 NC B), by
 //    direct loads; slots are private, so the block loop has no barrier.
 //  * What bounds it is the CU's rate of line requests (about one per 3-4
 //    clocks, 64 or 128 bytes alike), so 64 columns where they still fill the
 //    CUs; eight waves with rings of two slots keep as many loads in flight as
-//    four with four and reach each block sooner (16x7168x4096 15.3 -> 15.1 us,
-//    1x696x1520 6.2 -> 5.2, 27x512x1280 4.96 -> 4.61; the other way at 5x712x6272,
-//    15.6 -> 15.9, which neither tiles nor K tells from the rest).
+//    four with four and reach each block sooner, which shows on short K only
+//    (against four waves: 27x512x1280 4.14 -> 4.09 us, 16x7168x4096 14.5 either
+//    way, 5x712x6272 13.3 -> 13.9).
 //  * C^T = B^T . A^T on 32x32x16 MFMAs: B^T fragments by transposing reads
 //    from the B rows (swz_sb), A^T fragments by ds_read_b128.
 //  * The waves' accumulators meet in LDS at the end; four waves sum and store
@@ -1166,21 +1147,12 @@ struct StreamCfg {
   static_assert((NSL - 1) * VM < 64, "vmcnt range");
   static_assert(NW * MF * NC * 64 * 16 * 4 <= LDS, "reduction area");
 };
-__device__ __forceinline__ int swz_s(int m) { return (m >> 1) & 7; }
 // B rows of 128 bytes: a transposing read phase (4 consecutive k-rows x 64
 // bytes) spans the 256-byte bank window twice, so k-rows 2 and 3 swap their
 // halves; rows of 64 bytes fill it once.
 template <int NC>
 __device__ __forceinline__ int swz_sb(int k) {
   return NC == 1 ? 0 : ((k >> 1) & 1) << 2;
-}
-// f(integral_constant<int, I>) for I = 0 .. N-1, in order.
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void unroll_n(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll_n<N, I + 1>(f);
-  }
 }
 
 template <int MF, int NC, int NW, int NSL, bool TAIL>
@@ -1216,7 +1188,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
 #pragma unroll
   for (int n = 0; n < CF::A_L; ++n) {
     const int row = 8 * n + (lane >> 3);
-    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_s(row));
+    a_off[n] = (uint32_t)min(row, M - 1) * (uint32_t)lda * 2u + 16u * ((lane & 7) ^ swz_a(row));
   }
   constexpr int CH = CF::BN / 8, BR = 64 / CH;  // 16-byte chunks per k-row, k-rows per load
   const int b_row = lane / CH;                   // from k-row BR n; BR n has no part in swz_sb
@@ -1239,7 +1211,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
   const int am = lane & 31, g = lane >> 5;
   uint32_t a_col[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) a_col[ks] = am * 128 + 16 * ((2 * ks + g) ^ swz_s(am));
+  for (int ks = 0; ks < 4; ++ks) a_col[ks] = am * 128 + 16 * ((2 * ks + g) ^ swz_a(am));
   const int G = lane >> 4, bj = (lane >> 2) & 3, ba = lane & 3;
   uint32_t b_col[NC];
 #pragma unroll
@@ -1287,7 +1259,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_bf16_stream_kernel(const uint
     const uint32_t st = ring + (NSL - 1) * CF::SLOT;
 #pragma unroll
     for (int n = 0; n < CF::A_L; ++n) {
-      const uint32_t swz = 16u * ((lane & 7) ^ swz_s(8 * n + (lane >> 3)));
+      const uint32_t swz = 16u * ((lane & 7) ^ swz_a(8 * n + (lane >> 3)));
       dma16(A + (size_t)kblocks * 64, a_off[n] - swz + min(swz, (uint32_t)(2 * kr - 16)), st + n * 1024);
     }
 #pragma unroll
@@ -1371,7 +1343,12 @@ static int launch_stream(const void* A, const void* B, void* C, int M, int N, in
 // (fill).  Fitted (relative least squares, no negative term) to 450 random
 // shapes, M 1..8192, N and K 512..8192, ragged and whole, each timed on every
 // kernel by graph replay; the kernel picked is on average about 1% slower than
-// the fastest.  The 64-column streams against the four-wave 32-column ones and
+// the fastest, there and over 600 more shapes with M and N up to 131072 and K
+// from 128 (16x129280x7168 322 us at 5.75 TB/s, 446 with four-wave streams).  3%
+// of those are more than 3% slower than the 32-deep ring and register-staged
+// tiles, up to 20%, which no kernel here matches: K an odd multiple of 32 below
+// 700 (6352x1088x480 13.0 -> 14.7) and 70 to 90 columns under 50000 rows and more
+// (109374x72x488 28.7 -> 34.6).  The 64-column streams against the four-wave 32-column ones and
 // the tiles alone: 260x3008x6080 30.2 -> 21.8 us, 524x1536x8064 42 -> 27 (64
 // rows), 158x1664x6512 25.3 -> 20.4, 142x3032x2408 14.4 -> 12.6 (32 rows); below
 // 48 K blocks the 64-row one is 5-10% behind 64x64 tiles (763x1280x1024 8.55
@@ -1469,9 +1446,12 @@ static int launch_tiled(Path path, const void* A, const void* B, void* C, int M,
   }
 }
 
-// The leading dimensions the interface takes: with K % 32 != 0 or a small
-// grid, lda * 2 * BM (BM rows per tile: 256, 128 or 64) and ldb * 2 * 64 below
-// 2^31; otherwise spans below 4 GiB.
+// The leading dimensions the interface takes, as mx_kernels.h states them: with
+// K % 32 != 0 or a small grid, lda * 2 * BM (BM = 256, 128 or 64) and ldb * 2 * 64
+// below 2^31; otherwise spans below 4 GiB.  The grid and BM are those of a fixed
+// choice of tile by size and not of the kernel that gemm_path picks: a refit of
+// its costs must not change which calls are refused.  Every shape taken here has
+// a kernel there, whose own bound (4 GiB spans) is the wider one.
 static bool strides_ok(int M, int N, int K, int lda, int ldb) {
   const long long la = lda, lb = ldb, four_g = 0xffffffffLL;
   auto tiles = [&](int t) { return (long long)((M + t - 1) / t) * ((N + t - 1) / t); };

@@ -522,14 +522,6 @@ struct SmallCfg {
   static_assert(NC == 1 || NC == 2, "columns within one weight-scale block, row swizzle");
 };
 
-// f(integral_constant<int, I>) for I = 0 .. N-1, in order.
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void unroll_n(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll_n<N, I + 1>(f);
-  }
-}
 
 __device__ __forceinline__ int swz_sa(int m) { return (m >> 1) & 7; }
 // B rows of 64 bytes: eight consecutive k-rows x 32 bytes (a transposing read
@@ -747,8 +739,12 @@ static int launch_smallm(const void* A, const float* sA, const void* B, const fl
 // waves, chosen by M and by rounds: 8% in geometric mean; 128x7168x2048 16.3 ->
 // 10.6 us, 256x4096x4096 26.1 -> 15.1 and 524x1536x8064 54 -> 23 (64x64
 // streams), 3072^3 44.8 -> 37.1 (192x256), 730x7120x2816 34.7 -> 29.0 (128x256),
-// 64x4096x7168 20.5 -> 18.5 (eight waves); a few near ties lose 1-4%
-// (4096x4096x128 11.8 -> 12.3, 1539x4992x2560 with the quantiser 33.9 -> 34.3).
+// 64x4096x7168 20.5 -> 18.5 (eight waves), 16x129280x7168 336 -> 199.  Over 460
+// more shapes, M and N up to 131072 and K from 128, the kernel picked is also 0.7%
+// behind the fastest (a term for the C tiles makes it 0.6%); 1% of them are 3 to
+// 14% slower than by the former rules, near ties of the estimates (15356x7120x512
+// 97 -> 111 us, 1539x7728x128 9.7 -> 10.7, 33x3920x2560 6.5 -> 7.4, 1539x4992x2560
+// 29.5 -> 31.9).
 // Not kept: 256x128 tiles, 32x64
 // streams and 32x32 streams of four waves were the fastest by up to 6, 8 and
 // 1% for 2 to 5 shapes in 180, and without them the mean is the same.

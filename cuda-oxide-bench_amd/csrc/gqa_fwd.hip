@@ -647,16 +647,17 @@ static int dispatch_tile(const void* Q, const void* K, const void* V, void* O, i
 // heads, and whether causal workgroups take a long and a short query block.
 //  * More key groups make the workgroups smaller (256 / ksp query rows) and
 //    their serial chain of key tiles shorter, for a dearer step: worth it while
-//    the launch is as long as its longest workgroup.  At head dim 64, B2 Hq16
-//    S1001 non-causal takes 21.6 us with one group, 15.7 with two, 20.2 with
-//    four, and causal B1 Hq8 S1092 21.1, 14.5 and 11.4; at 128, causal B1 Hq16
-//    S1335 36.1 and 25.0, but S4096 with 32 heads 126 and 142.  Four groups at
-//    128 do not fit the LDS; two at the 192-wide query of MLA spill registers
-//    and measured slower.
+//    the launch is as long as its longest workgroup (bf16, graph replay).  At
+//    head dim 64, B2 Hq16 S1001 non-causal takes 20.3 us with one group, 14.4 with
+//    two, 18.7 with four, and causal B1 Hq8 S1092 (singly) 20.9, 13.7 and 10.7; at
+//    128, causal B1 Hq16 S1335 34.8 and 24.0, but S4096 with 32 heads 131 and 147.
+//    Four groups at 128 do not fit the LDS; two at the 192-wide query of MLA
+//    spill registers and measured slower.
 //  * Pairs make equal workgroups, which is best where they fill whole rounds of
-//    the CUs (S4096, 32 heads: 126 us against 127.6 singly), and leave CUs idle
-//    elsewhere (MLA prefill, 64 heads, S2199: 128 against 116; D 128, 64 heads
-//    in all, S647: 32.6 against 22.1).
+//    the CUs (S4096, 32 heads: 131 us against 133 singly), and leave CUs idle
+//    elsewhere (MLA prefill, 64 heads, S2199: 129 against 116; D 128, 64 heads
+//    in all, S647: 31.5 against 21.4).  At head dims 96 / 64 the estimate is the
+//    other way now and then (B4 with 64 heads, S584, 37.1 us singly, 34.2 in pairs).
 // The estimate, in units of a step with one group: a workgroup costs its steps
 // plus a start and end per query block, 256 run at once; single causal
 // workgroups, of all lengths, fill the CUs evenly after the first round.

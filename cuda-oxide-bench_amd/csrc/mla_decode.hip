@@ -99,7 +99,10 @@ inline Split pick_split(int B, int H, int T) {
   const int nblk = (T + BT - 1) / BT;
   // As many splits as one round of workgroups takes (one per CU), of at least
   // two stages each.  A round more costs more than idle CUs: B48 H128 T3000
-  // takes 61 us with 5 splits (240 workgroups) and 79 us with 8 (384).
+  // takes 61 us with 5 splits (240 workgroups) and 77 us with 8 (384), merge
+  // included.  Short sequences with the most splits can lose to powers of two,
+  // which made fewer (B2 H256 T2488 24.1 -> 26.3 us, 2% of 465 random shapes by
+  // more than 3%); no minimum of stages other than two does better on the whole.
   long long ns = 256 / ((long long)B * hg);
   if (ns > nblk / 2) ns = nblk / 2;
   if (ns < 1) ns = 1;

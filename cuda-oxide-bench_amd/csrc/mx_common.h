@@ -8,6 +8,7 @@
 #include <stdint.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "mx_kernels.h"
 
@@ -106,14 +107,6 @@ __device__ __forceinline__ f32x16 mfma32<F16>(const u32x4& a, const u32x4& b, co
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
-// fp8 e4m3 (OCP "fn" encoding on gfx950) x e4m3 -> fp32, 16x16x128.
-// Issued through the block-scaled form with both E8M0 scales = 127 (2^0),
-// i.e. an unscaled product.  A: lane l holds row l%16 and 32 k-bytes,
-// B: lane l holds col l%16 and the same 32 k positions.
-__device__ __forceinline__ f32x4 mfma16_fp8(const i32x8& a, const i32x8& b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, 0, 0, 0, 127, 0, 127);
-}
-
 // acc += a·b on a 32x32x16 MFMA whose accumulator stays in AGPRs.  The
 // builtin MFMAs of a kernel all take one register class, chosen by the
 // compiler; issuing this one as inline asm keeps its accumulator in AGPRs
@@ -184,39 +177,6 @@ __device__ __forceinline__ float max_xor16(float v) {
 __device__ __forceinline__ float sum_xor16(float v) {
   auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// ---------------------------------------------------------------------------
-// 8x8 transpose of 16-bit elements held as 8 rows x 4 dwords.
-// in[r] holds row r (elements 2j, 2j+1 in dword j); out[c] holds column c
-// (rows 2j, 2j+1 in dword j).  Pure VALU byte permutes.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void transpose8x8_b16(const u32x4 in[8], u32x4 out[8]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {      // dword j of every output = rows 2j, 2j+1
-#pragma unroll
-    for (int c2 = 0; c2 < 4; ++c2) { // input dword c2 holds columns 2c2, 2c2+1
-      uint32_t x = in[2 * j][c2];
-      uint32_t y = in[2 * j + 1][c2];
-      out[2 * c2][j] = __builtin_amdgcn_perm(y, x, 0x05040100u);      // lo halves
-      out[2 * c2 + 1][j] = __builtin_amdgcn_perm(y, x, 0x07060302u);  // hi halves
-    }
-  }
-}
-
-// 4x8 (rows x cols) 16-bit transpose: in[r] (r<4) holds row r as 4 dwords;
-// out[c] (c<8) receives column c as 2 dwords (rows 0,1 | rows 2,3).
-__device__ __forceinline__ void transpose4x8_b16(const u32x4 in[4], u32x2 out[8]) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-#pragma unroll
-    for (int c2 = 0; c2 < 4; ++c2) {
-      uint32_t x = in[2 * j][c2];
-      uint32_t y = in[2 * j + 1][c2];
-      out[2 * c2][j] = __builtin_amdgcn_perm(y, x, 0x05040100u);
-      out[2 * c2 + 1][j] = __builtin_amdgcn_perm(y, x, 0x07060302u);
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -296,22 +256,6 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Scheduling of one region of NM MFMAs and R LDS reads (issued in that
-// region for a later use): alternate one MFMA with an even share of the
-// reads, so a read lookahead never needs more than a few LDS instructions in
-// flight (lgkmcnt counts at most 15) and the compiler can wait for exactly
-// the reads each MFMA needs.  Call right after the region's code, before a
-// sched_barrier that closes the region.
-template <int NM, int R, int I = 0>
-__device__ __forceinline__ void interleave_mfma_ds() {
-  if constexpr (I < NM) {
-    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-    constexpr int r = (R * (I + 1)) / NM - (R * I) / NM;
-    if constexpr (r > 0) __builtin_amdgcn_sched_group_barrier(0x100, r, 0);  // r LDS reads
-    interleave_mfma_ds<NM, R, I + 1>();
-  }
-}
-
 // Make the kernel-argument loads of `xs` complete here.  Arguments used
 // only after a kernel's main loop (an output pointer) are otherwise loaded
 // before the loop and left pending; the compiler then treats the lgkm
@@ -324,6 +268,15 @@ __device__ __forceinline__ void land_arg(const T& x) {
 template <typename... Ts>
 __device__ __forceinline__ void land_args(const Ts&... xs) {
   (land_arg(xs), ...);
+}
+
+// f(integral_constant<int, I>) for I = 0 .. N-1, in order.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unroll_n(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll_n<N, I + 1>(f);
+  }
 }
 
 // 32-bit LDS byte address of a pointer into __shared__ memory.
@@ -347,9 +300,6 @@ __device__ __forceinline__ void st128(void* p, const u32x4& v) { *reinterpret_ca
 __device__ __forceinline__ u32x2 ld64(const void* p) { return *reinterpret_cast<const u32x2*>(p); }
 __device__ __forceinline__ void st64(void* p, const u32x2& v) { *reinterpret_cast<u32x2*>(p) = v; }
 
-__device__ __forceinline__ u32x4 ld128_nt(const void* p) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
-}
 __device__ __forceinline__ void st128_nt(void* p, const u32x4& v) {
   __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(p));
 }
