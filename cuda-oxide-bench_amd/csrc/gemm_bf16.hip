@@ -1372,6 +1372,21 @@ constexpr Kernel kKernels[] = {
     {Path::T256, 256, 256, 256, 2.082f, 6.139f, 0.977f, 0.532f, 64},
 };
 
+// The tiles over 16 items and more of a batched product: their operands are not
+// shared between items, so more of them at once cost more (fill).  Fitted to 670
+// random launches, 1 to 256 items of M 1..256, N and K to 2048, contiguous and
+// strided by head.  Over 450 others the choice is 1.5% behind the fastest tile on
+// average, with the costs of single products 5.4% (92 items of 168x224x384
+// 20.9 us with 64x64 tiles, 16.2 with 128x128).  Up to 15 items those are the
+// better ones (0.1% against 0.3%; 2 of 404x1048x1392 9.1 us, here 10.8).
+constexpr int kManyItems = 16;
+constexpr Kernel kBatchedKernels[] = {
+    {Path::T64, 64, 64, 512, 1.660f, 1.249f, 0.135f, 0.707f, 0},
+    {Path::T64x128, 64, 128, 256, 1.237f, 2.001f, 0.243f, 0.362f, 0},
+    {Path::T128, 128, 128, 256, 1.049f, 2.420f, 0.339f, 0.446f, 0},
+    {Path::T128x192, 128, 192, 256, 0.620f, 3.439f, 0.460f, 0.477f, 0},
+};
+
 // The same below K = 128, where tiles take gemm_bf16_short_kernel: fixed +
 // first K/64 + round ceil(x) + (tile + fill K/64) x with x = tiles / 256, since
 // a CU holds several workgroups of these.  Fitted to 440 random shapes, single
@@ -1419,10 +1434,13 @@ static Path gemm_path(int M, int N, int K, int lda, int ldb, int batch) {
         return c.fixed + c.first * kb + c.round * __builtin_ceil(x) + (c.tile + c.fill * kb) * x;
       });
   } else {
-    for (const Kernel& k : kKernels)
-      consider(k, [&](const Kernel& c, double tiles) {
-        return c.fixed + __builtin_ceil(tiles / c.slots) * (c.round + c.step * kb) + c.fill * kb * tiles / c.slots;
-      });
+    auto cost = [&](const Kernel& c, double tiles) {
+      return c.fixed + __builtin_ceil(tiles / c.slots) * (c.round + c.step * kb) + c.fill * kb * tiles / c.slots;
+    };
+    if (batch >= kManyItems)
+      for (const Kernel& k : kBatchedKernels) consider(k, cost);
+    else
+      for (const Kernel& k : kKernels) consider(k, cost);
   }
   return best;
 }
