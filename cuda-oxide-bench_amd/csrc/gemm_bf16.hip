@@ -809,11 +809,11 @@ static int launch_dma16s(const void* A, const void* B, void* C, int M, int N, in
 // NS-stage ring, NS-1 chunks ahead (6 stages for narrow tiles, 4 at NF = 4:
 // 48-80 KB of LDS, two workgroups per CU).  A single wave needs no barrier: the ring stage
 // it overwrites was consumed by its own MFMAs, which waited for those
-// reads.  With items first in the grid (by_item) the row chunks and column tiles
-// of an item run on one XCD, whose L2 then holds its A and B once: 64 items of
-// 32 x 128 x 512 6.33 -> 4.31 us, items with three and more chunks of K 5%
-// faster; one or two chunks gain nothing and keep the column tiles first (182
-// items of 2 x 512 x 128 7.5 us against 8.8).  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
+// reads.  With three and more chunks of K an item's row chunks and column tiles
+// run on one XCD, whose L2 then holds its A and B once (64 items of 32 x 128 x
+// 512 6.33 -> 4.31 us, 19 of 3 x 920 x 1024 17.4 -> 9.6); with one or two that
+// gains nothing, and the plain order is the faster one (182 items of 2 x 512 x
+// 128 7.5 us against 8.8).  A rows (128 B) use the 16-row chunk swizzle of the large kernel;
 // B rows (64 NF bytes) put chunk c of k-row k at c ^ (((k & 3) << 2) mod
 // (4 NF)) so the 4 consecutive k-rows of a transposing read phase occupy
 // distinct 64-byte quarters of the bank sweep (no swizzle needed at NF = 1,
@@ -827,22 +827,38 @@ __device__ __forceinline__ int sm_swz(int k) {
   return NF == 1 ? 0 : (((k & 3) << 2) & (4 * NF - 1));
 }
 
-// The tile of a workgroup: the grid's dimensions are the indices, since the
-// divisions of a flat one take 0.1 to 0.15 us of these 3 us launches.
-struct SmallTile {
-  int item, ct, mc;  // batch item, column tile, row chunk
+// Division of n < 2^31 by a number that the host knows: with s = ceil(log2 d) and
+// m = ceil(2^(31 + s) / d), n m / 2^(31 + s) exceeds n / d by less than
+// n / 2^31 / d.  Four plain divisions took 0.1 to 0.15 us of these 3 us launches.
+struct Div {
+  uint32_t d, m, shift;
 };
-__device__ __forceinline__ SmallTile small_tile(bool by_item) {
-  return by_item ? SmallTile{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z}
-                 : SmallTile{(int)blockIdx.y, (int)blockIdx.x, (int)blockIdx.z};
+inline Div make_div(uint32_t d) {
+  uint32_t s = 0;
+  while ((1ull << s) < d) ++s;
+  return Div{d, (uint32_t)(((1ull << (31 + s)) + d - 1) / d), 31 + s};
+}
+__host__ __device__ __forceinline__ uint32_t quot(uint32_t n, const Div& v) {
+  return (uint32_t)(((uint64_t)n * v.m) >> v.shift);
+}
+
+// The tile of a workgroup.  Consecutive ids are the row chunks of a column tile,
+// then an item's column tiles; with xcd each XCD takes a contiguous run of them.
+struct SmallTile {
+  uint32_t item, ct, mc;  // batch item, column tile, row chunk
+};
+__device__ __forceinline__ SmallTile small_tile(bool xcd, const Div& chunks, const Div& tiles) {
+  const uint32_t id = xcd ? (uint32_t)xcd_remap(blockIdx.x, (int)gridDim.x) : blockIdx.x;
+  const uint32_t rest = quot(id, chunks), item = quot(rest, tiles);
+  return SmallTile{item, rest - item * tiles.d, id - rest * chunks.d};
 }
 
 template <int NF>
 __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __restrict__ A,
                                                               const uint16_t* __restrict__ B,
-                                                              uint16_t* __restrict__ C, int batch, int M, int N, int K,
+                                                              uint16_t* __restrict__ C, int M, int N, int K,
                                                               int lda, int ldb, int ldc, long long sA, long long sB,
-                                                              long long sC, bool by_item) {
+                                                              long long sC, bool xcd, Div chunks, Div tiles) {
   constexpr int TN = 32 * NF;                 // columns per workgroup
   constexpr int RB = TN * 2;                  // B row bytes in LDS
   constexpr int B_B = SM_BK * RB;             // B chunk bytes
@@ -855,10 +871,9 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
   __shared__ __align__(1024) unsigned char smem[SM_NS * STAGE];
   const int lane = threadIdx.x;
   const int g = lane >> 5;
-  const SmallTile t = small_tile(by_item);
+  const SmallTile t = small_tile(xcd, chunks, tiles);
   const size_t item = t.item;
   const int n0 = t.ct * TN, m0 = t.mc * 32;
-  if (t.item >= batch) return;
   A += item * sA + (size_t)m0 * lda;
   B += item * sB;
   C += item * sC + (size_t)m0 * ldc;
@@ -954,19 +969,19 @@ __global__ __launch_bounds__(64) void gemm_bf16_smallm_kernel(const uint16_t* __
 template <int NF, int KW>
 __global__ __launch_bounds__(64 * KW) void gemm_bf16_smallm_sk_kernel(const uint16_t* __restrict__ A,
                                                                      const uint16_t* __restrict__ B,
-                                                                     uint16_t* __restrict__ C, int batch, int M, int N,
-                                                                     int K, int lda, int ldb, int ldc, long long sA,
-                                                                     long long sB, long long sC, bool by_item) {
+                                                                     uint16_t* __restrict__ C, int M, int N, int K,
+                                                                     int lda, int ldb, int ldc, long long sA,
+                                                                     long long sB, long long sC, bool xcd, Div chunks,
+                                                                     Div tiles) {
   constexpr int TN = 32 * NF, RB = TN * 2, B_B = SM_BK * RB, STAGE = SM_A_B + B_B;
   constexpr int BL = B_B / 1024, BCH = RB / 16, BRPL = 1024 / RB;
   extern __shared__ __align__(1024) unsigned char smem[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 5;
-  const SmallTile t = small_tile(by_item);
+  const SmallTile t = small_tile(xcd, chunks, tiles);
   const size_t item = t.item;
   const int n0 = t.ct * TN, m0 = t.mc * 32;
-  if (t.item >= batch) return;
   A += item * sA + (size_t)m0 * lda;
   B += item * sB;
   C += item * sC + (size_t)m0 * ldc;
@@ -1075,20 +1090,14 @@ static int small_width(int batch, int M, int N, int K) {  // 32-column fragments
 
 static int launch_smallm(const void* A, const void* B, void* C, int batch, int M, int N, int K, int lda, int ldb,
                          int ldc, long long sA, long long sB, long long sC, hipStream_t stream) {
-  // Grid: items (rounded up to whole XCDs; the extra workgroups return at
-  // once), column tiles, row chunks; with by_item off, column tiles, items, row
-  // chunks.  One launch covers the 65535 column tiles of a grid's second dimension.
-  auto go = [&](auto kern, int threads, int smem, int tn, bool by_item) {
-    const int most = 65535 * tn;
-    for (long long n0 = 0; n0 < N; n0 += most) {
-      const int n = (int)(N - n0 < most ? N - n0 : most);
-      const unsigned nt = (unsigned)((n + tn - 1) / tn), nb = (unsigned)(batch + 7) / 8 * 8,
-                     nm = (unsigned)((M + 31) / 32);
-      hipLaunchKernelGGL(kern, by_item ? dim3(nb, nt, nm) : dim3(nt, (unsigned)batch, nm), dim3(threads), smem, stream,
-                         (const uint16_t*)A, (const uint16_t*)B + n0, (uint16_t*)C + n0, batch, M, n, K, lda, ldb, ldc,
-                         sA, sB, sC, by_item);
-      MX_RETURN_IF_HIP(hipGetLastError());
-    }
+  auto go = [&](auto kern, int threads, int smem, int tn) {
+    const int chunks = (M + 31) / 32, tiles = (N + tn - 1) / tn;
+    const long long grid = (long long)batch * chunks * tiles;
+    if (grid > 0x7fffffffLL) return MX_ERR_SHAPE;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads), smem, stream, (const uint16_t*)A, (const uint16_t*)B,
+                       (uint16_t*)C, M, N, K, lda, ldb, ldc, sA, sB, sC, K / SM_BK > 2, make_div(chunks),
+                       make_div(tiles));
+    MX_RETURN_IF_HIP(hipGetLastError());
     return MX_OK;
   };
   const int nkc = K / SM_BK, nf = small_width(batch, M, N, K);
@@ -1097,14 +1106,13 @@ static int launch_smallm(const void* A, const void* B, void* C, int batch, int M
       constexpr int NF = decltype(nf_tag)::value, STAGE = SM_A_B + SM_BK * 64 * NF;
       constexpr auto kern = gemm_bf16_smallm_sk_kernel<NF, 4>;
       MX_RETURN_IF_HIP(lds_limit_once<kern>(12 * STAGE));
-      return go(kern, 256, nkc * STAGE, 32 * NF, true);
+      return go(kern, 256, nkc * STAGE, 32 * NF);
     };
     return nf == 2 ? split_k(std::integral_constant<int, 2>{}) : split_k(std::integral_constant<int, 1>{});
   }
-  const bool by_item = nkc > 2;
-  if (nf == 4) return go(gemm_bf16_smallm_kernel<4>, 64, 0, 128, by_item);
-  if (nf == 2) return go(gemm_bf16_smallm_kernel<2>, 64, 0, 64, by_item);
-  return go(gemm_bf16_smallm_kernel<1>, 64, 0, 32, by_item);
+  if (nf == 4) return go(gemm_bf16_smallm_kernel<4>, 64, 0, 128);
+  if (nf == 2) return go(gemm_bf16_smallm_kernel<2>, 64, 0, 64);
+  return go(gemm_bf16_smallm_kernel<1>, 64, 0, 32);
 }
 
 
@@ -1519,19 +1527,19 @@ static bool batched_small(int M, int K, int lda, int ldb) {
 }
 
 // More rows take the same kernels, 32 at a time, where that beats the tiles
-// (graph replay; 800 random items, contiguous and strided by head):  K split
-// among four waves while a workgroup per CU is enough (N 128, K 512: 16 items
-// of 48 rows 4.62 -> 3.49 us, 64 items 5.39 -> 5.22, but 128 items 7.3 -> 9.1),
-// and one or two chunks of K, which need a single round trip, while all
-// workgroups run at once (K 128: 14 items of 46 x 512 3.19 against 3.34 us with
-// tiles, 18 of 62 x 512 3.53 against 3.41, 75 of 38 x 512 8.1 against 5.4; K 64:
-// 51 of 55 x 88 2.73 against 3.26, 133 of 58 x 88 4.10 against 3.55).
+// (graph replay; 1200 random items, contiguous and strided by head): K split
+// among four waves while a workgroup per CU is enough (N 128, K 512: 16 items of
+// 48 rows 4.62 -> 3.49 us, 64 items 5.39 -> 5.22, but 128 items 7.3 -> 9.1), and
+// one or two chunks of K, which need a single round trip, while all workgroups
+// run at once, three of 32 x 32 to a CU (K 128: 14 items of 46 x 512 3.19 against
+// 3.34 us with tiles, 75 of 38 x 512 8.1 against 5.4; K 64: 120 of 36 x 72, 720
+// workgroups, 3.00 against 3.30, 133 of 58 x 88, 798, 4.10 against 3.55).
 static bool batched_rows(int batch, int M, int N, int K, int lda, int ldb) {
   if (K % 64 || !strides_2g<64>(lda, ldb)) return false;
   const int nkc = K / SM_BK;
   const long long rows = (long long)batch * ((M + 31) / 32);
   if (nkc % 4 == 0 && nkc <= 12) return rows * ((N + 63) / 64) <= 256;
-  return nkc <= 2 && rows * ((N + 31) / 32) <= 512;
+  return nkc <= 2 && small_width(batch, M, N, K) == 1 && rows * ((N + 31) / 32) <= 768;
 }
 
 // Every check mx_gemm_bf16_batched makes before it launches, the grid

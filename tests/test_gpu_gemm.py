@@ -362,8 +362,8 @@ def test_infinity_in_the_last_k_row(ops, mnk):
                                   # the most groups and one item more), and one and two chunks of K
                                   (7, 65, 136, 768), (16, 200, 128, 512), (64, 64, 128, 256), (65, 64, 128, 256),
                                   (16, 33, 512, 64), (37, 64, 264, 128), (128, 48, 512, 128), (3, 65, 72, 128),
-                                  # ... up to 512 workgroups of 32 x 32 at any M, and one item more
-                                  (32, 128, 128, 64), (33, 128, 128, 64), (9, 96, 520, 128), (5, 1000, 72, 128),
+                                  # ... up to 768 workgroups of 32 x 32 at any M, and one item more
+                                  (48, 128, 128, 64), (49, 128, 128, 64), (9, 96, 520, 128), (5, 1000, 72, 128),
                                   # 64x64 to 128x192 tiles from K 128 on, K tails on both sides of 32 and none
                                   (1, 1, 8, 152), (1, 104, 8, 240), (12, 542, 232, 800), (9, 815, 248, 888),
                                   (18, 222, 792, 176), (56, 374, 432, 216), (16, 563, 400, 296),
@@ -385,10 +385,9 @@ def test_batched_larger_items(ops, bmnk):
 
 
 @pytest.mark.parametrize("bmnk", [(1, 3, 65535 * 64 + 72, 256), (2, 2, 65535 * 128 + 8, 192)])
-def test_batched_more_column_tiles_than_a_grid_dimension(ops, bmnk):
-    """Small-row kernels whose grid has items first take the column tiles in
-    slices of 65535: every column is written, those around the seam and at both
-    ends are right."""
+def test_batched_many_column_tiles(ops, bmnk):
+    """Small-row kernels over more than 65535 column tiles: every column is
+    written, those around that tile and at both ends are right."""
     nb, m, n, k = bmnk
     announce(f"gemm_bf16_batched {nb}x{m}x{n}x{k}")
     g = torch.Generator(device="cuda").manual_seed(k)

@@ -107,3 +107,37 @@ def test_attention_key_groups(tmp_path):
     for d, most in ((64, {2, 4}), (128, {2})):
         for causal in (0, 1):
             assert {g[causal] for r, g in groups.items() if r[4] == d} - {1} == most
+
+
+def test_division_of_workgroup_ids(tmp_path):
+    """The batched kernels' division by multiplication, exact for every divisor
+    and n below 2^31: small divisors, powers of two and their neighbours, primes
+    and the largest, at multiples of each and beside them."""
+    out = query(tmp_path, "gemm_bf16.hip", r"""
+  using namespace mx::gemm;
+  const uint32_t top = 0x7fffffffu;
+  long long checked = 0;
+  auto test = [&](uint32_t d) {
+    const Div v = make_div(d);
+    auto at = [&](long long n) {
+      if (n < 0 || n > top) return true;
+      ++checked;
+      return quot((uint32_t)n, v) == (uint32_t)n / d;
+    };
+    bool ok = true;
+    for (long long q = 0; q < 40; ++q)
+      for (long long m : {q * d, (long long)(top / d - q) * d, (long long)(top / d / (q + 2)) * d})
+        ok = ok && at(m - 1) && at(m) && at(m + 1);
+    return ok && at(top);
+  };
+  for (uint32_t d = 1; d <= 70000; ++d)
+    if (!test(d)) { printf("wrong for %u\n", d); return 0; }
+  for (int b = 0; b < 31; ++b)
+    for (int e = -3; e <= 3; ++e) {
+      const long long d = (1LL << b) + e;
+      if (d >= 1 && d <= top && !test((uint32_t)d)) { printf("wrong for %lld\n", d); return 0; }
+    }
+  for (uint32_t d : {1000003u, 16777213u, 1073741789u, 2147483629u, 2147483646u, 2147483647u})
+    if (!test(d)) { printf("wrong for %u\n", d); return 0; }
+  printf("ok %d\n", checked > 10000000);""")
+    assert out == ["ok 1"]
