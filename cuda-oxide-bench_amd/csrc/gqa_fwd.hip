@@ -666,7 +666,9 @@ static int dispatch_tile(const void* Q, const void* K, const void* V, void* O, i
 // shorter prompts (up to 64 x 96 heads, S 16..20000), where the first fit split
 // keys that fill the CUs unsplit (B10 with 64 heads, S99: 24.4 us with one group,
 // 29.1 with two).  The choice is on average 0.8% slower than the best; B39 with
-// 4 heads, S288, takes 27.5 us in two groups against 24.6.
+// 4 heads, S288, takes 27.5 us in two groups against 24.6.  A step's cost shows
+// alone at long S (one sequence, 8 heads, S16462, no mask: 1196 us with one group,
+// 1101 with two).
 struct Split {
   int ksp, hpw;
   bool pairs;
@@ -678,7 +680,7 @@ static Split pick_split(int B, int Hq, int Hkv, int S, int causal) {
     double step, ends, fixed;
   };
   static constexpr Cost k64[] = {{1, 1.0, 4.0, 0.0}, {2, 1.08, 4.5, 1.0}, {4, 1.3, 3.5, 1.0}};
-  static constexpr Cost k128[] = {{1, 1.4, 5.75, 0.0}, {2, 1.72, 5.4, 0.15}};
+  static constexpr Cost k128[] = {{1, 1.4, 5.0, 0.0}, {2, 1.6, 5.0, 1.0}};
   const Cost* cost = DQK == 64 ? k64 : k128;
   const int choices = DQK != DV ? 1 : DQK == 64 ? 3 : 2;
   const int G = Hq / Hkv;
